@@ -52,18 +52,14 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-// Per-GEMM configuration: wave layout W (8 or 4), column tile BN and main-loop
-// pipeline PIPE (4: direct-to-LDS loads, needs K-major operands with K a
-// multiple of 64; 5: as 4 with an MN-major A read back transposed; 3:
-// register-staged loads, any K).  The "fallback" configuration serves
-// K % 64 != 0.
+// GEMM configuration: waves per workgroup and column tile BN (256, or 128 for
+// the tail of a hidden dimension).
 constexpr int kWarp8 = 8;
-constexpr int kFastBN = 256;    // PIPE 4 kernels
-constexpr int kSlowBN = 128;    // PIPE 3 kernels
+constexpr int kBN = 256;
+constexpr int kTailBN = 128;
 
 constexpr int kBM = 256;              // rows of a workgroup tile
 constexpr int kBK = 64;               // K slab per pipeline step
-constexpr int kPitch = kBK + 8;       // LDS row pitch in bf16 (144 B: conflict-free b128 reads)
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.69314718055994531f;
 constexpr float kNegBig = -FLT_MAX;   // finite "minus infinity" for running maxima
@@ -108,23 +104,6 @@ __device__ inline void grouped_map(int bid, int nb, int gm, int gn, int& pm, int
   pn = r / rows;
 }
 
-// ---------------------------------------------------------------------------
-// Global -> LDS operand loaders.  LDS holds every operand tile as [row][k]
-// (k contiguous, pitch kPitch) so one MFMA fragment read serves both layouts.
-// ---------------------------------------------------------------------------
-
-// 16 zero bytes in device memory: out-of-range lanes load from here.
-__device__ __attribute__((aligned(16))) uint32_t g_zero16[4];
-
-// 16-byte load that is issued unconditionally: out-of-range lanes read the
-// zero block instead, so the value needs no select after the load.  Keeping
-// the load out of divergent control flow and unconsumed until its LDS store
-// lets the compiler count outstanding loads exactly instead of draining them.
-__device__ inline u32x4 guarded_load(const bf16_t* __restrict__ X, long off, bool ok) {
-  const u32x4* p = ok ? reinterpret_cast<const u32x4*>(X + off) : reinterpret_cast<const u32x4*>(g_zero16);
-  return *p;
-}
-
 // Per-kernel wave layout.  W = 8: two waves per SIMD, 64-row wave tiles,
 // accumulators in VGPRs.  W = 4: one wave per SIMD, 128-row wave tiles,
 // accumulators in AGPRs.  Waves form (256 / kWaveRows) x 2 over a tile.
@@ -133,82 +112,6 @@ struct WaveCfg {
   static constexpr int kThreads = W * 64;
   static constexpr int kWaveRows = (W == 8) ? 64 : 128;
   static constexpr int kFM = kWaveRows / 32;  // 32-row MFMA blocks per wave tile
-};
-
-// K-major operand: element (r, k) at X[r*ld + k].
-template <int BR, int W>
-struct LoadKMajor {
-  static constexpr int kT = W * 64;
-  static constexpr int kN = BR * (kBK / 8) / kT;  // 16-byte chunks per thread
-  u32x4 v[kN];
-  __device__ inline void load(const bf16_t* __restrict__ X, long ld, int r0, int rlim, int k0, int K,
-                              int tid) {
-#pragma unroll
-    for (int i = 0; i < kN; ++i) {
-      const int c = tid + i * kT;
-      const int row = c >> 3, kc = (c & 7) * 8;
-      const int gr = r0 + row, gk = k0 + kc;
-      v[i] = guarded_load(X, (long)gr * ld + gk, gr < rlim && gk < K);
-    }
-  }
-  __device__ inline void store(bf16_t* S, int tid) const {
-#pragma unroll
-    for (int i = 0; i < kN; ++i) {
-      const int c = tid + i * kT;
-      const int row = c >> 3, kc = (c & 7) * 8;
-      *reinterpret_cast<u32x4*>(S + row * kPitch + kc) = v[i];
-    }
-  }
-};
-
-// MN-major operand (256-row tiles): element (r, k) at X[k*ld + r].  Each
-// thread loads 4(k) x 8(r) blocks with 16-byte loads, transposes them in
-// registers and writes 8-byte [r][k] pieces to LDS.  Lanes 0..15 of a wave
-// walk k, so the 8-byte LDS writes of 16 lanes cover 32 distinct banks.
-template <int W>
-struct LoadMNMajor256 {
-  static constexpr int kB = 512 / (W * 64);  // 4x8 blocks per thread
-  u32x4 v[kB][4];
-  __device__ inline void load(const bf16_t* __restrict__ X, long ld, int r0, int rlim, int k0, int K,
-                              int tid) {
-    const int w = tid >> 6, l = tid & 63;
-    const int kq = l & 15;
-#pragma unroll
-    for (int t = 0; t < kB; ++t) {
-      const int rb = (w * kB + t) * 4 + (l >> 4);
-      const int gr = r0 + rb * 8;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int gk = k0 + kq * 4 + i;
-        v[t][i] = guarded_load(X, (long)gk * ld + gr, gk < K && gr < rlim);
-      }
-    }
-  }
-  __device__ inline void store(bf16_t* S, int tid) const {
-    const int w = tid >> 6, l = tid & 63;
-    const int kq = l & 15;
-#pragma unroll
-    for (int t = 0; t < kB; ++t) {
-      const int rb = (w * kB + t) * 4 + (l >> 4);
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const uint32_t a0 = v[t][0][q], a1 = v[t][1][q], a2 = v[t][2][q], a3 = v[t][3][q];
-        const u32x2 ev = {(a0 & 0xffffu) | (a1 << 16), (a2 & 0xffffu) | (a3 << 16)};
-        const u32x2 od = {(a0 >> 16) | (a1 & 0xffff0000u), (a2 >> 16) | (a3 & 0xffff0000u)};
-        *reinterpret_cast<u32x2*>(S + (rb * 8 + 2 * q) * kPitch + kq * 4) = ev;
-        *reinterpret_cast<u32x2*>(S + (rb * 8 + 2 * q + 1) * kPitch + kq * 4) = od;
-      }
-    }
-  }
-};
-
-template <bool KMAJ, int BR, int W>
-struct LoaderSel {
-  typedef LoadKMajor<BR, W> type;
-};
-template <int W>
-struct LoaderSel<false, 256, W> {
-  typedef LoadMNMajor256<W> type;
 };
 
 // Row compaction: when `dyn` is set, `live` points at the device-side count
@@ -227,12 +130,11 @@ struct GemmShape {
   const int* live = nullptr;
   int dyn = kDynNone;
   int live_base = 0;
-  // k offset of B in elements (direct-to-LDS pipelines): B's k index kb + k.
-  // A slab that runs past K reads the rest of its row (zero padding or the
-  // next rows' finite values); it never runs past the row's end (ld), so never
-  // past B (kmajor_fits).
+  // k offset of B in elements: B's k index kb + k.  A slab that runs past K
+  // reads the rest of its row (zero padding or finite values); it never runs
+  // past the row's end (ld), so never past B (kmajor_fits).
   int kb = 0;
-  // Row map of a K-major A (PIPE 4): GEMM row m is row arow[m] of A, which
+  // Row map of a K-major A: GEMM row m is row arow[m] of A, which
   // has arows rows in all (arows * lda * 2 bytes below 2^31 - 16).  Null:
   // row m is row m.
   const int* arow = nullptr;
@@ -281,7 +183,7 @@ __device__ inline void pin_epilogue(int& l, int& tm, int& tn) {
 }
 
 // ---------------------------------------------------------------------------
-// Direct global -> LDS loads (PIPE 4).  A buffer load with the `lds` modifier
+// Direct global -> LDS loads.  A buffer load with the `lds` modifier
 // writes each lane's 16 bytes straight into LDS at M0 + 16*lane, so one wave
 // instruction fills 1 KB = 8 rows x 128 B of a [row][64 k] tile.  LDS rows
 // are not padded; instead the 16-byte chunk c of row r lives at physical chunk
@@ -306,9 +208,16 @@ __device__ inline __amdgpu_buffer_rsrc_t make_rsrc(const void* base, long bytes)
 // the swizzled LDS region S.  Rows past rlim fall outside the descriptor's
 // range and read as zero.  k0 goes in the scalar offset, which a raw buffer
 // does not range-check: every slab must end inside its row (k0 + 64 <= ld),
-// which kmajor_fits() checks on the host for every launch.
-template <int BR, int W>
-__device__ inline void dma_kmajor(const bf16_t* __restrict__ X, long ld, int r0, int rlim, int k0, bf16_t* S,
+// which kmajor_fits() checks on the host for every launch.  KTAIL: K is no
+// multiple of 64 and the rows hold only K columns; the lanes of the last slab
+// whose 8 columns start at K or later get an offset past the descriptor's
+// range, so they read as zero (K is a multiple of 8).  That costs a compare and
+// a select per DMA instruction, against a register-staged pipeline in 128-wide
+// tiles with separate recompute and gradient launches before: N 1500, d 1000,
+// V 50257 with bias, forward and backward 2116 -> 1200 us.
+constexpr int kOutOfRange = (int)0x80000000u;
+template <int BR, int W, bool KTAIL = false>
+__device__ inline void dma_kmajor(const bf16_t* __restrict__ X, long ld, int r0, int rlim, int k0, int K, bf16_t* S,
                                   int w, int l) {
   constexpr int kI = BR / (8 * W);  // wave instructions per wave
   const long rows_left = (long)rlim - r0;
@@ -318,7 +227,8 @@ __device__ inline void dma_kmajor(const bf16_t* __restrict__ X, long ld, int r0,
     const int blk = w * kI + j;           // 8-row block of the tile
     const int row = blk * 8 + (l >> 3);
     const int c = (l & 7) ^ swz(row);     // logical chunk this lane fetches
-    const int voff = (int)(((long)row * ld + c * 8) * 2);
+    int voff = (int)(((long)row * ld + c * 8) * 2);
+    if constexpr (KTAIL) voff = k0 + c * 8 < K ? voff : kOutOfRange;
     __builtin_amdgcn_raw_ptr_buffer_load_lds(
         rs, (__attribute__((address_space(3))) void*)(S + blk * 512), 16, voff, k0 * 2, 0, 0);
   }
@@ -346,7 +256,7 @@ struct ARows {
     for (int j = 0; j < kI; ++j) {
       const int row = (w * kI + j) * 8 + (l >> 3);
       const int c = (l & 7) ^ swz(row);
-      voff[j] = row < rows_left ? (int)(((long)arow[r0 + row] * ld + c * 8) * 2) : (int)0x80000000u;
+      voff[j] = row < rows_left ? (int)(((long)arow[r0 + row] * ld + c * 8) * 2) : kOutOfRange;
     }
   }
   // the DMA of k [k0, k0 + 64) into the swizzled LDS region S
@@ -359,24 +269,27 @@ struct ARows {
   }
 };
 
-// MN-major tile for PIPE 5: element (m, k) at X[k*ld + m].  The tile
-// k [k0, k0 + 64) x m [m0, m0 + 256) is copied in its natural [k][m] layout
-// (512 B per k row; one wave instruction = 2 rows), with 16-byte chunk c of
-// row k stored at physical chunk c ^ (4*(k & 3)) so the four rows touched by
-// one transposed fragment read land on distinct banks.  Rows k >= K fall
-// outside the descriptor's range and read as zero.
-template <int W>
-__device__ inline void dma_mnmajor256(const bf16_t* __restrict__ X, long ld, int m0, int k0, int K, bf16_t* S,
-                                      int w, int l) {
-  constexpr int kI = 32 / W;  // 32 wave instructions per 64 x 256 tile
+// MN-major tile: element (m, k) at X[k*ld + m].  The tile k [k0, k0 + 64) x
+// m [m0, m0 + BR) is copied in its natural [k][m] layout (BR * 2 bytes per k
+// row; one wave instruction = 512 / BR rows), with 16-byte chunk c of row k
+// stored at physical chunk c ^ (4*(k & 3)) so the four rows touched by one
+// transposed fragment read land on distinct banks.  Rows k >= K fall outside
+// the descriptor's range and read as zero; columns past a row's end read the
+// next row (the epilogues mask them).
+template <int BR, int W>
+__device__ inline void dma_mnmajor(const bf16_t* __restrict__ X, long ld, int m0, int k0, int K, bf16_t* S, int w,
+                                   int l) {
+  static_assert(BR == 256 || BR == 128, "whole or half rows of the swizzle");
+  constexpr int kI = BR / (8 * W);    // wave instructions per wave
+  constexpr int kLanes = BR / 8;      // lanes per k row
   const long rows_left = (long)K - k0;
   const long bytes = rows_left > 0 ? (rows_left * ld - m0) * 2 : 0;
   const __amdgpu_buffer_rsrc_t rs = make_rsrc(X + (long)k0 * ld + m0, bytes);
 #pragma unroll
   for (int j = 0; j < kI; ++j) {
-    const int blk = w * kI + j;  // pair of k rows
-    const int row = blk * 2 + (l >> 5);
-    const int c = (l & 31) ^ (4 * (row & 3));
+    const int blk = w * kI + j;  // 512 / BR k rows
+    const int row = blk * (64 / kLanes) + l / kLanes;
+    const int c = (l % kLanes) ^ (4 * (row & 3));
     const int voff = (int)(((long)row * ld + c * 8) * 2);
     __builtin_amdgcn_raw_ptr_buffer_load_lds(
         rs, (__attribute__((address_space(3))) void*)(S + blk * 512), 16, voff, 0, 0, 0);
@@ -389,10 +302,11 @@ typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 // ds_read_b64_tr_b16: in each 16-lane group, lane j receives element j&3 of
 // the 8-byte reads addressed by lanes (j>>2) + 4t, t = 0..3.  Lane a of the
 // group addresses row k = kb + (a>>2), columns m = mb + 4*(a&3) .. +3 of the
-// [k][m] tile, so lane j receives k = kb..kb+3 of column m = mb + j.
+// [k][m] tile (BR columns), so lane j receives k = kb..kb+3 of column m = mb + j.
+template <int BR>
 __device__ inline uint2 read_tr4(const bf16_t* S, int k, int m) {
   const int phys = (((m >> 3) ^ (4 * (k & 3))) << 3) + (m & 7);
-  const s16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(S + k * 256 + phys));
+  const s16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(S + k * BR + phys));
   return __builtin_bit_cast(uint2, v);
 }
 
@@ -402,55 +316,29 @@ struct Frags {
   u32x4 a[WaveCfg<W>::kFM], b[BN / 64];
 };
 
-template <int BN, int W>
-__device__ inline void read_frags(const bf16_t* __restrict__ As, const bf16_t* __restrict__ Bs, int kk,
-                                  Frags<BN, W>& f, int wm, int wn, int l) {
-  const int kof = kk * 16 + (l >> 5) * 8;
+// One operand's fragments of k-step kk from an unpadded LDS tile, for the
+// FR 32-row blocks from tile row r0: lane l gets row r0 + i*32 + (l & 31),
+// k = kk*16 + 8*(l >> 5) + 0..7.  KM: the swizzled [row][64 k] layout;
+// otherwise the [k][BR rows] layout, read transposed.
+template <bool KM, int BR, int FR>
+__device__ inline void read_op(const bf16_t* __restrict__ S, int kk, int r0, u32x4 (&f)[FR], int l) {
+  if constexpr (KM) {
+    const int c = kk * 2 + (l >> 5);
 #pragma unroll
-  for (int i = 0; i < WaveCfg<W>::kFM; ++i)
-    f.a[i] = *reinterpret_cast<const u32x4*>(As + (wm * WaveCfg<W>::kWaveRows + i * 32 + (l & 31)) * kPitch + kof);
+    for (int i = 0; i < FR; ++i) {
+      const int r = r0 + i * 32 + (l & 31);
+      f[i] = *reinterpret_cast<const u32x4*>(S + r * 64 + ((c ^ swz(r)) << 3));
+    }
+  } else {
+    const int a = l & 15;
+    const int kb = kk * 16 + 8 * (l >> 5) + (a >> 2);
 #pragma unroll
-  for (int j = 0; j < BN / 64; ++j)
-    f.b[j] = *reinterpret_cast<const u32x4*>(Bs + (wn * (BN / 2) + j * 32 + (l & 31)) * kPitch + kof);
-}
-
-// Fragment reads from the swizzled (unpadded, 64 bf16 per row) layout.
-template <int BN, int W>
-__device__ inline void read_frags_swz(const bf16_t* __restrict__ As, const bf16_t* __restrict__ Bs, int kk,
-                                      Frags<BN, W>& f, int wm, int wn, int l) {
-  const int c = kk * 2 + (l >> 5);
-#pragma unroll
-  for (int i = 0; i < WaveCfg<W>::kFM; ++i) {
-    const int r = wm * WaveCfg<W>::kWaveRows + i * 32 + (l & 31);
-    f.a[i] = *reinterpret_cast<const u32x4*>(As + r * 64 + ((c ^ swz(r)) << 3));
-  }
-#pragma unroll
-  for (int j = 0; j < BN / 64; ++j) {
-    const int r = wn * (BN / 2) + j * 32 + (l & 31);
-    f.b[j] = *reinterpret_cast<const u32x4*>(Bs + r * 64 + ((c ^ swz(r)) << 3));
-  }
-}
-
-// A fragments from the [k][m] tile with transposed reads (PIPE 5): lane l
-// gets m = i*32 + (l & 31), k = kk*16 + 8*(l >> 5) + 0..7 — the same k map as
-// the K-major B fragments.
-template <int BN, int W>
-__device__ inline void read_frags_tr(const bf16_t* __restrict__ As, const bf16_t* __restrict__ Bs, int kk,
-                                     Frags<BN, W>& f, int wm, int wn, int l) {
-  const int a = l & 15;
-  const int kb = kk * 16 + 8 * (l >> 5) + (a >> 2);
-#pragma unroll
-  for (int i = 0; i < WaveCfg<W>::kFM; ++i) {
-    const int mb = wm * WaveCfg<W>::kWaveRows + i * 32 + 16 * ((l >> 4) & 1) + 4 * (a & 3);
-    const uint2 lo = read_tr4(As, kb, mb);
-    const uint2 hi = read_tr4(As, kb + 4, mb);
-    f.a[i] = u32x4{lo.x, lo.y, hi.x, hi.y};
-  }
-  const int c = kk * 2 + (l >> 5);
-#pragma unroll
-  for (int j = 0; j < BN / 64; ++j) {
-    const int r = wn * (BN / 2) + j * 32 + (l & 31);
-    f.b[j] = *reinterpret_cast<const u32x4*>(Bs + r * 64 + ((c ^ swz(r)) << 3));
+    for (int i = 0; i < FR; ++i) {
+      const int mb = r0 + i * 32 + 16 * ((l >> 4) & 1) + 4 * (a & 3);
+      const uint2 lo = read_tr4<BR>(S, kb, mb);
+      const uint2 hi = read_tr4<BR>(S, kb + 4, mb);
+      f[i] = u32x4{lo.x, lo.y, hi.x, hi.y};
+    }
   }
 }
 
@@ -873,37 +761,20 @@ struct EpiAcc {
 };
 
 // ---------------------------------------------------------------------------
-// The GEMM kernel: C[M,N] = A[M,K] . B[N,K]^T, 256 x BN x 64 tiles.  PIPE 4 / 5
-// (direct-to-LDS) are described at their loop below.  PIPE 3 has two LDS
-// stages and two register sets of prefetched slabs.
-//
-// PIPE 3 software pipeline (per slab s, LDS stage p = s & 1):
-//   - global loads of slab s+2 go to register set p (issued unconditionally:
-//     past the last slab the loaders' bounds predicates read zeros, so the
-//     compiler's outstanding-load counts stay exact);
-//   - register set p^1 (slab s+1, loaded one slab earlier) drains into LDS
-//     stage p^1 after the first k-step;
-//   - the fragments of k-step kk+1 are read from LDS while the MFMAs of
-//     k-step kk run, and the first fragments of slab s+1 right after the
-//     barrier that closes slab s.
-// Tiles are walked in an even number of slabs (the loaders zero-fill past
-// K) so register-set and LDS-stage parities are static in the unrolled loop.
-// A workgroup may own a run of column tiles (forward); the pipeline then runs
-// on across tile boundaries.  Single-tile epilogues peel the last slab pair so
-// no prefetch registers are live while they run.
+// The GEMM kernel: C[M,N] = A[M,K] . B[N,K]^T, 256 x BN x 64 tiles, operands
+// copied straight into NST unpadded LDS stages (described at the loop below).
+// AK: A is K-major, else MN-major and read back transposed; B is K-major.
+// AROW: a K-major A is read through g.arow (ARows).  KTAIL: K-major operands
+// whose K is no multiple of 64 (dma_kmajor).
 // ---------------------------------------------------------------------------
-// LDS elements of the pipeline stages: unpadded for the direct-to-LDS
-// pipelines, kPitch-padded rows for the register-staged ones.
 template <int BN>
-constexpr int gemm_lds_elems(int pipe, int nst = 2) {
-  return (pipe >= 4 ? nst : 2) * (kBM + BN) * (pipe >= 4 ? 64 : kPitch);
+constexpr int gemm_lds_elems(int nst = 2) {
+  return nst * (kBM + BN) * kBK;
 }
 
-// AROW: A is read through g.arow (PIPE 4; see ARows).
-template <int BN, int W, bool AK, bool BKM, template <int, int> class EpiT, int PIPE, int NST = 2, bool AROW = false>
+template <int BN, int W, bool AK, template <int, int> class EpiT, int NST = 2, bool AROW = false, bool KTAIL = false>
 __device__ __forceinline__ void gemm_body(const GemmShape& g_in, const typename EpiT<BN, W>::Params& ep, int bid,
                                           int nb, bf16_t* smem) {
-  static_assert(PIPE >= 3 && PIPE <= 5, "pipelines: 3 (register-staged), 4 and 5 (direct-to-LDS)");
   typedef EpiT<BN, W> Epi;
   GemmShape g = g_in;
   if (g.dyn == kDynK) g.K = min(g.K, live_rows(g.live, g.live_base));
@@ -921,9 +792,8 @@ __device__ __forceinline__ void gemm_body(const GemmShape& g_in, const typename 
       if (bid >= nb) return;
     }
   }
-  constexpr int kStage = (kBM + BN) * kPitch;
   // epilogue staging area, past the pipeline's LDS stages
-  bf16_t* const scratch = smem + gemm_lds_elems<BN>(PIPE, NST);
+  bf16_t* const scratch = smem + gemm_lds_elems<BN>(NST);
 
   const int tid = threadIdx.x, l = tid & 63, w = tid >> 6;
   const int wm = w >> 1, wn = w & 1;
@@ -937,225 +807,130 @@ __device__ __forceinline__ void gemm_body(const GemmShape& g_in, const typename 
   WaveAcc<BN, W> acc;
 
   const int KT = (g.K + kBK - 1) / kBK;
-  const int KT2 = (KT + 1) & ~1;
   const int a_r0 = tm * kBM;
-  bf16_t* const S0 = smem;
-  bf16_t* const S1 = smem + kStage;
-
-  if constexpr (PIPE == 4 || PIPE == 5) {
-    // Direct-to-LDS pipeline over the workgroup's slabs s = 0, 1, ... (a run
-    // of column tiles times KT slabs each), LDS stage s & 1.  Per slab:
-    //   k-steps 0..2: MFMAs, with the fragments of the next k-step read
-    //                 from LDS behind them;
-    //   barrier B_s:  its implied vmcnt(0) / lgkmcnt(0) mean slab s+1's DMA
-    //                 (issued after B_{s-1}) has landed for every wave and no
-    //                 wave still reads slab s's stage;
-    //   then the DMA of slab s+2 into that stage and the first fragments of
-    //   slab s+1 are issued while the MFMAs of k-step 3 (whose fragments are
-    //   already in registers) run, so the barrier's read bubble is hidden.
-    // B is K-major; A is K-major (PIPE 4) or MN-major read back transposed
-    // (PIPE 5).  K-major operands need K a multiple of 64 (or zero padding).
-    static_assert(BKM && (PIPE == 5 || AK), "direct-to-LDS operand layouts");
-    static_assert(PIPE == 4 || (!AK && BN <= 256), "PIPE 5 reads an MN-major A");
-    constexpr int kSt = (kBM + BN) * 64;  // unpadded stage
-    static_assert(NST >= 2 && NST <= 3, "LDS holds two or three stages");
-    // DMA wave instructions per wave per slab
-    constexpr int kD = (PIPE == 4 ? kBM / (8 * W) : 32 / W) + BN / (8 * W);
-    auto frags = [&](const bf16_t* Sc, int kk, Frags<BN, W>& f) {
-      if constexpr (PIPE == 4)
-        read_frags_swz<BN, W>(Sc, Sc + kBM * 64, kk, f, wm, wn, l);
-      else
-        read_frags_tr<BN, W>(Sc, Sc + kBM * 64, kk, f, wm, wn, l);
-    };
-    // DMA of the next unissued slab (tile it2, k-slab ik2) into stage S
-    int it2 = t0, ik2 = 0;
-    // A through a row map: its lane offsets are computed once per workgroup
-    static_assert(!AROW || PIPE == 4, "row-mapped A is K-major");
-    ARows<W> arows;
-    if constexpr (AROW) arows.init(g.A, g.lda, a_r0, g.M, g.arow, g.arows, w, l);
-    auto issue = [&](bf16_t* S) {
-      if constexpr (AROW)
-        arows.dma(ik2 * kBK, S, w);
-      else if constexpr (PIPE == 4)
-        dma_kmajor<kBM, W>(g.A, g.lda, a_r0, g.M, ik2 * kBK, S, w, l);
-      else
-        dma_mnmajor256<W>(g.A, g.lda, a_r0, ik2 * kBK, g.K, S, w, l);
-      dma_kmajor<BN, W>(g.B, g.ldb, it2 * BN, g.N, g.kb + ik2 * kBK, S + kBM * 64, w, l);
-      if (++ik2 == KT) {
-        ik2 = 0;
-        ++it2;
-      }
-    };
-    // The DMA's LDS writes count on vmcnt; the barrier's own fence does not
-    // reliably wait for them, so each barrier B_s that publishes slab s+1 is
-    // preceded by an explicit wait.  Vector memory operations retire in
-    // issue order, so B_s may leave in flight exactly what was issued after
-    // slab s+1's DMA: the DMAs of slabs s+2 .. s+NST-1, and the previous
-    // tile's epilogue stores for the first NST-1 slabs of a tile (they then
-    // drain behind the MFMAs).  Near the end of the run, where some of those
-    // DMAs were never issued, it waits for everything.  sched_barrier fences
-    // keep the MFMAs on their side of the barrier.
-    auto publish = [&](int s_, bool after_epilogue) {
-      __builtin_amdgcn_sched_barrier(0);
-      const bool deep = s_ + NST - 1 < ((t1 - t0) * KT);
-      if (deep && Epi::kStores > 0 && after_epilogue)
-        __builtin_amdgcn_s_waitcnt(vmcnt_imm((NST - 2) * kD + Epi::kStores));
-      else if (deep && NST > 2)
-        __builtin_amdgcn_s_waitcnt(vmcnt_imm((NST - 2) * kD));
-      else
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      __syncthreads();
-      __builtin_amdgcn_sched_barrier(0);
-    };
-    // each k-step: the next k-step's fragment reads are issued first, then
-    // the MFMAs they hide behind
-    auto order = [&]() {
-      constexpr int kReads = (PIPE == 4 ? 1 : 2) * WaveCfg<W>::kFM + BN / 64;
-      __builtin_amdgcn_sched_group_barrier(0x100, kReads, 0);
-      __builtin_amdgcn_sched_group_barrier(0x008, WaveCfg<W>::kFM * (BN / 64), 0);
-    };
-    const int total = (t1 - t0) * KT;
-    // prologue: slabs 0 .. NST-1 in flight, wait for slab 0
-    issue(smem);
-    if (total > 1) issue(smem + kSt);
-    if constexpr (NST == 3) {
-      if (total > 2) issue(smem + 2 * kSt);
+  // Direct-to-LDS pipeline over the workgroup's slabs s = 0, 1, ... (a run
+  // of column tiles times KT slabs each), LDS stage s & 1.  Per slab:
+  //   k-steps 0..2: MFMAs, with the fragments of the next k-step read
+  //                 from LDS behind them;
+  //   barrier B_s:  its implied vmcnt(0) / lgkmcnt(0) mean slab s+1's DMA
+  //                 (issued after B_{s-1}) has landed for every wave and no
+  //                 wave still reads slab s's stage;
+  //   then the DMA of slab s+2 into that stage and the first fragments of
+  //   slab s+1 are issued while the MFMAs of k-step 3 (whose fragments are
+  //   already in registers) run, so the barrier's read bubble is hidden.
+  constexpr int kSt = (kBM + BN) * kBK;  // elements of a stage
+  static_assert(NST >= 2 && NST <= 3, "LDS holds two or three stages");
+  // DMA wave instructions per wave per slab
+  constexpr int kD = (kBM + BN) / (8 * W);
+  auto frags = [&](const bf16_t* Sc, int kk, Frags<BN, W>& f) {
+    read_op<AK, kBM>(Sc, kk, wm * WaveCfg<W>::kWaveRows, f.a, l);
+    read_op<true, BN>(Sc + kBM * kBK, kk, wn * (BN / 2), f.b, l);
+  };
+  // DMA of the next unissued slab (tile it2, k-slab ik2) into stage S
+  int it2 = t0, ik2 = 0;
+  // A through a row map: its lane offsets are computed once per workgroup
+  static_assert(AK || !(AROW || KTAIL), "the row map and the K tail are for a K-major A");
+  static_assert(!(AROW && KTAIL), "a row-mapped A has whole slabs");
+  ARows<W> arows;
+  if constexpr (AROW) arows.init(g.A, g.lda, a_r0, g.M, g.arow, g.arows, w, l);
+  auto issue = [&](bf16_t* S) {
+    if constexpr (AROW)
+      arows.dma(ik2 * kBK, S, w);
+    else if constexpr (AK)
+      dma_kmajor<kBM, W, KTAIL>(g.A, g.lda, a_r0, g.M, ik2 * kBK, g.K, S, w, l);
+    else
+      dma_mnmajor<kBM, W>(g.A, g.lda, a_r0, ik2 * kBK, g.K, S, w, l);
+    dma_kmajor<BN, W, KTAIL>(g.B, g.ldb, it2 * BN, g.N, g.kb + ik2 * kBK, g.K, S + kBM * kBK, w, l);
+    if (++ik2 == KT) {
+      ik2 = 0;
+      ++it2;
     }
-    // wait for slab 0 only: after its DMA come those of slabs 1 .. NST-1
-    // (all issued when total > NST)
+  };
+  // The DMA's LDS writes count on vmcnt; the barrier's own fence does not
+  // reliably wait for them, so each barrier B_s that publishes slab s+1 is
+  // preceded by an explicit wait.  Vector memory operations retire in
+  // issue order, so B_s may leave in flight exactly what was issued after
+  // slab s+1's DMA: the DMAs of slabs s+2 .. s+NST-1, and the previous
+  // tile's epilogue stores for the first NST-1 slabs of a tile (they then
+  // drain behind the MFMAs).  Near the end of the run, where some of those
+  // DMAs were never issued, it waits for everything.  sched_barrier fences
+  // keep the MFMAs on their side of the barrier.
+  auto publish = [&](int s_, bool after_epilogue) {
     __builtin_amdgcn_sched_barrier(0);
-    if (total > NST)
-      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NST - 1) * kD) : "memory");
+    const bool deep = s_ + NST - 1 < ((t1 - t0) * KT);
+    if (deep && Epi::kStores > 0 && after_epilogue)
+      __builtin_amdgcn_s_waitcnt(vmcnt_imm((NST - 2) * kD + Epi::kStores));
+    else if (deep && NST > 2)
+      __builtin_amdgcn_s_waitcnt(vmcnt_imm((NST - 2) * kD));
     else
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     __builtin_amdgcn_sched_barrier(0);
-    Frags<BN, W> fa, fb;
-    frags(smem, 0, fa);
-    int s = 0, cur = 0;  // cur = s % NST
-    for (int tn = t0; tn < t1; ++tn) {
-      acc.zero();
-      for (int kt = 0; kt < KT; ++kt, ++s) {
-        const int nxt = (cur + 1 == NST) ? 0 : cur + 1;
-        bf16_t* const Sc = smem + cur * kSt;
-        bf16_t* const Sn = smem + nxt * kSt;
-        frags(Sc, 1, fb);
-        mfma_frags<BN, W>(fa, acc);
-        order();
-        frags(Sc, 2, fa);
-        mfma_frags<BN, W>(fb, acc);
-        order();
-        frags(Sc, 3, fb);
-        mfma_frags<BN, W>(fa, acc);
-        order();
-        publish(s, kt <= NST - 2 && tn != t0);  // B_s
-        // the next tile's first fragments are read after this tile's
-        // epilogue, so they are not live (24 VGPRs) while it runs
-        if (kt + 1 < KT) frags(Sn, 0, fa);
-        mfma_frags<BN, W>(fb, acc);
-        order();
-        __builtin_amdgcn_sched_barrier(0);
-        if (s + NST < total) issue(Sc);  // stage of slab s is free after B_s
-        cur = nxt;
-      }
-      Epi::tile(ep, st, acc, g, tm, tn, wm, wn, l, scratch);
-      if (tn + 1 < t1) frags(smem + cur * kSt, 0, fa);  // slab s+1, published at B_s
-    }
-    Epi::finish(ep, st, g, tm, split, smem, wm, wn, l);
-    return;
-  }
-
-  typename LoaderSel<AK, kBM, W>::type la0, la1;
-  typename LoaderSel<BKM, BN, W>::type lb0, lb1;
-  Frags<BN, W> f0, f1;
-
-  // One slab on LDS stage P.  LOAD: refill register set P with slab (nt, nk).
-  // DRAIN: store register set P^1 into stage P^1.  SYNC: close the slab with
-  // a barrier and read the first fragments of the next slab.
-  auto slab = [&](auto P, auto LOAD, auto DRAIN, auto SYNC, int nt, int nk) {
-    constexpr int p = decltype(P)::value;
-    bf16_t* const Sc = p ? S1 : S0;
-    bf16_t* const Sn = p ? S0 : S1;
-    auto& la = [&]() -> auto& { if constexpr (p == 0) return la0; else return la1; }();
-    auto& lb = [&]() -> auto& { if constexpr (p == 0) return lb0; else return lb1; }();
-    auto& la_n = [&]() -> auto& { if constexpr (p == 0) return la1; else return la0; }();
-    auto& lb_n = [&]() -> auto& { if constexpr (p == 0) return lb1; else return lb0; }();
-    if constexpr (decltype(LOAD)::value) {
-      la.load(g.A, g.lda, a_r0, g.M, nk * kBK, g.K, tid);
-      lb.load(g.B, g.ldb, nt * BN, g.N, nk * kBK, g.K, tid);
-    }
-    read_frags<BN, W>(Sc, Sc + kBM * kPitch, 1, f1, wm, wn, l);
-    mfma_frags<BN, W>(f0, acc);
-    if constexpr (decltype(DRAIN)::value) {
-      la_n.store(Sn, tid);
-      lb_n.store(Sn + kBM * kPitch, tid);
-    }
-    read_frags<BN, W>(Sc, Sc + kBM * kPitch, 2, f0, wm, wn, l);
-    mfma_frags<BN, W>(f1, acc);
-    read_frags<BN, W>(Sc, Sc + kBM * kPitch, 3, f1, wm, wn, l);
-    mfma_frags<BN, W>(f0, acc);
-    mfma_frags<BN, W>(f1, acc);
-    __builtin_amdgcn_iglp_opt(0);
-    if constexpr (decltype(SYNC)::value) {
-      __syncthreads();
-      read_frags<BN, W>(Sn, Sn + kBM * kPitch, 0, f0, wm, wn, l);
-    }
   };
-  typedef std::integral_constant<int, 0> I0;
-  typedef std::integral_constant<int, 1> I1;
-  typedef std::true_type T;
-  typedef std::false_type F;
-
-  // prologue: slabs 0 and 1 of tile t0 in flight, slab 0 in stage 0
-  la0.load(g.A, g.lda, a_r0, g.M, 0, g.K, tid);
-  lb0.load(g.B, g.ldb, t0 * BN, g.N, 0, g.K, tid);
-  la1.load(g.A, g.lda, a_r0, g.M, kBK, g.K, tid);
-  lb1.load(g.B, g.ldb, t0 * BN, g.N, kBK, g.K, tid);
-  la0.store(S0, tid);
-  lb0.store(S0 + kBM * kPitch, tid);
+  // each k-step: the next k-step's fragment reads are issued first, then
+  // the MFMAs they hide behind
+  auto order = [&]() {
+    constexpr int kReads = (AK ? 1 : 2) * WaveCfg<W>::kFM + BN / 64;
+    __builtin_amdgcn_sched_group_barrier(0x100, kReads, 0);
+    __builtin_amdgcn_sched_group_barrier(0x008, WaveCfg<W>::kFM * (BN / 64), 0);
+  };
+  const int total = (t1 - t0) * KT;
+  // prologue: slabs 0 .. NST-1 in flight, wait for slab 0
+  issue(smem);
+  if (total > 1) issue(smem + kSt);
+  if constexpr (NST == 3) {
+    if (total > 2) issue(smem + 2 * kSt);
+  }
+  // wait for slab 0 only: after its DMA come those of slabs 1 .. NST-1
+  // (all issued when total > NST)
+  __builtin_amdgcn_sched_barrier(0);
+  if (total > NST)
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NST - 1) * kD) : "memory");
+  else
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-  read_frags<BN, W>(S0, S0 + kBM * kPitch, 0, f0, wm, wn, l);
-
+  __builtin_amdgcn_sched_barrier(0);
+  Frags<BN, W> fa, fb;
+  frags(smem, 0, fa);
+  int s = 0, cur = 0;  // cur = s % NST
   for (int tn = t0; tn < t1; ++tn) {
     acc.zero();
-    const int kt_end = Epi::kMultiTile ? KT2 : KT2 - 2;
-    for (int kt = 0; kt < kt_end; kt += 2) {
-      const bool w0 = kt + 2 >= KT2, w1 = kt + 3 >= KT2;
-      slab(I0{}, T{}, T{}, T{}, w0 ? tn + 1 : tn, w0 ? kt + 2 - KT2 : kt + 2);
-      slab(I1{}, T{}, T{}, T{}, w1 ? tn + 1 : tn, w1 ? kt + 3 - KT2 : kt + 3);
-    }
-    if constexpr (!Epi::kMultiTile) {
-      // last slab pair of a single-tile workgroup: nothing left to load
-      slab(I0{}, F{}, T{}, T{}, 0, 0);
-      slab(I1{}, F{}, F{}, F{}, 0, 0);
+    for (int kt = 0; kt < KT; ++kt, ++s) {
+      const int nxt = (cur + 1 == NST) ? 0 : cur + 1;
+      bf16_t* const Sc = smem + cur * kSt;
+      bf16_t* const Sn = smem + nxt * kSt;
+      frags(Sc, 1, fb);
+      mfma_frags<BN, W>(fa, acc);
+      order();
+      frags(Sc, 2, fa);
+      mfma_frags<BN, W>(fb, acc);
+      order();
+      frags(Sc, 3, fb);
+      mfma_frags<BN, W>(fa, acc);
+      order();
+      publish(s, kt <= NST - 2 && tn != t0);  // B_s
+      // the next tile's first fragments are read after this tile's
+      // epilogue, so they are not live (24 VGPRs) while it runs
+      if (kt + 1 < KT) frags(Sn, 0, fa);
+      mfma_frags<BN, W>(fb, acc);
+      order();
+      __builtin_amdgcn_sched_barrier(0);
+      if (s + NST < total) issue(Sc);  // stage of slab s is free after B_s
+      cur = nxt;
     }
     Epi::tile(ep, st, acc, g, tm, tn, wm, wn, l, scratch);
+    if (tn + 1 < t1) frags(smem + cur * kSt, 0, fa);  // slab s+1, published at B_s
   }
   Epi::finish(ep, st, g, tm, split, smem, wm, wn, l);
 }
 
-template <int BN, int W, bool AK, bool BKM, template <int, int> class EpiT, int PIPE, int NST = 2, bool AROW = false>
+template <int BN, int W, bool AK, template <int, int> class EpiT, int NST = 2, bool AROW = false, bool KTAIL = false>
 __global__ __launch_bounds__(W * 64) void gemm_kernel(GemmShape g, typename EpiT<BN, W>::Params ep) {
-  __shared__ __attribute__((aligned(16))) bf16_t smem[gemm_lds_elems<BN>(PIPE, NST) + EpiT<BN, W>::kScratch];
-  gemm_body<BN, W, AK, BKM, EpiT, PIPE, NST, AROW>(g, ep, blockIdx.x, gridDim.x, smem);
+  __shared__ __attribute__((aligned(16))) bf16_t smem[gemm_lds_elems<BN>(NST) + EpiT<BN, W>::kScratch];
+  gemm_body<BN, W, AK, EpiT, NST, AROW, KTAIL>(g, ep, blockIdx.x, gridDim.x, smem);
 }
 
-// dW and dH GEMMs of one vocabulary band in a single launch.  The first
-// nb_dw workgroups take dW tiles (K = N, the longer ones), the rest dH tiles
-// (K = band width), so the two tile populations pack the CUs together where
-// each alone would leave a partial last wave.
-template <int W, int BN_DW, int PIPE_DW, int BN_DH, int PIPE_DH>
-__global__ __launch_bounds__(W * 64) void dual_acc_kernel(GemmShape g_dw, AccParams e_dw, int nb_dw, GemmShape g_dh,
-                                                          AccParams e_dh) {
-  constexpr int kMaxBN = BN_DW > BN_DH ? BN_DW : BN_DH;
-  __shared__ __attribute__((aligned(16))) bf16_t smem[2 * (kBM + kMaxBN) * kPitch];
-  if ((int)blockIdx.x < nb_dw)
-    gemm_body<BN_DW, W, false, true, EpiAcc, PIPE_DW>(g_dw, e_dw, blockIdx.x, nb_dw, smem);
-  else
-    gemm_body<BN_DH, W, true, true, EpiAcc, PIPE_DH>(g_dh, e_dh, blockIdx.x - nb_dw, gridDim.x - nb_dw, smem);
-}
-
-// One launch per vocabulary band b of the backward (d a multiple of 64): the
+// One launch per vocabulary band b of the backward: the
 // dW and dH GEMMs of band b and the logits recompute of band b+1, which
 // writes the other G buffer.  Both gradient GEMMs tile d in 256-wide column
 // tiles plus one 128-wide tail tile when d % 256 <= 128 (no MFMA work spent
@@ -1175,7 +950,7 @@ __global__ __launch_bounds__(W * 64) void dual_acc_kernel(GemmShape g_dw, AccPar
 // the GEMM epilogue applies an unsplit tile: 0 out = s, 1 acc = s,
 // 2 acc += s, 3 out = acc + s, 4 out += s (fp32 out); out rows go through the
 // row map.  The rows are a block starting at row live_base of the compacted
-// order (P, acc and rowmap point at the block).  d % 64 == 0.
+// order (P, acc and rowmap point at the block).
 struct DhReduce {
   const float* P;
   long stride;
@@ -1263,7 +1038,7 @@ __device__ inline void dh_split_body(const GemmShape& g0, const AccParams& e0, i
   g.B += k0;
   g.K = min(kc, g0.K - k0);
   e.acc32 += k * stride;
-  gemm_body<BN, kWarp8, true, true, EpiAcc, 4, NST>(g, e, b / ks, nb / ks, smem);
+  gemm_body<BN, kWarp8, true, EpiAcc, NST>(g, e, b / ks, nb / ks, smem);
 }
 
 template <int NT>
@@ -1271,42 +1046,43 @@ __device__ inline void transpose_tile(const bf16_t* __restrict__ in, long ldi, i
                                       long ldo, int Rpad, int r0, int c0, bf16_t (*t)[66], int tid,
                                       const int* __restrict__ rmap);
 
-// AROW: the recompute reads H's rows through the row order.
-template <bool HB, bool AROW>
+// HB: with a bias.  AROW: the recompute reads H's rows through the row order.
+// KTAIL: d is no multiple of 64 (the recompute's K).
+template <bool HB, bool AROW, bool KTAIL>
 __global__ __launch_bounds__(kWarp8 * 64) void band_kernel(BandLaunch p) {
-  __shared__ __attribute__((aligned(16))) bf16_t smem[gemm_lds_elems<kFastBN>(4) + EpiGrad<kFastBN, kWarp8>::kScratch];
+  __shared__ __attribute__((aligned(16))) bf16_t smem[gemm_lds_elems<kBN>() + EpiGrad<kBN, kWarp8>::kScratch];
   int b = blockIdx.x;
   if (b < p.nb_dw) {
-    gemm_body<kFastBN, kWarp8, false, true, EpiAcc, 5>(p.dw, p.e_dw, b, p.nb_dw, smem);
+    gemm_body<kBN, kWarp8, false, EpiAcc>(p.dw, p.e_dw, b, p.nb_dw, smem);
     return;
   }
   b -= p.nb_dw;
   if (b < p.nb_dw2) {
-    gemm_body<kSlowBN, kWarp8, false, true, EpiAcc, 5, 3>(p.dw2, p.e_dw2, b, p.nb_dw2, smem);
+    gemm_body<kTailBN, kWarp8, false, EpiAcc, 3>(p.dw2, p.e_dw2, b, p.nb_dw2, smem);
     return;
   }
   b -= p.nb_dw2;
   if (b < p.nb_dh) {
     if (p.dh_split)
-      dh_split_body<kFastBN, 2>(p.dh, p.e_dh_part, p.dh_ks, p.dh_kc, p.dh_part_stride, b, p.nb_dh, smem);
+      dh_split_body<kBN, 2>(p.dh, p.e_dh_part, p.dh_ks, p.dh_kc, p.dh_part_stride, b, p.nb_dh, smem);
     else
-      gemm_body<kFastBN, kWarp8, true, true, EpiAcc, 4>(p.dh, p.e_dh, b, p.nb_dh, smem);
+      gemm_body<kBN, kWarp8, true, EpiAcc>(p.dh, p.e_dh, b, p.nb_dh, smem);
     return;
   }
   b -= p.nb_dh;
   if (b < p.nb_dh2) {
     if (p.dh_split)
-      dh_split_body<kSlowBN, 3>(p.dh2, p.e_dh2_part, p.dh_ks, p.dh_kc, p.dh_part_stride, b, p.nb_dh2, smem);
+      dh_split_body<kTailBN, 3>(p.dh2, p.e_dh2_part, p.dh_ks, p.dh_kc, p.dh_part_stride, b, p.nb_dh2, smem);
     else
-      gemm_body<kSlowBN, kWarp8, true, true, EpiAcc, 4, 3>(p.dh2, p.e_dh2, b, p.nb_dh2, smem);
+      gemm_body<kTailBN, kWarp8, true, EpiAcc, 3>(p.dh2, p.e_dh2, b, p.nb_dh2, smem);
     return;
   }
   b -= p.nb_dh2;
   if (b < p.nb_gr) {
     if constexpr (HB)
-      gemm_body<kFastBN, kWarp8, true, true, EpiGradBias, 4, 2, AROW>(p.gr, p.e_gr, b, p.nb_gr, smem);
+      gemm_body<kBN, kWarp8, true, EpiGradBias, 2, AROW, KTAIL>(p.gr, p.e_gr, b, p.nb_gr, smem);
     else
-      gemm_body<kFastBN, kWarp8, true, true, EpiGrad, 4, 2, AROW>(p.gr, p.e_gr, b, p.nb_gr, smem);
+      gemm_body<kBN, kWarp8, true, EpiGrad, 2, AROW, KTAIL>(p.gr, p.e_gr, b, p.nb_gr, smem);
     return;
   }
   b -= p.nb_gr;
@@ -2131,8 +1907,7 @@ struct Carver {
 
 // Forward vocabulary splits: enough (row tile x split) workgroups to cover
 // the 256 CUs several times over.
-bool fast_k(long K) { return K % 64 == 0; }
-int lse_bn(long d) { return fast_k(d) ? kFastBN : kSlowBN; }
+bool whole_slabs(long d) { return d % kBK == 0; }
 
 // Vocabulary splits per row tile of a forward over every row tile: about 512
 // workgroups for few row tiles (runs of several vocabulary tiles, so the
@@ -2140,7 +1915,7 @@ int lse_bn(long d) { return fast_k(d) ? kFastBN : kSlowBN; }
 // min(32, 2048 / row tiles): large batches keep their split counts.
 int forward_splits(long N, long d, long V) {
   if (N <= 0) return 1;
-  const long gm = ceil_div(N, kBM), tn = ceil_div(V, lse_bn(d));
+  const long gm = ceil_div(N, kBM), tn = ceil_div(V, kBN);
   long s = std::max(ceil_div(512, gm), std::min<long>(32, ceil_div(2048, gm)));
   if (s > tn) s = tn;
   if (s < 1) s = 1;
@@ -2160,7 +1935,7 @@ long forward_slots(long N, long d, long V, bool compact) {
   const long gm = ceil_div(std::max<long>(N, 1), kBM);
   const long base = gm * forward_splits(N, d, V);
   if (!compact) return base;
-  const long tn = ceil_div(V, lse_bn(d));
+  const long tn = ceil_div(V, kBN);
   return std::max(base, std::min(gm * std::min<long>(64, tn), 8192L));
 }
 
@@ -2235,11 +2010,12 @@ long block_rows(long N, long Vb) {
 // whose scratch is fixed) reads in place wherever the offsets allow.
 // CHRONICALS_CCE_ROW_GATHER=0 forces the copy, =1 reads in place wherever the
 // offsets allow (read on every call, so a workspace query and the call it
-// sizes must see the same value).
+// sizes must see the same value).  With d no multiple of 64 only the gathered
+// copy is read (the row map takes whole slabs).
 constexpr long kInPlaceMinBytes = 256L << 20;
 bool rows_in_place(long N, long d, bool prefer = false) {
   const long bytes = N * d * 2;
-  if (bytes > 0x7ffffff0L) return false;
+  if (bytes > 0x7ffffff0L || !whole_slabs(d)) return false;
   const char* e = getenv("CHRONICALS_CCE_ROW_GATHER");
   if (e && (e[0] == '0' || e[0] == '1') && e[1] == 0) return e[0] == '1';
   return prefer || bytes >= kInPlaceMinBytes;
@@ -2270,7 +2046,7 @@ int wsum_splits(long d, long V) {
 
 // The forward compacts its rows when only the labelled rows' lse is wanted
 // and the direct-to-LDS GEMM runs (d a multiple of 64).
-bool fwd_compacts(long d, int lse_rows) { return lse_rows == CCE_LSE_LABELLED_ROWS && fast_k(d); }
+bool fwd_compacts(long d, int lse_rows) { return lse_rows == CCE_LSE_LABELLED_ROWS && whole_slabs(d); }
 
 FwdLayout fwd_layout(void* ws, long N, long d, long V, int reduction, int lse_rows, bool prefer_in_place = false) {
   Carver c(ws);
@@ -2304,8 +2080,8 @@ struct BwdLayout {
   bf16_t* G[2];   // band gradient of a block; the second only when units alternate
   bf16_t* WT[2];  // W band transposes; the second only when bands alternate
   bf16_t* HT;
-  // Caller output memory that is not yet written doubles as scratch (banded
-  // backward, bf16 dH and dW wanted, several bands):
+  // Caller output memory that is not yet written doubles as scratch (bf16 dH
+  // and dW wanted, several bands):
   //  - ht_out: H^T ([d][N], N a multiple of 64) lives in grad_hidden, which
   //    the bands leave unwritten: the last band adds into the fp32 dH
   //    accumulator, and dH goes to grad_hidden after the last band launch;
@@ -2320,7 +2096,7 @@ struct BwdLayout {
   bool ht_out, wt_out, wt_last_in_place, wt_dh, dh_late;
   float* dHacc;   // dH over the bands (bf16 dH with several bands; fp32 dH accumulates in place)
   float* dWacc;   // dW of a band over the row blocks (bf16 dW with several blocks)
-  // row compaction (banded backward): row order, live row count, and H in
+  // row compaction: row order, live row count, and H in
   // that order when the GEMMs cannot read H through the row order
   int* idx;
   int* live;
@@ -2333,11 +2109,7 @@ struct BwdLayout {
   size_t bytes;
 };
 
-// The banded backward with the band kernel (d a multiple of 64) overlaps the
-// recompute of band b+1 with the dW / dH GEMMs of band b: two G buffers.
-bool banded(long d) { return d % 64 == 0; }
-
-// Hidden columns of the banded backward's 256-wide dW / dH tiles; the rest,
+// Hidden columns of the backward's 256-wide dW / dH tiles; the rest,
 // when d % 256 <= 128, is one 128-wide tail tile.
 long band_dmain(long d) { return (d % 256 == 0 || d % 256 > 128) ? d : d - d % 256; }
 
@@ -2346,16 +2118,16 @@ long band_dmain(long d) { return (d % 256 == 0 || d % 256 > 128) ? d : d - d % 2
 // buffers, alternating); with 2-3 splits it is a launch of its own.
 bool dh_fold(int ks) { return ks >= 4; }
 
-// K splits of the banded dH.  dH has one tile per (256-row tile, hidden
+// K splits of dH.  dH has one tile per (256-row tile, hidden
 // column tile), each reducing over the whole band; with few rows those tiles
 // cannot fill the CUs and the band launch waits on their long K loops.  Then
 // K is split so that tiles x splits reaches about 128 workgroups, with at
 // least 8 slabs of 64 per split (more splits cost more in the fp32 partials'
 // reduction than their shorter K loops return).
 int dh_splits(long N, long d, long Vb) {
-  if (!banded(d) || N <= 0 || d <= 0) return 1;
+  if (N <= 0 || d <= 0) return 1;
   const long dmain = band_dmain(d);
-  const long tiles = ceil_div(N, kBM) * (ceil_div(dmain, kFastBN) + (dmain < d ? 1 : 0));
+  const long tiles = ceil_div(N, kBM) * (ceil_div(dmain, kBN) + (dmain < d ? 1 : 0));
   if (tiles <= 0 || tiles >= 128) return 1;
   const long ks = std::min<long>(ceil_div(128, tiles), Vb / 512);
   return ks < 2 ? 1 : (int)ks;
@@ -2379,23 +2151,22 @@ BwdLayout bwd_layout(void* ws, long N, long d, long V, long Vb, bool need_dh, bo
   const long N64 = ht_cols(N);
   L.rowp = c.take<float4>((size_t)N);
   L.rowlab = c.take<int>((size_t)N);
-  L.ht_out = banded(d) && need_dh && need_dw && !dh_f32 && nbands > 1 && N % 64 == 0;
-  L.wt_out = banded(d) && need_dh && need_dw && nbands > 1;
+  L.ht_out = need_dh && need_dw && !dh_f32 && nbands > 1 && N % 64 == 0;
+  L.wt_out = need_dh && need_dw && nbands > 1;
   L.wt_last_in_place = L.wt_out && L.nblocks > 1 && !dw_f32;
-  L.wt_dh = banded(d) && need_dh && !need_dw && !dh_f32 && nbands > 1 && N >= 2 * Vb;
+  L.wt_dh = need_dh && !need_dw && !dh_f32 && nbands > 1 && N >= 2 * Vb;
   L.dh_late = L.ht_out || L.wt_dh;
   L.G[0] = c.take<bf16_t>((size_t)L.Nb * Vb);
-  L.G[1] = (banded(d) && units > 1) ? c.take<bf16_t>((size_t)L.Nb * Vb) : L.G[0];
+  L.G[1] = (units > 1) ? c.take<bf16_t>((size_t)L.Nb * Vb) : L.G[0];
   L.WT[0] = need_dh && !L.wt_last_in_place && !L.wt_dh ? c.take<bf16_t>((size_t)d * Vb) : nullptr;
-  L.WT[1] = (need_dh && banded(d) && nbands > 1 && !L.wt_out && !L.wt_dh) ? c.take<bf16_t>((size_t)d * Vb)
+  L.WT[1] = (need_dh && nbands > 1 && !L.wt_out && !L.wt_dh) ? c.take<bf16_t>((size_t)d * Vb)
                                                                           : L.WT[0];
   L.HT = need_dw && !L.ht_out ? c.take<bf16_t>((size_t)d * N64) : nullptr;
   L.dHacc = (need_dh && nbands > 1 && !dh_f32) ? c.take<float>((size_t)N * d) : nullptr;
   L.dWacc = (need_dw && L.nblocks > 1 && !dw_f32) ? c.take<float>((size_t)Vb * d) : nullptr;
-  const bool compact = banded(d);
-  L.idx = compact ? c.take<int>((size_t)N) : nullptr;
-  L.live = compact ? c.take<int>(1) : nullptr;
-  L.Hc = compact && !rows_in_place(N, d) ? c.take<bf16_t>((size_t)N * d) : nullptr;
+  L.idx = c.take<int>((size_t)N);
+  L.live = c.take<int>(1);
+  L.Hc = !rows_in_place(N, d) ? c.take<bf16_t>((size_t)N * d) : nullptr;
   L.dh_ks = need_dh ? dh_splits(L.Nb, d, Vb) : 1;
   // a second partial buffer only when the reduction rides in the next
   // launch (dh_fold); otherwise each unit's reduction runs before the next
@@ -2413,9 +2184,12 @@ bool misaligned(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) !
 // operand row must hold every slab the GEMM reads: kb + K rounded up to 64
 // columns at most ld.  Checked on the host before each launch; a layout that
 // broke it would otherwise read past the operand.
-bool kmajor_fits(long ld, long kb, long K) { return K <= 0 || kb + (long)align_up((size_t)K, kBK) <= ld; }
-int check_kmajor(const GemmShape& g, bool a_kmajor) {
-  if ((a_kmajor && !kmajor_fits(g.lda, 0, g.K)) || !kmajor_fits(g.ldb, g.kb, g.K))
+// With ktail (dma_kmajor's KTAIL) the columns from K on are not read.
+bool kmajor_fits(long ld, long kb, long K, bool ktail = false) {
+  return K <= 0 || kb + (ktail ? K : (long)align_up((size_t)K, kBK)) <= ld;
+}
+int check_kmajor(const GemmShape& g, bool a_kmajor, bool ktail = false) {
+  if ((a_kmajor && !kmajor_fits(g.lda, 0, g.K, ktail)) || !kmajor_fits(g.ldb, g.kb, g.K, ktail))
     return fail(CCE_ERR_INVALID_ARG, "internal: a K-major operand row (lda %ld, ldb %ld) is shorter than the "
                 "slabs of K = %d at k offset %d", g.lda, g.ldb, g.K, g.kb);
   return CCE_OK;
@@ -2478,18 +2252,15 @@ double gemm_flops(long M, long N, long K) { return 2.0 * (double)M * (double)N *
 
 // A GEMM launch; `credited` is the algorithmic share of its FLOPs (the
 // logits recompute of the backward is executed but not credited).
-template <int BN, int W, bool AK, bool BK, template <int, int> class EpiT, int PIPE = 3, int NST = 2,
-          bool AROW = false>
+template <int BN, int W, template <int, int> class EpiT, bool AROW = false, bool KTAIL = false>
 int launch_gemm(const GemmShape& g, const typename EpiT<BN, W>::Params& ep, int nblocks, hipStream_t st,
                 int kind, bool credited) {
   if (nblocks <= 0) return CCE_OK;
-  if (PIPE >= 4) {
-    const int rc = check_kmajor(g, AK);
-    if (rc) return rc;
-  }
+  const int rc = check_kmajor(g, true, KTAIL);
+  if (rc) return rc;
   hipEvent_t e0 = nullptr, e1 = nullptr;
   const bool timed = timing_begin(st, &e0, &e1);
-  hipLaunchKernelGGL((gemm_kernel<BN, W, AK, BK, EpiT, PIPE, NST, AROW>), dim3(nblocks), dim3(W * 64), 0, st, g, ep);
+  hipLaunchKernelGGL((gemm_kernel<BN, W, true, EpiT, 2, AROW, KTAIL>), dim3(nblocks), dim3(W * 64), 0, st, g, ep);
   HIP_TRY(hipGetLastError());
   if (timed) {
     const double f = gemm_flops(g.M, g.N, g.K);
@@ -2510,35 +2281,6 @@ int zero_fill(void* p, size_t bytes, hipStream_t st) {
   return CCE_OK;
 }
 
-
-int launch_dual_acc(const GemmShape& g_dw, const AccParams& e_dw, const GemmShape& g_dh, const AccParams& e_dh,
-                    hipStream_t st) {
-  // dH operands are K-major with K a multiple of 64 (the band is zero-padded);
-  // dW reads G transposed from LDS (its K tail reads as zero past row N)
-  constexpr int kBNdw = kSlowBN, kBNdh = kFastBN;
-  const int nb_dw = (int)(ceil_div(g_dw.M, kBM) * ceil_div(g_dw.N, kBNdw));
-  const int nb_dh = (int)(ceil_div(g_dh.M, kBM) * ceil_div(g_dh.N, kBNdh));
-  if (nb_dw + nb_dh <= 0) return CCE_OK;
-  int rc = nb_dw ? check_kmajor(g_dw, false) : CCE_OK;
-  if (!rc && nb_dh) rc = check_kmajor(g_dh, true);
-  if (rc) return rc;
-  hipEvent_t t0 = nullptr, t1 = nullptr;
-  const bool timed = timing_begin(st, &t0, &t1);
-  hipLaunchKernelGGL((dual_acc_kernel<kWarp8, kBNdw, 5, kBNdh, 4>), dim3(nb_dw + nb_dh), dim3(kWarp8 * 64), 0, st,
-                     g_dw, e_dw, nb_dw, g_dh, e_dh);
-  HIP_TRY(hipGetLastError());
-  if (timed) {
-    const double f = gemm_flops(g_dw.M, g_dw.N, g_dw.K) + gemm_flops(g_dh.M, g_dh.N, g_dh.K);
-    timing_end(CCE_KERNEL_BWD_DHDW, st, t0, t1, f, f);
-  }
-  return CCE_OK;
-}
-
-template <int BN, bool AK, int PIPE>
-int launch_acc(const GemmShape& g, const AccParams& ep, hipStream_t st, int kind) {
-  const int nb = (int)(ceil_div(g.M, kBM) * ceil_div(g.N, BN));
-  return launch_gemm<BN, kWarp8, AK, true, EpiAcc, PIPE>(g, ep, nb, st, kind, true);
-}
 
 // Recompute launch shape of one unit: G[n][c] for the rows [m0, m0 + rows)
 // of the compacted order (a row block) and columns [v0, v0 + vb).
@@ -2575,19 +2317,16 @@ int launch_band(const BandLaunch& p, bool has_bias, hipStream_t st, int kind = C
   if (!rc && p.nb_dw2) rc = check_kmajor(p.dw2, false);
   if (!rc && p.nb_dh) rc = check_kmajor(p.dh, true);
   if (!rc && p.nb_dh2) rc = check_kmajor(p.dh2, true);
-  if (!rc && p.nb_gr) rc = check_kmajor(p.gr, true);
+  const bool ktail = !whole_slabs(p.gr.K);
+  if (!rc && p.nb_gr) rc = check_kmajor(p.gr, true, ktail);
   if (rc) return rc;
   hipEvent_t t0 = nullptr, t1 = nullptr;
   const bool timed = timing_begin(st, &t0, &t1);
   const bool arow = p.gr.arow != nullptr;
-  if (has_bias && arow)
-    hipLaunchKernelGGL((band_kernel<true, true>), dim3(nb), dim3(kWarp8 * 64), 0, st, p);
-  else if (has_bias)
-    hipLaunchKernelGGL((band_kernel<true, false>), dim3(nb), dim3(kWarp8 * 64), 0, st, p);
-  else if (arow)
-    hipLaunchKernelGGL((band_kernel<false, true>), dim3(nb), dim3(kWarp8 * 64), 0, st, p);
-  else
-    hipLaunchKernelGGL((band_kernel<false, false>), dim3(nb), dim3(kWarp8 * 64), 0, st, p);
+  auto* const kernel = ktail ? (has_bias ? band_kernel<true, false, true> : band_kernel<false, false, true>)
+                       : arow ? (has_bias ? band_kernel<true, true, false> : band_kernel<false, true, false>)
+                              : (has_bias ? band_kernel<true, false, false> : band_kernel<false, false, false>);
+  hipLaunchKernelGGL(kernel, dim3(nb), dim3(kWarp8 * 64), 0, st, p);
   HIP_TRY(hipGetLastError());
   if (timed) {
     double cr = 0.0;
@@ -2676,7 +2415,7 @@ int forward_run(const void* hidden, const void* weight, const void* labels, int 
   // over the row tiles that hold them (the partials then follow that order)
   if (L.idx) {
     hipLaunchKernelGGL(compact_rows_kernel, dim3(1), dim3(1024), 0, st, labels, labels_int64, (int)N,
-                       (long)ignore_index, L.idx, L.live, slots, (int)ceil_div(V, lse_bn(d)), device_cus());
+                       (long)ignore_index, L.idx, L.live, slots, (int)ceil_div(V, kBN), device_cus());
     HIP_TRY(hipGetLastError());
     if (L.Hc) {
       const long chunks = (long)N * (d / 8);
@@ -2706,18 +2445,17 @@ int forward_run(const void* hidden, const void* weight, const void* labels, int 
   ep.ps = L.ps;
   ep.ldp = N;
   ep.splits = S;
-  ep.tiles_n = (int)ceil_div(V, lse_bn(d));
-  if (fast_k(d) && g.arow)
-    rc = bias ? launch_gemm<kFastBN, kWarp8, true, true, EpiLseBias, 4, 2, true>(g, ep, slots, st,
-                                                                                CCE_KERNEL_FWD_LSE, true)
-              : launch_gemm<kFastBN, kWarp8, true, true, EpiLse, 4, 2, true>(g, ep, slots, st, CCE_KERNEL_FWD_LSE,
-                                                                            true);
-  else if (fast_k(d))
-    rc = bias ? launch_gemm<kFastBN, kWarp8, true, true, EpiLseBias, 4>(g, ep, slots, st, CCE_KERNEL_FWD_LSE, true)
-              : launch_gemm<kFastBN, kWarp8, true, true, EpiLse, 4>(g, ep, slots, st, CCE_KERNEL_FWD_LSE, true);
+  ep.tiles_n = (int)ceil_div(V, kBN);
+  constexpr int kKind = CCE_KERNEL_FWD_LSE;
+  if (!whole_slabs(d))
+    rc = bias ? launch_gemm<kBN, kWarp8, EpiLseBias, false, true>(g, ep, slots, st, kKind, true)
+              : launch_gemm<kBN, kWarp8, EpiLse, false, true>(g, ep, slots, st, kKind, true);
+  else if (g.arow)
+    rc = bias ? launch_gemm<kBN, kWarp8, EpiLseBias, true>(g, ep, slots, st, kKind, true)
+              : launch_gemm<kBN, kWarp8, EpiLse, true>(g, ep, slots, st, kKind, true);
   else
-    rc = bias ? launch_gemm<kSlowBN, kWarp8, true, true, EpiLseBias, 3>(g, ep, slots, st, CCE_KERNEL_FWD_LSE, true)
-              : launch_gemm<kSlowBN, kWarp8, true, true, EpiLse, 3>(g, ep, slots, st, CCE_KERNEL_FWD_LSE, true);
+    rc = bias ? launch_gemm<kBN, kWarp8, EpiLseBias>(g, ep, slots, st, kKind, true)
+              : launch_gemm<kBN, kWarp8, EpiLse>(g, ep, slots, st, kKind, true);
   if (rc) return rc;
 
   const bool uniform = smoothing_form == CCE_SMOOTH_UNIFORM && label_smoothing > 0.f;
@@ -3057,208 +2795,165 @@ int cce_backward(const float* grad_out, const void* hidden, const void* weight, 
     grad_shape(H, W, bias, L, L.G[u & 1], m0, rows, d, v0, vb, bn, in_band, g, e, nb);
   };
 
-  if (banded(d)) {
-    // launch u: dW and dH of unit u from G[u & 1] and the recompute of unit
-    // u+1 into G[(u+1) & 1]; unit 0's recompute runs alone first.
-    const long dmain = band_dmain(d);
-    {
-      GemmShape g1 = {};
-      GradParams e1 = {};
-      int nb1 = 0;
-      grad_unit(0, false, kFastBN, g1, e1, nb1);
-      if (g1.arow) {
-        // reading H through the row order: run it as a band launch with only
-        // this recompute population (the stand-alone GEMM kernel with the row
-        // map spills registers; the band kernel's allocation does not)
-        BandLaunch p0 = {};
-        p0.gr = g1;
-        p0.e_gr = e1;
-        p0.nb_gr = nb1;
-        rc = launch_band(p0, bias != nullptr, st, CCE_KERNEL_BWD_GRAD);
-      } else
-        rc = bias ? launch_gemm<kFastBN, kWarp8, true, true, EpiGradBias, 4>(g1, e1, nb1, st, CCE_KERNEL_BWD_GRAD,
-                                                                              false)
-                  : launch_gemm<kFastBN, kWarp8, true, true, EpiGrad, 4>(g1, e1, nb1, st, CCE_KERNEL_BWD_GRAD, false);
-      if (rc) return rc;
-      if (need_dh) {
-        rc = transpose_band(0);
-        if (rc) return rc;
-      }
-    }
-    // With 4 or more splits (very few rows) the band launches are short and the
-    // reduction rides in the next launch, so the partials alternate between
-    // two buffers; with 2-3 splits the launches are full and it runs as a
-    // launch of its own after each unit, on the one buffer.
-    const bool fold = L.dhpart && dh_fold(L.dh_ks);
-    auto dh_part = [&](long u) { return L.dhpart + (fold ? (u & 1) : 0) * (long)L.dh_ks * Nb * d; };
-    // the reduction of unit u's K-split dH partials, with its band's
-    // accumulator mode (as dh_shape sets it)
-    auto dh_reduction = [&](long u, int ks) {
-      const long b = u / R;
-      long m0, rows;
-      block_span(u % R, m0, rows);
-      DhReduce r;
-      r.P = dh_part(u);
-      r.stride = Nb * d;
-      r.ks = ks; r.N = (int)rows; r.d = (int)d;
-      r.live = L.live; r.live_base = (int)m0;
-      r.acc = L.dHacc ? L.dHacc + m0 * d : nullptr;
-      r.mode = dh_mode(b);
-      r.out = L.idx ? grad_hidden
-                    : (dh_f32 ? static_cast<void*>(static_cast<float*>(grad_hidden) + m0 * d)
-                              : static_cast<void*>(static_cast<bf16_t*>(grad_hidden) + m0 * d));
-      r.out_f32 = dh_f32;
-      r.rowmap = L.idx ? L.idx + m0 : nullptr;
-      return r;
-    };
-    int prev_ks = 1;
-    for (long u = 0; u < units; ++u) {
-      const long b = u / R, r = u % R;
-      const bf16_t* G = L.G[u & 1];
-      BandLaunch p = {};
-      if (need_dw) {
-        if (dmain > 0) {
-          dw_shape(b, r, G, 0, dmain, p.dw, p.e_dw);
-          p.nb_dw = (int)(ceil_div(p.dw.M, kBM) * ceil_div(dmain, kFastBN));
-        }
-        if (dmain < d) {
-          dw_shape(b, r, G, dmain, d - dmain, p.dw2, p.e_dw2);
-          p.nb_dw2 = (int)(ceil_div(p.dw2.M, kBM) * ceil_div(d - dmain, kSlowBN));
-        }
-      }
-      if (need_dh) {
-        // the next band's W rows, transposed into the other WT buffer by the
-        // band's first launch (band b reads WT[b & 1] in all its launches);
-        // the last band's W^T, when it takes the memory that this band's
-        // W^T occupies (wt_last_in_place), by a launch of its own once this
-        // band is done
-        const bool tr_late = L.wt_last_in_place && b + 2 == nbands;
-        if (r == 0 && b + 1 < nbands && !tr_late) p.nb_tr = transpose_params(b + 1, p.tr);
-        long m0, rows;
-        block_span(r, m0, rows);
-        const int gm = (int)ceil_div(rows, kBM);
-        // K splits of this unit: every split non-empty and a whole number of slabs
-        int ks = 1;
-        if (L.dhpart) {
-          long v0, vb, vb64;
-          band_cols(b, v0, vb, vb64);
-          p.dh_kc = (int)align_up((size_t)ceil_div(vb64, L.dh_ks), 64);
-          ks = (int)ceil_div(vb64, p.dh_kc);
-        }
-        p.dh_split = L.dhpart != nullptr;  // every unit, even one left with a single split
-        p.dh_ks = ks;
-        p.dh_part_stride = Nb * d;
-        float* const part = L.dhpart ? dh_part(u) : nullptr;
-        if (dmain > 0) {
-          dh_shape(b, r, G, 0, dmain, p.dh, p.e_dh);
-          p.nb_dh = gm * (int)ceil_div(dmain, kFastBN) * ks;
-          p.e_dh_part = p.e_dh;
-          p.e_dh_part.acc32 = part; p.e_dh_part.ldacc = d; p.e_dh_part.mode = 1; p.e_dh_part.rowmap = nullptr;
-        }
-        if (dmain < d) {
-          dh_shape(b, r, G, dmain, d - dmain, p.dh2, p.e_dh2);
-          p.nb_dh2 = gm * (int)ceil_div(d - dmain, kSlowBN) * ks;
-          p.e_dh2_part = p.e_dh2;
-          p.e_dh2_part.acc32 = part ? part + dmain : nullptr; p.e_dh2_part.ldacc = d;
-          p.e_dh2_part.mode = 1; p.e_dh2_part.rowmap = nullptr;
-        }
-        // the previous unit's partials (the other buffer) into the accumulator
-        if (fold && u > 0) {
-          p.red = dh_reduction(u - 1, prev_ks);
-          long pm0, prows;
-          block_span((u - 1) % R, pm0, prows);
-          p.nb_red = (int)std::min<long>(ceil_div(prows * (d / 4), kWarp8 * 64 * 4), 1024);
-        }
-        prev_ks = ks;
-      }
-      if (u + 1 < units) grad_unit(u + 1, true, kFastBN, p.gr, p.e_gr, p.nb_gr);
-      rc = launch_band(p, bias != nullptr, st);
-      if (rc) return rc;
-      if (need_dh && L.dhpart && (!fold || u + 1 == units)) {
-        // this unit's partials (the last band's go to the output: mode 0, 3 or 4)
-        long m0, rows;
-        block_span(r, m0, rows);
-        hipLaunchKernelGGL(dh_reduce_kernel, dim3((unsigned)std::min<long>(ceil_div(rows * (d / 4), 256), 2048)),
-                           dim3(256), 0, st, dh_reduction(u, prev_ks));
-        HIP_TRY(hipGetLastError());
-      }
-      if (need_dh && L.wt_last_in_place && b + 2 == nbands && r == R - 1) {
-        rc = transpose_band(b + 1);
-        if (rc) return rc;
-      }
-      if (need_db) {
-        rc = colsum_unit(b, r, G);
-        if (rc) return rc;
-      }
-    }
-    // outputs whose memory held W^T / H^T during the bands: the last band's
-    // dW from its fp32 accumulator, then dH (the labelled rows) through the
-    // row map; the rows without a label are zeroed last
-    auto convert = [&](const float* src, long rows, const int* live, const int* rowmap, void* out) {
-      DhReduce c = {};
-      c.P = src;
-      c.ks = 1;
-      c.N = (int)rows; c.d = (int)d;
-      c.live = live; c.live_base = 0;
-      c.mode = 0;
-      c.out = out; c.out_f32 = 0;
-      c.rowmap = rowmap;
-      hipLaunchKernelGGL(dh_reduce_kernel, dim3((unsigned)std::min<long>(ceil_div(rows * (d / 4), 256), 2048)),
-                         dim3(256), 0, st, c);
-      return hipGetLastError();
-    };
-    if (L.wt_last_in_place) {
-      long v0, vb, vb64;
-      band_cols(nbands - 1, v0, vb, vb64);
-      HIP_TRY(convert(L.dWacc, vb, nullptr, nullptr, dw_rows(nbands - 1)));
-    }
-    if (L.dh_late) HIP_TRY(convert(L.dHacc, N, L.live, L.idx, grad_hidden));
-    if (need_dh) {
-      const long row_bytes = d * (dh_f32 ? 4 : 2);
-      hipLaunchKernelGGL(zero_rows_kernel, dim3((unsigned)std::min<long>(ceil_div(N * (row_bytes / 16), 256), 4096)),
-                         dim3(256), 0, st, static_cast<char*>(grad_hidden), row_bytes, L.idx, L.live, (int)N);
-      HIP_TRY(hipGetLastError());
-    }
-    return CCE_OK;
-  }
-
-  // d not a multiple of 64: one G buffer; per unit the recompute (register-
-  // staged pipeline), then dH and dW
-  for (long u = 0; u < units; ++u) {
-    const long b = u / R, r = u % R;
+  // launch u: dW and dH of unit u from G[u & 1] and the recompute of unit
+  // u+1 into G[(u+1) & 1]; unit 0's recompute runs alone first.
+  const long dmain = band_dmain(d);
+  {
     GemmShape g1 = {};
     GradParams e1 = {};
     int nb1 = 0;
-    {
-      long v0, vb, vb64, m0, rows;
-      band_cols(b, v0, vb, vb64);
-      block_span(r, m0, rows);
-      grad_shape(H, W, bias, L, L.G[0], m0, rows, d, v0, vb, kSlowBN, false, g1, e1, nb1);
-    }
-    rc = bias ? launch_gemm<kSlowBN, kWarp8, true, true, EpiGradBias, 3>(g1, e1, nb1, st, CCE_KERNEL_BWD_GRAD, false)
-              : launch_gemm<kSlowBN, kWarp8, true, true, EpiGrad, 3>(g1, e1, nb1, st, CCE_KERNEL_BWD_GRAD, false);
+    grad_unit(0, false, kBN, g1, e1, nb1);
+    if (g1.arow || !whole_slabs(d)) {
+      // reading H through the row order, or d no multiple of 64: a band launch
+      // with only this recompute population (the stand-alone GEMM kernel with
+      // the row map spills registers; the band kernel's allocation does not)
+      BandLaunch p0 = {};
+      p0.gr = g1;
+      p0.e_gr = e1;
+      p0.nb_gr = nb1;
+      rc = launch_band(p0, bias != nullptr, st, CCE_KERNEL_BWD_GRAD);
+    } else
+      rc = bias ? launch_gemm<kBN, kWarp8, EpiGradBias>(g1, e1, nb1, st, CCE_KERNEL_BWD_GRAD, false)
+                : launch_gemm<kBN, kWarp8, EpiGrad>(g1, e1, nb1, st, CCE_KERNEL_BWD_GRAD, false);
     if (rc) return rc;
-    GemmShape g2 = {}, g3 = {};
-    AccParams e2 = {}, e3 = {};
     if (need_dh) {
-      if (r == 0) {
-        rc = transpose_band(b);
-        if (rc) return rc;
-      }
-      dh_shape(b, r, L.G[0], 0, d, g2, e2);
-    }
-    if (need_dw) dw_shape(b, r, L.G[0], 0, d, g3, e3);
-    if (need_dh && need_dw)
-      rc = launch_dual_acc(g3, e3, g2, e2, st);
-    else if (need_dh)
-      rc = launch_acc<kFastBN, true, 4>(g2, e2, st, CCE_KERNEL_BWD_DH);
-    else if (need_dw)
-      rc = launch_acc<kSlowBN, false, 5>(g3, e3, st, CCE_KERNEL_BWD_DW);
-    if (rc) return rc;
-    if (need_db) {
-      rc = colsum_unit(b, r, L.G[0]);
+      rc = transpose_band(0);
       if (rc) return rc;
     }
+  }
+  // With 4 or more splits (very few rows) the band launches are short and the
+  // reduction rides in the next launch, so the partials alternate between
+  // two buffers; with 2-3 splits the launches are full and it runs as a
+  // launch of its own after each unit, on the one buffer.
+  const bool fold = L.dhpart && dh_fold(L.dh_ks);
+  auto dh_part = [&](long u) { return L.dhpart + (fold ? (u & 1) : 0) * (long)L.dh_ks * Nb * d; };
+  // the reduction of unit u's K-split dH partials, with its band's
+  // accumulator mode (as dh_shape sets it)
+  auto dh_reduction = [&](long u, int ks) {
+    const long b = u / R;
+    long m0, rows;
+    block_span(u % R, m0, rows);
+    DhReduce r;
+    r.P = dh_part(u);
+    r.stride = Nb * d;
+    r.ks = ks; r.N = (int)rows; r.d = (int)d;
+    r.live = L.live; r.live_base = (int)m0;
+    r.acc = L.dHacc ? L.dHacc + m0 * d : nullptr;
+    r.mode = dh_mode(b);
+    r.out = L.idx ? grad_hidden
+                  : (dh_f32 ? static_cast<void*>(static_cast<float*>(grad_hidden) + m0 * d)
+                            : static_cast<void*>(static_cast<bf16_t*>(grad_hidden) + m0 * d));
+    r.out_f32 = dh_f32;
+    r.rowmap = L.idx ? L.idx + m0 : nullptr;
+    return r;
+  };
+  int prev_ks = 1;
+  for (long u = 0; u < units; ++u) {
+    const long b = u / R, r = u % R;
+    const bf16_t* G = L.G[u & 1];
+    BandLaunch p = {};
+    if (need_dw) {
+      if (dmain > 0) {
+        dw_shape(b, r, G, 0, dmain, p.dw, p.e_dw);
+        p.nb_dw = (int)(ceil_div(p.dw.M, kBM) * ceil_div(dmain, kBN));
+      }
+      if (dmain < d) {
+        dw_shape(b, r, G, dmain, d - dmain, p.dw2, p.e_dw2);
+        p.nb_dw2 = (int)(ceil_div(p.dw2.M, kBM) * ceil_div(d - dmain, kTailBN));
+      }
+    }
+    if (need_dh) {
+      // the next band's W rows, transposed into the other WT buffer by the
+      // band's first launch (band b reads WT[b & 1] in all its launches);
+      // the last band's W^T, when it takes the memory that this band's
+      // W^T occupies (wt_last_in_place), by a launch of its own once this
+      // band is done
+      const bool tr_late = L.wt_last_in_place && b + 2 == nbands;
+      if (r == 0 && b + 1 < nbands && !tr_late) p.nb_tr = transpose_params(b + 1, p.tr);
+      long m0, rows;
+      block_span(r, m0, rows);
+      const int gm = (int)ceil_div(rows, kBM);
+      // K splits of this unit: every split non-empty and a whole number of slabs
+      int ks = 1;
+      if (L.dhpart) {
+        long v0, vb, vb64;
+        band_cols(b, v0, vb, vb64);
+        p.dh_kc = (int)align_up((size_t)ceil_div(vb64, L.dh_ks), 64);
+        ks = (int)ceil_div(vb64, p.dh_kc);
+      }
+      p.dh_split = L.dhpart != nullptr;  // every unit, even one left with a single split
+      p.dh_ks = ks;
+      p.dh_part_stride = Nb * d;
+      float* const part = L.dhpart ? dh_part(u) : nullptr;
+      if (dmain > 0) {
+        dh_shape(b, r, G, 0, dmain, p.dh, p.e_dh);
+        p.nb_dh = gm * (int)ceil_div(dmain, kBN) * ks;
+        p.e_dh_part = p.e_dh;
+        p.e_dh_part.acc32 = part; p.e_dh_part.ldacc = d; p.e_dh_part.mode = 1; p.e_dh_part.rowmap = nullptr;
+      }
+      if (dmain < d) {
+        dh_shape(b, r, G, dmain, d - dmain, p.dh2, p.e_dh2);
+        p.nb_dh2 = gm * (int)ceil_div(d - dmain, kTailBN) * ks;
+        p.e_dh2_part = p.e_dh2;
+        p.e_dh2_part.acc32 = part ? part + dmain : nullptr; p.e_dh2_part.ldacc = d;
+        p.e_dh2_part.mode = 1; p.e_dh2_part.rowmap = nullptr;
+      }
+      // the previous unit's partials (the other buffer) into the accumulator
+      if (fold && u > 0) {
+        p.red = dh_reduction(u - 1, prev_ks);
+        long pm0, prows;
+        block_span((u - 1) % R, pm0, prows);
+        p.nb_red = (int)std::min<long>(ceil_div(prows * (d / 4), kWarp8 * 64 * 4), 1024);
+      }
+      prev_ks = ks;
+    }
+    if (u + 1 < units) grad_unit(u + 1, true, kBN, p.gr, p.e_gr, p.nb_gr);
+    rc = launch_band(p, bias != nullptr, st);
+    if (rc) return rc;
+    if (need_dh && L.dhpart && (!fold || u + 1 == units)) {
+      // this unit's partials (the last band's go to the output: mode 0, 3 or 4)
+      long m0, rows;
+      block_span(r, m0, rows);
+      hipLaunchKernelGGL(dh_reduce_kernel, dim3((unsigned)std::min<long>(ceil_div(rows * (d / 4), 256), 2048)),
+                         dim3(256), 0, st, dh_reduction(u, prev_ks));
+      HIP_TRY(hipGetLastError());
+    }
+    if (need_dh && L.wt_last_in_place && b + 2 == nbands && r == R - 1) {
+      rc = transpose_band(b + 1);
+      if (rc) return rc;
+    }
+    if (need_db) {
+      rc = colsum_unit(b, r, G);
+      if (rc) return rc;
+    }
+  }
+  // outputs whose memory held W^T / H^T during the bands: the last band's
+  // dW from its fp32 accumulator, then dH (the labelled rows) through the
+  // row map; the rows without a label are zeroed last
+  auto convert = [&](const float* src, long rows, const int* live, const int* rowmap, void* out) {
+    DhReduce c = {};
+    c.P = src;
+    c.ks = 1;
+    c.N = (int)rows; c.d = (int)d;
+    c.live = live; c.live_base = 0;
+    c.mode = 0;
+    c.out = out; c.out_f32 = 0;
+    c.rowmap = rowmap;
+    hipLaunchKernelGGL(dh_reduce_kernel, dim3((unsigned)std::min<long>(ceil_div(rows * (d / 4), 256), 2048)),
+                       dim3(256), 0, st, c);
+    return hipGetLastError();
+  };
+  if (L.wt_last_in_place) {
+    long v0, vb, vb64;
+    band_cols(nbands - 1, v0, vb, vb64);
+    HIP_TRY(convert(L.dWacc, vb, nullptr, nullptr, dw_rows(nbands - 1)));
+  }
+  if (L.dh_late) HIP_TRY(convert(L.dHacc, N, L.live, L.idx, grad_hidden));
+  if (need_dh) {
+    const long row_bytes = d * (dh_f32 ? 4 : 2);
+    hipLaunchKernelGGL(zero_rows_kernel, dim3((unsigned)std::min<long>(ceil_div(N * (row_bytes / 16), 256), 4096)),
+                       dim3(256), 0, st, static_cast<char*>(grad_hidden), row_bytes, L.idx, L.live, (int)N);
+    HIP_TRY(hipGetLastError());
   }
   return CCE_OK;
 }

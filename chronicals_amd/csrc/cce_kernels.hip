@@ -134,6 +134,8 @@ struct GemmShape {
   // reads the rest of its row (zero padding or finite values); it never runs
   // past the row's end (ld), so never past B (kmajor_fits).
   int kb = 0;
+  // column origin of an MN-major B: B's row n is column b0 + n of [K][ldb]
+  int b0 = 0;
   // Row map of a K-major A: GEMM row m is row arow[m] of A, which
   // has arows rows in all (arows * lda * 2 bytes below 2^31 - 16).  Null:
   // row m is row m.
@@ -270,16 +272,29 @@ struct ARows {
 };
 
 // MN-major tile: element (m, k) at X[k*ld + m].  The tile k [k0, k0 + 64) x
-// m [m0, m0 + BR) is copied in its natural [k][m] layout (BR * 2 bytes per k
-// row; one wave instruction = 512 / BR rows), with 16-byte chunk c of row k
-// stored at physical chunk c ^ (4*(k & 3)) so the four rows touched by one
-// transposed fragment read land on distinct banks.  Rows k >= K fall outside
-// the descriptor's range and read as zero; columns past a row's end read the
-// next row (the epilogues mask them).
+// m [m0, m0 + BR) goes to LDS in rows of one k.  One wave instruction fills
+// 1 KB = 512 / BR rows, k = 8q + s and its followers in steps of 4 (k mod 4 is
+// the same for all of them when BR = 256; with BR = 128 it takes the four rows
+// k, k + 4, k + 8, k + 12 of a group of 16), and blocks lie kMnBlock elements
+// apart: 64 bytes of padding shift the four rows that one transposed fragment
+// read touches (k mod 4 = 0..3) onto distinct banks, and every fragment's
+// address is one lane address plus a constant.  Rows k >= K fall outside the
+// descriptor's range and read as zero; columns past a row's end read the next
+// row (the epilogues mask them).
+constexpr int kMnBlock = 512 + 32;
+template <int BR>
+__host__ __device__ constexpr int mn_rows() { return 512 / BR; }  // k rows of a block
+// Element offset of k row `k`: groups of 4 * mn_rows k rows are 4 blocks, block k & 3.
+template <int BR>
+__device__ constexpr int mn_row(int k) {
+  constexpr int R = mn_rows<BR>();
+  return ((k / (4 * R)) * 4 + (k & 3)) * kMnBlock + ((k >> 2) % R) * BR;
+}
 template <int BR, int W>
 __device__ inline void dma_mnmajor(const bf16_t* __restrict__ X, long ld, int m0, int k0, int K, bf16_t* S, int w,
                                    int l) {
-  static_assert(BR == 256 || BR == 128, "whole or half rows of the swizzle");
+  static_assert(BR == 256 || BR == 128, "2 or 4 rows in a block");
+  constexpr int R = mn_rows<BR>();
   constexpr int kI = BR / (8 * W);    // wave instructions per wave
   constexpr int kLanes = BR / 8;      // lanes per k row
   const long rows_left = (long)K - k0;
@@ -287,12 +302,11 @@ __device__ inline void dma_mnmajor(const bf16_t* __restrict__ X, long ld, int m0
   const __amdgpu_buffer_rsrc_t rs = make_rsrc(X + (long)k0 * ld + m0, bytes);
 #pragma unroll
   for (int j = 0; j < kI; ++j) {
-    const int blk = w * kI + j;  // 512 / BR k rows
-    const int row = blk * (64 / kLanes) + l / kLanes;
-    const int c = (l % kLanes) ^ (4 * (row & 3));
-    const int voff = (int)(((long)row * ld + c * 8) * 2);
+    const int blk = w * kI + j;
+    const int row = (blk >> 2) * 4 * R + (blk & 3) + 4 * (l / kLanes);
+    const int voff = (int)(((long)row * ld + (l % kLanes) * 8) * 2);
     __builtin_amdgcn_raw_ptr_buffer_load_lds(
-        rs, (__attribute__((address_space(3))) void*)(S + blk * 512), 16, voff, 0, 0, 0);
+        rs, (__attribute__((address_space(3))) void*)(S + blk * kMnBlock), 16, voff, 0, 0, 0);
   }
 }
 
@@ -302,11 +316,9 @@ typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 // ds_read_b64_tr_b16: in each 16-lane group, lane j receives element j&3 of
 // the 8-byte reads addressed by lanes (j>>2) + 4t, t = 0..3.  Lane a of the
 // group addresses row k = kb + (a>>2), columns m = mb + 4*(a&3) .. +3 of the
-// [k][m] tile (BR columns), so lane j receives k = kb..kb+3 of column m = mb + j.
-template <int BR>
-__device__ inline uint2 read_tr4(const bf16_t* S, int k, int m) {
-  const int phys = (((m >> 3) ^ (4 * (k & 3))) << 3) + (m & 7);
-  const s16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(S + k * BR + phys));
+// [k][m] tile, so lane j receives k = kb..kb+3 of column m = mb + j.
+__device__ inline uint2 read_tr4(const bf16_t* S) {
+  const s16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)S);
   return __builtin_bit_cast(uint2, v);
 }
 
@@ -330,13 +342,13 @@ __device__ inline void read_op(const bf16_t* __restrict__ S, int kk, int r0, u32
       f[i] = *reinterpret_cast<const u32x4*>(S + r * 64 + ((c ^ swz(r)) << 3));
     }
   } else {
+    // k = kk*16 + 8*(l >> 5) + (a >> 2) and that + 4, a = l & 15
     const int a = l & 15;
-    const int kb = kk * 16 + 8 * (l >> 5) + (a >> 2);
+    const bf16_t* const base = S + mn_row<BR>(8 * (l >> 5) + (a >> 2)) + r0 + 16 * ((l >> 4) & 1) + 4 * (a & 3);
 #pragma unroll
     for (int i = 0; i < FR; ++i) {
-      const int mb = r0 + i * 32 + 16 * ((l >> 4) & 1) + 4 * (a & 3);
-      const uint2 lo = read_tr4<BR>(S, kb, mb);
-      const uint2 hi = read_tr4<BR>(S, kb + 4, mb);
+      const uint2 lo = read_tr4(base + mn_row<BR>(kk * 16) + i * 32);
+      const uint2 hi = read_tr4(base + mn_row<BR>(kk * 16) + mn_row<BR>(4) + i * 32);
       f[i] = u32x4{lo.x, lo.y, hi.x, hi.y};
     }
   }
@@ -382,7 +394,7 @@ __host__ __device__ inline float split_cost(int gl, int tn, int s, int ncu) {
 template <int BN, int W, bool HB>
 struct EpiLseT {
   typedef LseParams Params;
-  static constexpr bool kMultiTile = true;
+  static constexpr bool kOneTile = false;
   static constexpr bool kDynSplits = true;
   static constexpr int FM = WaveCfg<W>::kFM;
   struct State {
@@ -528,12 +540,13 @@ struct GradParams {
 // row so the 16 lanes of a write phase hit distinct banks), reads it back
 // row-major and stores whole 128-byte row segments, 8 rows per instruction.
 // A wave's LDS operations execute in order, so no barrier is needed.
-template <int BN, int W, bool HB>
+// ONE: a workgroup takes one column tile (splits == tiles_n); otherwise it
+// walks a run of column tiles of one row tile, so the next tile's loads are in
+// flight while this tile's epilogue runs.
+template <int BN, int W, bool HB, bool ONE>
 struct EpiGradT {
   typedef GradParams Params;
-  // Each workgroup walks a run of column tiles of one row tile, so the next
-  // tile's loads are in flight while this tile's epilogue runs.
-  static constexpr bool kMultiTile = true;
+  static constexpr bool kOneTile = ONE;
   static constexpr bool kDynSplits = false;
   static constexpr int FM = WaveCfg<W>::kFM;
   static constexpr int kScratch = W * 2048;  // 32 x 64 bf16 per wave
@@ -668,9 +681,13 @@ struct EpiGradT {
 };
 
 template <int BN, int W>
-using EpiGrad = EpiGradT<BN, W, false>;
+using EpiGrad = EpiGradT<BN, W, false, false>;
 template <int BN, int W>
-using EpiGradBias = EpiGradT<BN, W, true>;
+using EpiGradBias = EpiGradT<BN, W, true, false>;
+template <int BN, int W>
+using EpiGradTile = EpiGradT<BN, W, false, true>;
+template <int BN, int W>
+using EpiGradBiasTile = EpiGradT<BN, W, true, true>;
 
 struct AccParams {
   float* acc32;
@@ -689,7 +706,7 @@ struct AccParams {
 template <int BN, int W>
 struct EpiAcc {
   typedef AccParams Params;
-  static constexpr bool kMultiTile = false;
+  static constexpr bool kOneTile = true;
   static constexpr bool kDynSplits = false;
   static constexpr int FM = WaveCfg<W>::kFM;
   static constexpr int kScratch = 0;
@@ -763,16 +780,18 @@ struct EpiAcc {
 // ---------------------------------------------------------------------------
 // The GEMM kernel: C[M,N] = A[M,K] . B[N,K]^T, 256 x BN x 64 tiles, operands
 // copied straight into NST unpadded LDS stages (described at the loop below).
-// AK: A is K-major, else MN-major and read back transposed; B is K-major.
+// AK, BK: the operand is K-major, else MN-major and read back transposed.
 // AROW: a K-major A is read through g.arow (ARows).  KTAIL: K-major operands
 // whose K is no multiple of 64 (dma_kmajor).
 // ---------------------------------------------------------------------------
-template <int BN>
-constexpr int gemm_lds_elems(int nst = 2) {
-  return nst * (kBM + BN) * kBK;
-}
+// LDS elements of an operand's tile of BR rows, and of NST stages.
+template <bool KM, int BR>
+constexpr int tile_elems() { return KM ? BR * kBK : BR * kBK / 512 * kMnBlock; }
+template <int BN, bool AK, bool BK, int NST = 2>
+constexpr int gemm_lds_elems() { return NST * (tile_elems<AK, kBM>() + tile_elems<BK, BN>()); }
 
-template <int BN, int W, bool AK, template <int, int> class EpiT, int NST = 2, bool AROW = false, bool KTAIL = false>
+template <int BN, int W, bool AK, bool BK, template <int, int> class EpiT, int NST = 2, bool AROW = false,
+          bool KTAIL = false>
 __device__ __forceinline__ void gemm_body(const GemmShape& g_in, const typename EpiT<BN, W>::Params& ep, int bid,
                                           int nb, bf16_t* smem) {
   typedef EpiT<BN, W> Epi;
@@ -793,14 +812,17 @@ __device__ __forceinline__ void gemm_body(const GemmShape& g_in, const typename 
     }
   }
   // epilogue staging area, past the pipeline's LDS stages
-  bf16_t* const scratch = smem + gemm_lds_elems<BN>(NST);
+  bf16_t* const scratch = smem + gemm_lds_elems<BN, AK, BK, NST>();
 
   const int tid = threadIdx.x, l = tid & 63, w = tid >> 6;
   const int wm = w >> 1, wn = w & 1;
 
   int tm, t0, t1, split;
   Epi::assign(g, ep, bid, nb, tm, t0, t1, split);
-  if (t0 >= t1) return;  // uniform for the whole workgroup
+  if constexpr (Epi::kOneTile)
+    t1 = t0 + 1;
+  else if (t0 >= t1)
+    return;  // uniform for the whole workgroup
 
   typename Epi::State st;
   Epi::init(ep, st, g, tm, wm, l);
@@ -818,18 +840,18 @@ __device__ __forceinline__ void gemm_body(const GemmShape& g_in, const typename 
   //   then the DMA of slab s+2 into that stage and the first fragments of
   //   slab s+1 are issued while the MFMAs of k-step 3 (whose fragments are
   //   already in registers) run, so the barrier's read bubble is hidden.
-  constexpr int kSt = (kBM + BN) * kBK;  // elements of a stage
+  constexpr int kStA = tile_elems<AK, kBM>(), kSt = kStA + tile_elems<BK, BN>();  // elements of a stage
   static_assert(NST >= 2 && NST <= 3, "LDS holds two or three stages");
   // DMA wave instructions per wave per slab
   constexpr int kD = (kBM + BN) / (8 * W);
   auto frags = [&](const bf16_t* Sc, int kk, Frags<BN, W>& f) {
     read_op<AK, kBM>(Sc, kk, wm * WaveCfg<W>::kWaveRows, f.a, l);
-    read_op<true, BN>(Sc + kBM * kBK, kk, wn * (BN / 2), f.b, l);
+    read_op<BK, BN>(Sc + kStA, kk, wn * (BN / 2), f.b, l);
   };
   // DMA of the next unissued slab (tile it2, k-slab ik2) into stage S
   int it2 = t0, ik2 = 0;
   // A through a row map: its lane offsets are computed once per workgroup
-  static_assert(AK || !(AROW || KTAIL), "the row map and the K tail are for a K-major A");
+  static_assert((AK && BK) || !(AROW || KTAIL), "the row map and the K tail are for K-major operands");
   static_assert(!(AROW && KTAIL), "a row-mapped A has whole slabs");
   ARows<W> arows;
   if constexpr (AROW) arows.init(g.A, g.lda, a_r0, g.M, g.arow, g.arows, w, l);
@@ -840,7 +862,10 @@ __device__ __forceinline__ void gemm_body(const GemmShape& g_in, const typename 
       dma_kmajor<kBM, W, KTAIL>(g.A, g.lda, a_r0, g.M, ik2 * kBK, g.K, S, w, l);
     else
       dma_mnmajor<kBM, W>(g.A, g.lda, a_r0, ik2 * kBK, g.K, S, w, l);
-    dma_kmajor<BN, W, KTAIL>(g.B, g.ldb, it2 * BN, g.N, g.kb + ik2 * kBK, g.K, S + kBM * kBK, w, l);
+    if constexpr (BK)
+      dma_kmajor<BN, W, KTAIL>(g.B, g.ldb, it2 * BN, g.N, g.kb + ik2 * kBK, g.K, S + kStA, w, l);
+    else
+      dma_mnmajor<BN, W>(g.B, g.ldb, g.b0 + it2 * BN, ik2 * kBK, g.K, S + kStA, w, l);
     if (++ik2 == KT) {
       ik2 = 0;
       ++it2;
@@ -870,7 +895,7 @@ __device__ __forceinline__ void gemm_body(const GemmShape& g_in, const typename 
   // each k-step: the next k-step's fragment reads are issued first, then
   // the MFMAs they hide behind
   auto order = [&]() {
-    constexpr int kReads = (AK ? 1 : 2) * WaveCfg<W>::kFM + BN / 64;
+    constexpr int kReads = (AK ? 1 : 2) * WaveCfg<W>::kFM + (BK ? 1 : 2) * (BN / 64);
     __builtin_amdgcn_sched_group_barrier(0x100, kReads, 0);
     __builtin_amdgcn_sched_group_barrier(0x008, WaveCfg<W>::kFM * (BN / 64), 0);
   };
@@ -924,10 +949,11 @@ __device__ __forceinline__ void gemm_body(const GemmShape& g_in, const typename 
   Epi::finish(ep, st, g, tm, split, smem, wm, wn, l);
 }
 
-template <int BN, int W, bool AK, template <int, int> class EpiT, int NST = 2, bool AROW = false, bool KTAIL = false>
+template <int BN, int W, bool AK, bool BK, template <int, int> class EpiT, int NST = 2, bool AROW = false,
+          bool KTAIL = false>
 __global__ __launch_bounds__(W * 64) void gemm_kernel(GemmShape g, typename EpiT<BN, W>::Params ep) {
-  __shared__ __attribute__((aligned(16))) bf16_t smem[gemm_lds_elems<BN>(NST) + EpiT<BN, W>::kScratch];
-  gemm_body<BN, W, AK, EpiT, NST, AROW, KTAIL>(g, ep, blockIdx.x, gridDim.x, smem);
+  __shared__ __attribute__((aligned(16))) bf16_t smem[gemm_lds_elems<BN, AK, BK, NST>() + EpiT<BN, W>::kScratch];
+  gemm_body<BN, W, AK, BK, EpiT, NST, AROW, KTAIL>(g, ep, blockIdx.x, gridDim.x, smem);
 }
 
 // One launch per vocabulary band b of the backward: the
@@ -939,10 +965,10 @@ __global__ __launch_bounds__(W * 64) void gemm_kernel(GemmShape g, typename EpiT
 // then the short recompute tiles, which fill the CUs the long tiles leave
 // idle at the end of the band.  The 128-wide tail tiles fit three LDS stages
 // (two slabs in flight) in the space the 256-wide tiles use for two.
-// The transpose of the next band's W rows (dH's B operand) rides along as the
-// last, shortest population: one 64 x 64 tile per workgroup.  With dH split
-// over K on very few rows, the previous band's partials are reduced by a
-// population placed just before the transposes.
+// dH reads W's rows as they are (an MN-major B): against a transposed copy of
+// each band's rows the band launch takes the same time at d = 896 and 1.4% less
+// at d = 4096 (8192 rows), and the copies and their memory are gone.  With dH split over K on very
+// few rows, the previous band's partials are reduced by the last population.
 
 // dH of one band split over the band's K (few row tiles): the ks fp32
 // partials P[k] = P + k * stride ([rows][d], GEMM row order) of each live row
@@ -990,16 +1016,6 @@ __device__ inline void dh_reduce_body(const DhReduce& r, long first, long step) 
   }
 }
 
-struct TransposeParams {
-  const bf16_t* in;
-  long ldi;
-  int R, C;
-  bf16_t* out;
-  long ldo;
-  int Rpad;
-  int tiles_r;  // 64-row tiles of in
-};
-
 struct BandLaunch {
   GemmShape dw;
   AccParams e_dw;
@@ -1011,8 +1027,7 @@ struct BandLaunch {
   AccParams e_dh2;
   GemmShape gr;
   GradParams e_gr;
-  TransposeParams tr;
-  int nb_dw, nb_dw2, nb_dh, nb_dh2, nb_gr, nb_tr;
+  int nb_dw, nb_dw2, nb_dh, nb_dh2, nb_gr;
   // dH split over the band's K (few row tiles): with dh_split each dH tile
   // has dh_ks workgroups (possibly one, for a narrow band); split k covers K
   // columns [k*dh_kc, (k+1)*dh_kc) and writes its fp32 partial with
@@ -1035,30 +1050,28 @@ __device__ inline void dh_split_body(const GemmShape& g0, const AccParams& e0, i
   GemmShape g = g0;
   AccParams e = e0;
   g.A += k0;
-  g.B += k0;
+  g.B += k0 * g.ldb;
   g.K = min(kc, g0.K - k0);
   e.acc32 += k * stride;
-  gemm_body<BN, kWarp8, true, EpiAcc, NST>(g, e, b / ks, nb / ks, smem);
+  gemm_body<BN, kWarp8, true, false, EpiAcc, NST>(g, e, b / ks, nb / ks, smem);
 }
-
-template <int NT>
-__device__ inline void transpose_tile(const bf16_t* __restrict__ in, long ldi, int R, int C, bf16_t* __restrict__ out,
-                                      long ldo, int Rpad, int r0, int c0, bf16_t (*t)[66], int tid,
-                                      const int* __restrict__ rmap);
 
 // HB: with a bias.  AROW: the recompute reads H's rows through the row order.
 // KTAIL: d is no multiple of 64 (the recompute's K).
 template <bool HB, bool AROW, bool KTAIL>
 __global__ __launch_bounds__(kWarp8 * 64) void band_kernel(BandLaunch p) {
-  __shared__ __attribute__((aligned(16))) bf16_t smem[gemm_lds_elems<kBN>() + EpiGrad<kBN, kWarp8>::kScratch];
+  __shared__ __attribute__((aligned(16))) bf16_t smem[gemm_lds_elems<kBN, true, true>() + EpiGrad<kBN, kWarp8>::kScratch];
+  static_assert(sizeof(smem) >= 2 * gemm_lds_elems<kBN, false, true>() && sizeof(smem) >= 2 * gemm_lds_elems<kBN, true, false>() &&
+                sizeof(smem) >= 2 * gemm_lds_elems<kTailBN, false, true, 3>() &&
+                sizeof(smem) >= 2 * gemm_lds_elems<kTailBN, true, false, 3>(), "every population's stages fit");
   int b = blockIdx.x;
   if (b < p.nb_dw) {
-    gemm_body<kBN, kWarp8, false, EpiAcc>(p.dw, p.e_dw, b, p.nb_dw, smem);
+    gemm_body<kBN, kWarp8, false, true, EpiAcc>(p.dw, p.e_dw, b, p.nb_dw, smem);
     return;
   }
   b -= p.nb_dw;
   if (b < p.nb_dw2) {
-    gemm_body<kTailBN, kWarp8, false, EpiAcc, 3>(p.dw2, p.e_dw2, b, p.nb_dw2, smem);
+    gemm_body<kTailBN, kWarp8, false, true, EpiAcc, 3>(p.dw2, p.e_dw2, b, p.nb_dw2, smem);
     return;
   }
   b -= p.nb_dw2;
@@ -1066,7 +1079,7 @@ __global__ __launch_bounds__(kWarp8 * 64) void band_kernel(BandLaunch p) {
     if (p.dh_split)
       dh_split_body<kBN, 2>(p.dh, p.e_dh_part, p.dh_ks, p.dh_kc, p.dh_part_stride, b, p.nb_dh, smem);
     else
-      gemm_body<kBN, kWarp8, true, EpiAcc>(p.dh, p.e_dh, b, p.nb_dh, smem);
+      gemm_body<kBN, kWarp8, true, false, EpiAcc>(p.dh, p.e_dh, b, p.nb_dh, smem);
     return;
   }
   b -= p.nb_dh;
@@ -1074,25 +1087,19 @@ __global__ __launch_bounds__(kWarp8 * 64) void band_kernel(BandLaunch p) {
     if (p.dh_split)
       dh_split_body<kTailBN, 3>(p.dh2, p.e_dh2_part, p.dh_ks, p.dh_kc, p.dh_part_stride, b, p.nb_dh2, smem);
     else
-      gemm_body<kTailBN, kWarp8, true, EpiAcc, 3>(p.dh2, p.e_dh2, b, p.nb_dh2, smem);
+      gemm_body<kTailBN, kWarp8, true, false, EpiAcc, 3>(p.dh2, p.e_dh2, b, p.nb_dh2, smem);
     return;
   }
   b -= p.nb_dh2;
   if (b < p.nb_gr) {
     if constexpr (HB)
-      gemm_body<kBN, kWarp8, true, EpiGradBias, 2, AROW, KTAIL>(p.gr, p.e_gr, b, p.nb_gr, smem);
+      gemm_body<kBN, kWarp8, true, true, EpiGradBiasTile, 2, AROW, KTAIL>(p.gr, p.e_gr, b, p.nb_gr, smem);
     else
-      gemm_body<kBN, kWarp8, true, EpiGrad, 2, AROW, KTAIL>(p.gr, p.e_gr, b, p.nb_gr, smem);
+      gemm_body<kBN, kWarp8, true, true, EpiGradTile, 2, AROW, KTAIL>(p.gr, p.e_gr, b, p.nb_gr, smem);
     return;
   }
   b -= p.nb_gr;
-  if (b < p.nb_red) {
-    dh_reduce_body(p.red, b * (long)(kWarp8 * 64) + threadIdx.x, (long)p.nb_red * (kWarp8 * 64));
-    return;
-  }
-  b -= p.nb_red;
-  transpose_tile<kWarp8 * 64>(p.tr.in, p.tr.ldi, p.tr.R, p.tr.C, p.tr.out, p.tr.ldo, p.tr.Rpad, (b % p.tr.tiles_r) * 64,
-                              (b / p.tr.tiles_r) * 64, reinterpret_cast<bf16_t(*)[66]>(smem), threadIdx.x, nullptr);
+  dh_reduce_body(p.red, b * (long)(kWarp8 * 64) + threadIdx.x, (long)p.nb_red * (kWarp8 * 64));
 }
 
 // ---------------------------------------------------------------------------
@@ -1757,16 +1764,16 @@ __global__ __launch_bounds__(256) void bwd_prep_kernel(const float* __restrict__
   }
 }
 
-// out[c][r] = in[r][c] for r < R (zero for R <= r < Rpad), c < C, over the
-// 64 x 64 tile at (r0, c0), by NT threads staging through t.  With a row map,
-// row r of the input is row rmap[r] of in.
-template <int NT>
-__device__ inline void transpose_tile(const bf16_t* __restrict__ in, long ldi, int R, int C, bf16_t* __restrict__ out,
-                                      long ldo, int Rpad, int r0, int c0, bf16_t (*t)[66], int tid,
-                                      const int* __restrict__ rmap) {
+// out[c][r] = in[r][c] for r < R (zero for R <= r < Rpad), c < C, one 64 x 64
+// tile per workgroup.  With a row map, row r of the input is row rmap[r] of in.
+__global__ __launch_bounds__(256) void transpose_kernel(const bf16_t* __restrict__ in, long ldi, int R, int C,
+                                                        bf16_t* __restrict__ out, long ldo, int Rpad,
+                                                        const int* __restrict__ rmap) {
+  __shared__ bf16_t t[64][66];
+  const int tid = threadIdx.x, r0 = blockIdx.x * 64, c0 = blockIdx.y * 64;
 #pragma unroll
-  for (int it = 0; it < 512 / NT; ++it) {
-    const int q = tid + it * NT;         // 512 chunks of 8 elements
+  for (int it = 0; it < 2; ++it) {
+    const int q = tid + it * 256;        // 512 chunks of 8 elements
     const int rr = q >> 3, cc = (q & 7) * 8;
     u32x4 v = u32x4{0u, 0u, 0u, 0u};
     if (r0 + rr < R && c0 + cc < C) {
@@ -1781,8 +1788,8 @@ __device__ inline void transpose_tile(const bf16_t* __restrict__ in, long ldi, i
   }
   __syncthreads();
 #pragma unroll
-  for (int it = 0; it < 512 / NT; ++it) {
-    const int q = tid + it * NT;
+  for (int it = 0; it < 2; ++it) {
+    const int q = tid + it * 256;
     const int cc = q >> 3, rr = (q & 7) * 8;
     if (c0 + cc < C && r0 + rr < Rpad) {
       u32x4 v;
@@ -1791,13 +1798,6 @@ __device__ inline void transpose_tile(const bf16_t* __restrict__ in, long ldi, i
       *reinterpret_cast<u32x4*>(out + (long)(c0 + cc) * ldo + r0 + rr) = v;
     }
   }
-}
-
-__global__ __launch_bounds__(256) void transpose_kernel(const bf16_t* __restrict__ in, long ldi, int R, int C,
-                                                        bf16_t* __restrict__ out, long ldo, int Rpad,
-                                                        const int* __restrict__ rmap) {
-  __shared__ bf16_t t[64][66];
-  transpose_tile<256>(in, ldi, R, C, out, ldo, Rpad, blockIdx.x * 64, blockIdx.y * 64, t, threadIdx.x, rmap);
 }
 
 // dB[c] = sum_m G[m][c] for c < C (fixed order: deterministic).  Block = 64
@@ -1962,13 +1962,18 @@ constexpr long kBandCap = 8192;
 long band_width(long V, long chunk, long N, long d) {
   long vb = chunk <= 0 ? kBandCap : std::min(chunk, kBandCap);
   vb = align_up((size_t)vb, 256);
-  // with few rows a band launch is short and its fixed costs dominate: up to
-  // 4x wider bands, while the band buffers (G: rows x band, W^T: d x band)
-  // stay within what 4096 rows take at that band.  Below 1024 rows W^T and
-  // the dH partials would outgrow the logits themselves, for no measured gain.
+  // with few rows a band launch is short and its fixed costs dominate: the
+  // bands widen to what 3072 rows' band gradient (rows x band) takes at the
+  // unwidened band (which leaves room for the K-split dH's partials within
+  // what 4096 rows take), in equal parts of the vocabulary.  Forward and
+  // backward, against bands that widen from 1024 rows on with W transposed for
+  // each: N 64, d 896, V 32000 305 -> 222 us; N 256, d 768, V 50257 fp32
+  // 463 -> 252 us; N 2048, d 896, V 151936 2492 -> 2446 us.
   const long rows = (long)align_up((size_t)(N > 0 ? N : 1), 256);
-  const long f = rows < 1024 ? 1 : std::min<long>(4, std::max<long>(1, (4096 + d) / (rows + d)));
-  vb = std::min<long>(vb * f, kMaxBand);
+  if (rows < 3072) {
+    vb = std::min<long>(vb * 3072 / rows, kMaxBand);
+    vb = (long)align_up((size_t)ceil_div(V, ceil_div(V, vb)), 256);
+  }
   const long vmax = (long)align_up((size_t)V, 256);
   if (vb > vmax) vb = vmax;
   if (vb < 256) vb = 256;
@@ -2046,12 +2051,15 @@ int wsum_splits(long d, long V) {
 
 // The forward compacts its rows when only the labelled rows' lse is wanted
 // and the direct-to-LDS GEMM runs (d a multiple of 64).
-bool fwd_compacts(long d, int lse_rows) { return lse_rows == CCE_LSE_LABELLED_ROWS && whole_slabs(d); }
+// More than one row tile: otherwise there is none to skip.
+bool fwd_compacts(long N, long d, int lse_rows) {
+  return lse_rows == CCE_LSE_LABELLED_ROWS && whole_slabs(d) && N > kBM;
+}
 
 FwdLayout fwd_layout(void* ws, long N, long d, long V, int reduction, int lse_rows, bool prefer_in_place = false) {
   Carver c(ws);
   FwdLayout L;
-  const bool compact = fwd_compacts(d, lse_rows) && N > 0;
+  const bool compact = fwd_compacts(N, d, lse_rows);
   const long nb = ceil_div(N, 4);
   // [S][N rounded up to 256] partials, or for a compacted forward one slot of
   // 256 rows per launched workgroup
@@ -2078,22 +2086,14 @@ struct BwdLayout {
   float4* rowp;
   int* rowlab;
   bf16_t* G[2];   // band gradient of a block; the second only when units alternate
-  bf16_t* WT[2];  // W band transposes; the second only when bands alternate
   bf16_t* HT;
-  // Caller output memory that is not yet written doubles as scratch (bf16 dH
-  // and dW wanted, several bands):
-  //  - ht_out: H^T ([d][N], N a multiple of 64) lives in grad_hidden, which
-  //    the bands leave unwritten: the last band adds into the fp32 dH
-  //    accumulator, and dH goes to grad_hidden after the last band launch;
-  //  - wt_out: W^T of band b lives in the rows of band b + 1 of grad_weight,
-  //    which dW writes only in band b + 1.  The last band's W^T takes WT[0],
-  //    or, when dW accumulates over row blocks in dWacc (wt_last_in_place),
-  //    the last band's own rows of grad_weight, whose dW is then written
-  //    after the last band launch;
-  //  - wt_dh (no dW wanted, N >= 2 * Vb): both W^T buffers live in
-  //    grad_hidden.
-  // dh_late = ht_out || wt_dh: dH is written after the last band launch.
-  bool ht_out, wt_out, wt_last_in_place, wt_dh, dh_late;
+  // grad_hidden, which nothing writes before the last band launch of a bf16
+  // dH over several bands, doubles as scratch until then:
+  //  - ht_out (dW wanted, N a multiple of 64): it holds H^T ([d][N]);
+  //  - hc_out (no dW wanted): it holds H in row order, where that is copied.
+  // Then the last band adds into the fp32 dH accumulator like the others, and
+  // dH goes to grad_hidden after the last band launch (dh_late).
+  bool ht_out, hc_out, dh_late;
   float* dHacc;   // dH over the bands (bf16 dH with several bands; fp32 dH accumulates in place)
   float* dWacc;   // dW of a band over the row blocks (bf16 dW with several blocks)
   // row compaction: row order, live row count, and H in
@@ -2151,22 +2151,20 @@ BwdLayout bwd_layout(void* ws, long N, long d, long V, long Vb, bool need_dh, bo
   const long N64 = ht_cols(N);
   L.rowp = c.take<float4>((size_t)N);
   L.rowlab = c.take<int>((size_t)N);
-  L.ht_out = need_dh && need_dw && !dh_f32 && nbands > 1 && N % 64 == 0;
-  L.wt_out = need_dh && need_dw && nbands > 1;
-  L.wt_last_in_place = L.wt_out && L.nblocks > 1 && !dw_f32;
-  L.wt_dh = need_dh && !need_dw && !dh_f32 && nbands > 1 && N >= 2 * Vb;
-  L.dh_late = L.ht_out || L.wt_dh;
+  const bool copied = N > kBM && !rows_in_place(N, d);  // H in row order is a copy
+  const bool late = need_dh && !dh_f32 && nbands > 1;
+  L.ht_out = late && need_dw && N % 64 == 0;
+  L.hc_out = late && !need_dw && copied;
+  L.dh_late = L.ht_out || L.hc_out;
   L.G[0] = c.take<bf16_t>((size_t)L.Nb * Vb);
-  L.G[1] = (units > 1) ? c.take<bf16_t>((size_t)L.Nb * Vb) : L.G[0];
-  L.WT[0] = need_dh && !L.wt_last_in_place && !L.wt_dh ? c.take<bf16_t>((size_t)d * Vb) : nullptr;
-  L.WT[1] = (need_dh && nbands > 1 && !L.wt_out && !L.wt_dh) ? c.take<bf16_t>((size_t)d * Vb)
-                                                                          : L.WT[0];
+  L.G[1] = units > 1 ? c.take<bf16_t>((size_t)L.Nb * Vb) : L.G[0];
   L.HT = need_dw && !L.ht_out ? c.take<bf16_t>((size_t)d * N64) : nullptr;
   L.dHacc = (need_dh && nbands > 1 && !dh_f32) ? c.take<float>((size_t)N * d) : nullptr;
   L.dWacc = (need_dw && L.nblocks > 1 && !dw_f32) ? c.take<float>((size_t)Vb * d) : nullptr;
-  L.idx = c.take<int>((size_t)N);
-  L.live = c.take<int>(1);
-  L.Hc = !rows_in_place(N, d) ? c.take<bf16_t>((size_t)N * d) : nullptr;
+  // one row tile has no row tiles to skip: no row order
+  L.idx = N > kBM ? c.take<int>((size_t)N) : nullptr;
+  L.live = N > kBM ? c.take<int>(1) : nullptr;
+  L.Hc = copied && !L.hc_out ? c.take<bf16_t>((size_t)N * d) : nullptr;
   L.dh_ks = need_dh ? dh_splits(L.Nb, d, Vb) : 1;
   // a second partial buffer only when the reduction rides in the next
   // launch (dh_fold); otherwise each unit's reduction runs before the next
@@ -2188,10 +2186,12 @@ bool misaligned(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) !
 bool kmajor_fits(long ld, long kb, long K, bool ktail = false) {
   return K <= 0 || kb + (ktail ? K : (long)align_up((size_t)K, kBK)) <= ld;
 }
-int check_kmajor(const GemmShape& g, bool a_kmajor, bool ktail = false) {
-  if ((a_kmajor && !kmajor_fits(g.lda, 0, g.K, ktail)) || !kmajor_fits(g.ldb, g.kb, g.K, ktail))
-    return fail(CCE_ERR_INVALID_ARG, "internal: a K-major operand row (lda %ld, ldb %ld) is shorter than the "
-                "slabs of K = %d at k offset %d", g.lda, g.ldb, g.K, g.kb);
+int check_operands(const GemmShape& g, bool a_kmajor, bool b_kmajor, bool ktail = false) {
+  // an MN-major B's tiles start inside its rows
+  const bool b_ok = b_kmajor ? kmajor_fits(g.ldb, g.kb, g.K, ktail) : (long)g.b0 + g.N <= g.ldb;
+  if ((a_kmajor && !kmajor_fits(g.lda, 0, g.K, ktail)) || !b_ok)
+    return fail(CCE_ERR_INVALID_ARG, "internal: an operand row (lda %ld, ldb %ld) is shorter than the tiles of "
+                "N = %d, K = %d at offsets %d, %d", g.lda, g.ldb, g.N, g.K, g.b0, g.kb);
   return CCE_OK;
 }
 
@@ -2256,11 +2256,11 @@ template <int BN, int W, template <int, int> class EpiT, bool AROW = false, bool
 int launch_gemm(const GemmShape& g, const typename EpiT<BN, W>::Params& ep, int nblocks, hipStream_t st,
                 int kind, bool credited) {
   if (nblocks <= 0) return CCE_OK;
-  const int rc = check_kmajor(g, true, KTAIL);
+  const int rc = check_operands(g, true, true, KTAIL);
   if (rc) return rc;
   hipEvent_t e0 = nullptr, e1 = nullptr;
   const bool timed = timing_begin(st, &e0, &e1);
-  hipLaunchKernelGGL((gemm_kernel<BN, W, true, EpiT, 2, AROW, KTAIL>), dim3(nblocks), dim3(W * 64), 0, st, g, ep);
+  hipLaunchKernelGGL((gemm_kernel<BN, W, true, true, EpiT, 2, AROW, KTAIL>), dim3(nblocks), dim3(W * 64), 0, st, g, ep);
   HIP_TRY(hipGetLastError());
   if (timed) {
     const double f = gemm_flops(g.M, g.N, g.K);
@@ -2310,15 +2310,15 @@ void grad_shape(const bf16_t* H, const bf16_t* W, const float* bias, const BwdLa
 }
 
 int launch_band(const BandLaunch& p, bool has_bias, hipStream_t st, int kind = CCE_KERNEL_BWD_BAND) {
-  const int nb = p.nb_dw + p.nb_dw2 + p.nb_dh + p.nb_dh2 + p.nb_gr + p.nb_red + p.nb_tr;
+  const int nb = p.nb_dw + p.nb_dw2 + p.nb_dh + p.nb_dh2 + p.nb_gr + p.nb_red;
   if (nb <= 0) return CCE_OK;
   int rc = CCE_OK;
-  if (p.nb_dw) rc = check_kmajor(p.dw, false);
-  if (!rc && p.nb_dw2) rc = check_kmajor(p.dw2, false);
-  if (!rc && p.nb_dh) rc = check_kmajor(p.dh, true);
-  if (!rc && p.nb_dh2) rc = check_kmajor(p.dh2, true);
+  if (p.nb_dw) rc = check_operands(p.dw, false, true);
+  if (!rc && p.nb_dw2) rc = check_operands(p.dw2, false, true);
+  if (!rc && p.nb_dh) rc = check_operands(p.dh, true, false);
+  if (!rc && p.nb_dh2) rc = check_operands(p.dh2, true, false);
   const bool ktail = !whole_slabs(p.gr.K);
-  if (!rc && p.nb_gr) rc = check_kmajor(p.gr, true, ktail);
+  if (!rc && p.nb_gr) rc = check_operands(p.gr, true, true, ktail);
   if (rc) return rc;
   hipEvent_t t0 = nullptr, t1 = nullptr;
   const bool timed = timing_begin(st, &t0, &t1);
@@ -2642,10 +2642,7 @@ int cce_backward(const float* grad_out, const void* hidden, const void* weight, 
   if (!need_dh && !need_dw && !need_db) return CCE_OK;
   BwdLayout L = bwd_layout(workspace, N, d, V, Vb, need_dh, need_dw, dh_f32, dw_f32);
   if (L.ht_out) L.HT = static_cast<bf16_t*>(grad_hidden);
-  if (L.wt_dh) {
-    L.WT[0] = static_cast<bf16_t*>(grad_hidden);
-    L.WT[1] = L.WT[0] + d * Vb;
-  }
+  if (L.hc_out) L.Hc = static_cast<bf16_t*>(grad_hidden);
   const long NT = ht_cols(N);  // row length of H^T
   const bf16_t* H = static_cast<const bf16_t*>(hidden);
   const bf16_t* W = static_cast<const bf16_t*>(weight);
@@ -2686,10 +2683,9 @@ int cce_backward(const float* grad_out, const void* hidden, const void* weight, 
   // which has no next unit's recompute to fill the CUs its long dW tiles
   // leave idle, gets a full band.
   const long head = V - (nbands - 1) * Vb;
-  auto band_cols = [&](long b, long& v0, long& vb, long& vb64) {
+  auto band_cols = [&](long b, long& v0, long& vb) {
     v0 = b == 0 ? 0 : head + (b - 1) * Vb;
     vb = b == 0 ? head : Vb;
-    vb64 = (long)align_up((size_t)vb, 64);
   };
   auto block_span = [&](long r, long& m0, long& rows) {
     m0 = r * Nb;
@@ -2697,38 +2693,26 @@ int cce_backward(const float* grad_out, const void* hidden, const void* weight, 
   };
   // dH accumulates over the bands: the first band stores, middle bands add,
   // the last writes the output (fp32 dH: the output is the accumulator; with
-  // grad_hidden holding H^T or W^T the last band adds too, and dH is written
+  // grad_hidden holding scratch the last band adds too, and dH is written
   // afterwards)
   auto dh_mode = [&](long b) {
     if (nbands == 1) return 0;
     if (dh_f32) return b == 0 ? 0 : 4;
     return b == 0 ? 1 : (b == nbands - 1 && !L.dh_late ? 3 : 2);
   };
-  // dW of a band accumulates over the row blocks in the same way (the last
-  // band's W^T in its own rows of grad_weight: written afterwards)
-  auto dw_mode = [&](long b, long r) {
+  // dW of a band accumulates over the row blocks in the same way
+  auto dw_mode = [&](long r) {
     if (R == 1) return 0;
     if (dw_f32) return r == 0 ? 0 : 4;
-    return r == 0 ? 1 : (r == R - 1 && !(L.wt_last_in_place && b == nbands - 1) ? 3 : 2);
+    return r == 0 ? 1 : (r == R - 1 ? 3 : 2);
   };
-  // rows [v0, v0 + vb) of grad_weight, as bf16 elements
-  auto dw_rows = [&](long b) {
-    const long v0 = b == 0 ? 0 : head + (b - 1) * Vb;
-    return reinterpret_cast<bf16_t*>(static_cast<char*>(grad_weight) + v0 * d * (dw_f32 ? 4 : 2));
-  };
-  // where W^T of band b lives ([d][Vb], see BwdLayout::wt_out)
-  auto wt_of = [&](long b) -> bf16_t* {
-    if (!L.wt_out) return L.WT[b & 1];
-    if (b + 1 < nbands) return dw_rows(b + 1);
-    return L.wt_last_in_place ? dw_rows(b) : L.WT[0];
-  };
-  // dH of unit (b, r): G[rows][vb64] . WT[d][vb64]^T over hidden columns [c0, c0 + nc)
+  // dH of unit (b, r): G[rows][vb] . W[v0 .. v0 + vb) over hidden columns [c0, c0 + nc)
   auto dh_shape = [&](long b, long r, const bf16_t* G, long c0, long nc, GemmShape& g, AccParams& e) {
-    long v0, vb, vb64, m0, rows;
-    band_cols(b, v0, vb, vb64);
+    long v0, vb, m0, rows;
+    band_cols(b, v0, vb);
     block_span(r, m0, rows);
-    g.A = G; g.lda = Vb; g.B = wt_of(b) + c0 * Vb; g.ldb = Vb;
-    g.M = (int)rows; g.N = (int)nc; g.K = (int)vb64;
+    g.A = G; g.lda = Vb; g.B = W + v0 * d; g.ldb = d; g.b0 = (int)c0;
+    g.M = (int)rows; g.N = (int)nc; g.K = (int)vb;
     g.live = L.live; g.dyn = L.live ? kDynM : kDynNone; g.live_base = (int)m0;
     e.rowmap = L.idx ? L.idx + m0 : nullptr;
     e.acc32 = L.dHacc ? L.dHacc + m0 * d + c0 : nullptr; e.ldacc = d;
@@ -2744,8 +2728,8 @@ int cce_backward(const float* grad_out, const void* hidden, const void* weight, 
   // dW of unit (b, r): rows [v0, v0 + vb), hidden columns [c0, c0 + nc) of
   // grad_weight = G^T . H over the block's rows
   auto dw_shape = [&](long b, long r, const bf16_t* G, long c0, long nc, GemmShape& g, AccParams& e) {
-    long v0, vb, vb64, m0, rows;
-    band_cols(b, v0, vb, vb64);
+    long v0, vb, m0, rows;
+    band_cols(b, v0, vb);
     block_span(r, m0, rows);
     g.A = G; g.lda = Vb;  // MN-major: element (v, n) at G[n*Vb + v]
     g.B = L.HT + c0 * NT; g.ldb = NT; g.kb = (int)m0;  // H^T columns [m0, m0 + rows)
@@ -2758,30 +2742,12 @@ int cce_backward(const float* grad_out, const void* hidden, const void* weight, 
                    : static_cast<void*>(static_cast<bf16_t*>(grad_weight) + o);
     e.ldo = d;
     e.out_f32 = dw_f32;
-    e.mode = dw_mode(b, r);
-  };
-  // WT[b & 1][j][c] = W[v0 + c][j], zero for vb <= c < vb64: as its own
-  // launch, or as the transpose population of an earlier launch
-  auto transpose_params = [&](long b, TransposeParams& t) -> int {
-    long v0, vb, vb64;
-    band_cols(b, v0, vb, vb64);
-    t.in = W + v0 * d; t.ldi = d; t.R = (int)vb; t.C = (int)d;
-    t.out = wt_of(b); t.ldo = Vb; t.Rpad = (int)vb64;
-    t.tiles_r = (int)ceil_div(vb64, 64);
-    return t.tiles_r * (int)ceil_div(d, 64);
-  };
-  auto transpose_band = [&](long b) -> int {
-    TransposeParams t;
-    const int tiles = transpose_params(b, t);
-    hipLaunchKernelGGL(transpose_kernel, dim3((unsigned)t.tiles_r, (unsigned)(tiles / t.tiles_r)), dim3(256), 0, st,
-                       t.in, t.ldi, t.R, t.C, t.out, t.ldo, t.Rpad, nullptr);
-    HIP_TRY(hipGetLastError());
-    return CCE_OK;
+    e.mode = dw_mode(r);
   };
   // dB[v0 .. v0 + vb) = sum over the block's rows of G, added over the blocks
   auto colsum_unit = [&](long b, long r, const bf16_t* G) -> int {
-    long v0, vb, vb64, m0, rows;
-    band_cols(b, v0, vb, vb64);
+    long v0, vb, m0, rows;
+    band_cols(b, v0, vb);
     block_span(r, m0, rows);
     hipLaunchKernelGGL(colsum_kernel, dim3((unsigned)ceil_div(vb, 64)), dim3(256), 0, st, G, (long)Vb, (int)rows,
                        (int)vb, L.live, (int)m0, r > 0 ? 1 : 0, grad_bias + v0);
@@ -2789,8 +2755,8 @@ int cce_backward(const float* grad_out, const void* hidden, const void* weight, 
     return CCE_OK;
   };
   auto grad_unit = [&](long u, bool in_band, int bn, GemmShape& g, GradParams& e, int& nb) {
-    long v0, vb, vb64, m0, rows;
-    band_cols(u / R, v0, vb, vb64);
+    long v0, vb, m0, rows;
+    band_cols(u / R, v0, vb);
     block_span(u % R, m0, rows);
     grad_shape(H, W, bias, L, L.G[u & 1], m0, rows, d, v0, vb, bn, in_band, g, e, nb);
   };
@@ -2802,11 +2768,12 @@ int cce_backward(const float* grad_out, const void* hidden, const void* weight, 
     GemmShape g1 = {};
     GradParams e1 = {};
     int nb1 = 0;
-    grad_unit(0, false, kBN, g1, e1, nb1);
-    if (g1.arow || !whole_slabs(d)) {
+    const bool in_band = (L.idx && !L.Hc) || !whole_slabs(d);
+    grad_unit(0, in_band, kBN, g1, e1, nb1);
+    if (in_band) {
       // reading H through the row order, or d no multiple of 64: a band launch
-      // with only this recompute population (the stand-alone GEMM kernel with
-      // the row map spills registers; the band kernel's allocation does not)
+      // with only this recompute population (the stand-alone GEMM kernel's
+      // column runs with the row map spill registers)
       BandLaunch p0 = {};
       p0.gr = g1;
       p0.e_gr = e1;
@@ -2816,10 +2783,6 @@ int cce_backward(const float* grad_out, const void* hidden, const void* weight, 
       rc = bias ? launch_gemm<kBN, kWarp8, EpiGradBias>(g1, e1, nb1, st, CCE_KERNEL_BWD_GRAD, false)
                 : launch_gemm<kBN, kWarp8, EpiGrad>(g1, e1, nb1, st, CCE_KERNEL_BWD_GRAD, false);
     if (rc) return rc;
-    if (need_dh) {
-      rc = transpose_band(0);
-      if (rc) return rc;
-    }
   }
   // With 4 or more splits (very few rows) the band launches are short and the
   // reduction rides in the next launch, so the partials alternate between
@@ -2863,23 +2826,16 @@ int cce_backward(const float* grad_out, const void* hidden, const void* weight, 
       }
     }
     if (need_dh) {
-      // the next band's W rows, transposed into the other WT buffer by the
-      // band's first launch (band b reads WT[b & 1] in all its launches);
-      // the last band's W^T, when it takes the memory that this band's
-      // W^T occupies (wt_last_in_place), by a launch of its own once this
-      // band is done
-      const bool tr_late = L.wt_last_in_place && b + 2 == nbands;
-      if (r == 0 && b + 1 < nbands && !tr_late) p.nb_tr = transpose_params(b + 1, p.tr);
       long m0, rows;
       block_span(r, m0, rows);
       const int gm = (int)ceil_div(rows, kBM);
       // K splits of this unit: every split non-empty and a whole number of slabs
       int ks = 1;
       if (L.dhpart) {
-        long v0, vb, vb64;
-        band_cols(b, v0, vb, vb64);
-        p.dh_kc = (int)align_up((size_t)ceil_div(vb64, L.dh_ks), 64);
-        ks = (int)ceil_div(vb64, p.dh_kc);
+        long v0, vb;
+        band_cols(b, v0, vb);
+        p.dh_kc = (int)align_up((size_t)ceil_div(vb, L.dh_ks), 64);
+        ks = (int)ceil_div(vb, p.dh_kc);
       }
       p.dh_split = L.dhpart != nullptr;  // every unit, even one left with a single split
       p.dh_ks = ks;
@@ -2918,38 +2874,27 @@ int cce_backward(const float* grad_out, const void* hidden, const void* weight, 
                          dim3(256), 0, st, dh_reduction(u, prev_ks));
       HIP_TRY(hipGetLastError());
     }
-    if (need_dh && L.wt_last_in_place && b + 2 == nbands && r == R - 1) {
-      rc = transpose_band(b + 1);
-      if (rc) return rc;
-    }
     if (need_db) {
       rc = colsum_unit(b, r, G);
       if (rc) return rc;
     }
   }
-  // outputs whose memory held W^T / H^T during the bands: the last band's
-  // dW from its fp32 accumulator, then dH (the labelled rows) through the
-  // row map; the rows without a label are zeroed last
-  auto convert = [&](const float* src, long rows, const int* live, const int* rowmap, void* out) {
+  // dH of the labelled rows from its accumulator, where grad_hidden held
+  // scratch; the rows without a label are zeroed last
+  if (L.dh_late) {
     DhReduce c = {};
-    c.P = src;
+    c.P = L.dHacc;
     c.ks = 1;
-    c.N = (int)rows; c.d = (int)d;
-    c.live = live; c.live_base = 0;
+    c.N = (int)N; c.d = (int)d;
+    c.live = L.live; c.live_base = 0;
     c.mode = 0;
-    c.out = out; c.out_f32 = 0;
-    c.rowmap = rowmap;
-    hipLaunchKernelGGL(dh_reduce_kernel, dim3((unsigned)std::min<long>(ceil_div(rows * (d / 4), 256), 2048)),
-                       dim3(256), 0, st, c);
-    return hipGetLastError();
-  };
-  if (L.wt_last_in_place) {
-    long v0, vb, vb64;
-    band_cols(nbands - 1, v0, vb, vb64);
-    HIP_TRY(convert(L.dWacc, vb, nullptr, nullptr, dw_rows(nbands - 1)));
+    c.out = grad_hidden; c.out_f32 = 0;
+    c.rowmap = L.idx;
+    hipLaunchKernelGGL(dh_reduce_kernel, dim3((unsigned)std::min<long>(ceil_div(N * (d / 4), 256), 2048)), dim3(256),
+                       0, st, c);
+    HIP_TRY(hipGetLastError());
   }
-  if (L.dh_late) HIP_TRY(convert(L.dHacc, N, L.live, L.idx, grad_hidden));
-  if (need_dh) {
+  if (need_dh && L.idx) {
     const long row_bytes = d * (dh_f32 ? 4 : 2);
     hipLaunchKernelGGL(zero_rows_kernel, dim3((unsigned)std::min<long>(ceil_div(N * (row_bytes / 16), 256), 4096)),
                        dim3(256), 0, st, static_cast<char*>(grad_hidden), row_bytes, L.idx, L.live, (int)N);

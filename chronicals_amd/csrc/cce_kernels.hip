@@ -52,13 +52,16 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-// GEMM configuration: waves per workgroup and column tile BN (256, or 128 for
-// the tail of a hidden dimension).
-constexpr int kWarp8 = 8;
+// GEMM configuration: a workgroup of 4 waves (one per SIMD, 2 x 2 over the
+// tile) computes 256 x BN tiles, BN = 256, or 128 for the tail of a hidden
+// dimension.
+constexpr int kThreads = 256;
 constexpr int kBN = 256;
 constexpr int kTailBN = 128;
 
 constexpr int kBM = 256;              // rows of a workgroup tile
+constexpr int kWaveRows = 128;        // rows of a wave tile (its columns: BN / 2)
+constexpr int kFM = kWaveRows / 32;   // 32-row MFMA blocks of a wave tile
 constexpr int kBK = 64;               // K slab per pipeline step
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.69314718055994531f;
@@ -104,16 +107,6 @@ __device__ inline void grouped_map(int bid, int nb, int gm, int gn, int& pm, int
   pn = r / rows;
 }
 
-// Per-kernel wave layout.  W = 8: two waves per SIMD, 64-row wave tiles,
-// accumulators in VGPRs.  W = 4: one wave per SIMD, 128-row wave tiles,
-// accumulators in AGPRs.  Waves form (256 / kWaveRows) x 2 over a tile.
-template <int W>
-struct WaveCfg {
-  static constexpr int kThreads = W * 64;
-  static constexpr int kWaveRows = (W == 8) ? 64 : 128;
-  static constexpr int kFM = kWaveRows / 32;  // 32-row MFMA blocks per wave tile
-};
-
 // Row compaction: when `dyn` is set, `live` points at the device-side count
 // of live rows (a multiple of 256, or the row count), and the operand's rows
 // start at row live_base of that order (a block of rows), so the block holds
@@ -148,29 +141,46 @@ __device__ inline int live_rows(const int* live, int base) { return max(0, *live
 
 // Accumulator tile of one wave: kWaveRows rows x (BN/2) columns as
 // kFM x (BN/64) blocks of 32x32 fp32.
-template <int BN, int W>
+template <int BN>
 struct WaveAcc {
-  static constexpr int FM = WaveCfg<W>::kFM;
   static constexpr int FN = BN / 64;
-  f32x16 v[FM][FN];
-  __device__ inline void zero() {
+  f32x16 v[kFM][FN];
+  // Orders the accumulators' MFMAs: those of one k-step stay between two
+  // pins (MFMA builtins have no side effects, so nothing else would hold them
+  // in program order and the interleaving of the main loop would not survive).
+  __device__ inline void pin() {
 #pragma unroll
-    for (int i = 0; i < FM; ++i)
+    for (int i = 0; i < kFM; ++i)
 #pragma unroll
-      for (int j = 0; j < FN; ++j)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) v[i][j][r] = 0.f;
+      for (int j = 0; j < FN; ++j) asm volatile("" : "+a"(v[i][j]));
+  }
+  // Block (i, j) in vector registers, copied here and not earlier (the
+  // epilogue holds a few blocks at a time).
+  __device__ inline f32x16 take(int i, int j) {
+    asm volatile("" : "+a"(v[i][j]));
+    f32x16 x = v[i][j];
+    asm volatile("" : "+v"(x));
+    return x;
   }
 };
+
+__device__ inline __amdgpu_buffer_rsrc_t make_rsrc(const void* base, long bytes) {
+  const long cap = 0x7ffffff0L;
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)(bytes < cap ? bytes : cap),
+                                           0x00020000);
+}
+
+// Four consecutive floats of a buffer from byte offset `off` on (4-byte
+// aligned); those past its end are 0.
+__device__ inline f32x4 load4(__amdgpu_buffer_rsrc_t rs, int off) {
+  return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0));
+}
 
 // Lane <-> element map of a wave tile.  The B fragment is passed as the
 // instruction's first operand, so each 32x32 block holds C^T in the hardware
 // layout: lane l owns row m = i*32 + (l & 31) and, for register r = 4q + e,
 // column n = j*32 + 8q + 4*(l >> 5) + e — four consecutive columns per q.
-template <int W>
-__device__ inline int acc_row(int wm, int i, int l) {
-  return wm * WaveCfg<W>::kWaveRows + i * 32 + (l & 31);
-}
+__device__ inline int acc_row(int wm, int i, int l) { return wm * kWaveRows + i * 32 + (l & 31); }
 template <int BN>
 __device__ inline int acc_col(int wn, int j, int q, int l) {
   return wn * (BN / 2) + j * 32 + q * 8 + (l >> 5) * 4;
@@ -196,119 +206,100 @@ __device__ inline void pin_epilogue(int& l, int& tm, int& tn) {
 // ---------------------------------------------------------------------------
 __device__ inline int swz(int r) { return (r ^ (r >> 3)) & 7; }
 
-// s_waitcnt immediate for vmcnt(n) alone (expcnt and lgkmcnt at their no-wait
-// maxima): vmcnt bits [3:0] and [15:14], expcnt [6:4], lgkmcnt [11:8].
-constexpr int vmcnt_imm(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }
+// s_waitcnt immediate (vmcnt bits [3:0] and [15:14], expcnt [6:4], lgkmcnt
+// [11:8]; all ones: no wait).
+constexpr int kWaitLds = 15 | (3 << 14) | (7 << 4);  // lgkmcnt(0) alone
 
-__device__ inline __amdgpu_buffer_rsrc_t make_rsrc(const void* base, long bytes) {
-  const long cap = 0x7ffffff0L;
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)(bytes < cap ? bytes : cap),
-                                           0x00020000);
-}
+constexpr int kOutOfRange = (int)0x80000000u;  // a lane offset past every descriptor's range
 
-// Issue the DMA of a K-major tile: rows [r0, r0 + BR) x k [k0, k0 + 64) into
-// the swizzled LDS region S.  Rows past rlim fall outside the descriptor's
-// range and read as zero.  k0 goes in the scalar offset, which a raw buffer
-// does not range-check: every slab must end inside its row (k0 + 64 <= ld),
-// which kmajor_fits() checks on the host for every launch.  KTAIL: K is no
-// multiple of 64 and the rows hold only K columns; the lanes of the last slab
-// whose 8 columns start at K or later get an offset past the descriptor's
-// range, so they read as zero (K is a multiple of 8).  That costs a compare and
-// a select per DMA instruction, against a register-staged pipeline in 128-wide
-// tiles with separate recompute and gradient launches before: N 1500, d 1000,
-// V 50257 with bias, forward and backward 2116 -> 1200 us.
-constexpr int kOutOfRange = (int)0x80000000u;
-template <int BR, int W, bool KTAIL = false>
-__device__ inline void dma_kmajor(const bf16_t* __restrict__ X, long ld, int r0, int rlim, int k0, int K, bf16_t* S,
-                                  int w, int l) {
-  constexpr int kI = BR / (8 * W);  // wave instructions per wave
-  const long rows_left = (long)rlim - r0;
-  const __amdgpu_buffer_rsrc_t rs = make_rsrc(X + (long)r0 * ld, rows_left > 0 ? rows_left * ld * 2 : 0);
-#pragma unroll
-  for (int j = 0; j < kI; ++j) {
-    const int blk = w * kI + j;           // 8-row block of the tile
-    const int row = blk * 8 + (l >> 3);
-    const int c = (l & 7) ^ swz(row);     // logical chunk this lane fetches
-    int voff = (int)(((long)row * ld + c * 8) * 2);
-    if constexpr (KTAIL) voff = k0 + c * 8 < K ? voff : kOutOfRange;
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(
-        rs, (__attribute__((address_space(3))) void*)(S + blk * 512), 16, voff, k0 * 2, 0, 0);
-  }
-}
-
-// The K-major A tile a workgroup streams (rows [r0, r0 + kBM) of a GEMM with
-// rlim rows) read through a row map: GEMM row m is row arow[m] of A, which
-// has arows rows.  The buffer descriptor spans all of A; for each DMA
-// instruction j of the wave, each lane keeps the byte offset of its 16-byte
-// chunk at k = 0 (the slab's k0 goes in the instruction's scalar offset),
-// computed once per workgroup.  Rows past rlim get an offset past the descriptor's
-// range and read as zero.
-template <int W>
-struct ARows {
-  static constexpr int kI = kBM / (8 * W);
+// The stream of 64-deep slabs of one operand, copied into LDS units of
+// [BR rows][64 k] one wave instruction (1 KB) at a time: instruction j of wave
+// w fills elements [512 * (w * kI + j), +512) of the unit.  The lane offsets
+// are computed once per workgroup; a slab's position is in the descriptor's
+// base or in the instruction's scalar offset.
+//
+// KM (element (r, k) at X[r*ld + k]): an instruction fills 8 rows x 128 B, with
+// 16-byte chunk c of row r at physical chunk c ^ swz(r).  Rows past the end
+// fall outside the descriptor's range and read as zero.  The slab's k goes in
+// the scalar offset, which a raw buffer does not range-check: every slab must
+// end inside its row (k + 64 <= ld), which kmajor_fits() checks on the host for
+// every launch.  TAIL: K is no multiple of 64 and the rows hold only K columns;
+// the lanes of the last slab whose 8 columns start at K or later get an offset
+// past the descriptor's range, so they read as zero (K is a multiple of 8).
+// That costs a compare and a select per instruction, against a register-staged
+// pipeline in 128-wide tiles with separate recompute and gradient launches
+// before: N 1500, d 1000, V 50257 with bias, forward and backward 2116 -> 1200
+// us.  ROWS: row r of the tile is row map[r] of X, which has xrows rows; the
+// descriptor spans all of X.
+//
+// Otherwise (element (r, k) at X[k*ld + r], MN-major): an instruction fills
+// 512 / BR k rows, with 16-byte chunk c of k row q at physical chunk
+// c ^ (4*(q & 3)), so the four rows touched by one transposed fragment read
+// land on distinct banks.  Rows k >= K fall outside the range and read as zero;
+// columns past a row's end read the next row (the epilogues mask them).
+template <bool KM, int BR, bool TAIL = false, bool ROWS = false>
+struct Stream {
+  static_assert(KM || !(TAIL || ROWS), "the K tail and the row map are for K-major operands");
+  static constexpr int kI = BR / 32;  // wave instructions per wave and slab
   const bf16_t* base;
-  long bytes;
-  int voff[kI];
-  __device__ inline void init(const bf16_t* __restrict__ X, long ld, int r0, int rlim, const int* __restrict__ arow,
-                              long arows, int w, int l) {
-    const long rows_left = (long)rlim - r0;
-    base = X;
-    bytes = arows * ld * 2;
+  long bytes;   // in the descriptor's range from base
+  long step;    // bytes from slab to slab (MN-major)
+  int v[kI];
+  int k, K, cl;  // k of the next slab (K-major: with kb), its limit, lane chunk before the swizzle
+  // the tile that starts at row r0 of the operand (rlim rows), from k = kb on
+  __device__ inline void init(const bf16_t* X, long ld, int r0, int rlim, int kb, int K_, const int* map, long xrows,
+                              int w, int l) {
+    k = KM ? kb : 0;
+    K = kb + K_;
+    if constexpr (KM) {
+      const long left = max((long)rlim - r0, 0L);
+      base = ROWS ? X : X + (long)r0 * ld;
+      bytes = (ROWS ? xrows : left) * ld * 2;
+      cl = (l & 7) ^ (l >> 3);
 #pragma unroll
-    for (int j = 0; j < kI; ++j) {
-      const int row = (w * kI + j) * 8 + (l >> 3);
-      const int c = (l & 7) ^ swz(row);
-      voff[j] = row < rows_left ? (int)(((long)arow[r0 + row] * ld + c * 8) * 2) : kOutOfRange;
+      for (int j = 0; j < kI; ++j) {
+        const int row = (w * kI + j) * 8 + (l >> 3), c = (l & 7) ^ swz(row);
+        if constexpr (ROWS)
+          v[j] = row < left ? (int)(((long)map[r0 + row] * ld + c * 8) * 2) : kOutOfRange;
+        else
+          v[j] = (int)(((long)row * ld + c * 8) * 2);
+      }
+    } else {
+      constexpr int kLanes = BR / 8;  // lanes per k row
+      base = X + r0;
+      bytes = max(((long)K_ * ld - r0) * 2, 0L);
+      step = ld * (kBK * 2);
+#pragma unroll
+      for (int j = 0; j < kI; ++j) {
+        const int row = (w * kI + j) * (64 / kLanes) + l / kLanes;
+        v[j] = (int)(((long)row * ld + ((l % kLanes) ^ (4 * (row & 3))) * 8) * 2);
+      }
     }
   }
-  // the DMA of k [k0, k0 + 64) into the swizzled LDS region S
-  __device__ inline void dma(int k0, bf16_t* S, int w) const {
-    const __amdgpu_buffer_rsrc_t rs = make_rsrc(base, bytes);
+  // instructions [J0, J1) of the next slab into unit S; without `some` they
+  // read nothing and write zeros (the stream's end)
+  template <int J0, int J1>
+  __device__ inline void issue(bf16_t* S, bool some, int w) const {
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc(base, some ? bytes : 0L);
+    const int so = KM ? k * 2 : 0;
 #pragma unroll
-    for (int j = 0; j < kI; ++j)
+    for (int j = J0; j < J1; ++j) {
+      int vo = v[j];
+      if constexpr (TAIL) vo = k + (cl ^ ((w * kI + j) & 7)) * 8 < K ? vo : kOutOfRange;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          rs, (__attribute__((address_space(3))) void*)(S + (w * kI + j) * 512), 16, voff[j], k0 * 2, 0, 0);
+          rs, (__attribute__((address_space(3))) void*)(S + (w * kI + j) * 512), 16, vo, so, 0, 0);
+    }
+  }
+  // on to the next slab of the tile
+  __device__ inline void next() {
+    if constexpr (KM) {
+      k += kBK;
+    } else {
+      base += step / 2;
+      bytes = max(bytes - step, 0L);
+    }
   }
 };
-
-// MN-major tile: element (m, k) at X[k*ld + m].  The tile k [k0, k0 + 64) x
-// m [m0, m0 + BR) goes to LDS in rows of one k.  One wave instruction fills
-// 1 KB = 512 / BR rows, k = 8q + s and its followers in steps of 4 (k mod 4 is
-// the same for all of them when BR = 256; with BR = 128 it takes the four rows
-// k, k + 4, k + 8, k + 12 of a group of 16), and blocks lie kMnBlock elements
-// apart: 64 bytes of padding shift the four rows that one transposed fragment
-// read touches (k mod 4 = 0..3) onto distinct banks, and every fragment's
-// address is one lane address plus a constant.  Rows k >= K fall outside the
-// descriptor's range and read as zero; columns past a row's end read the next
-// row (the epilogues mask them).
-constexpr int kMnBlock = 512 + 32;
-template <int BR>
-__host__ __device__ constexpr int mn_rows() { return 512 / BR; }  // k rows of a block
-// Element offset of k row `k`: groups of 4 * mn_rows k rows are 4 blocks, block k & 3.
-template <int BR>
-__device__ constexpr int mn_row(int k) {
-  constexpr int R = mn_rows<BR>();
-  return ((k / (4 * R)) * 4 + (k & 3)) * kMnBlock + ((k >> 2) % R) * BR;
-}
-template <int BR, int W>
-__device__ inline void dma_mnmajor(const bf16_t* __restrict__ X, long ld, int m0, int k0, int K, bf16_t* S, int w,
-                                   int l) {
-  static_assert(BR == 256 || BR == 128, "2 or 4 rows in a block");
-  constexpr int R = mn_rows<BR>();
-  constexpr int kI = BR / (8 * W);    // wave instructions per wave
-  constexpr int kLanes = BR / 8;      // lanes per k row
-  const long rows_left = (long)K - k0;
-  const long bytes = rows_left > 0 ? (rows_left * ld - m0) * 2 : 0;
-  const __amdgpu_buffer_rsrc_t rs = make_rsrc(X + (long)k0 * ld + m0, bytes);
-#pragma unroll
-  for (int j = 0; j < kI; ++j) {
-    const int blk = w * kI + j;
-    const int row = (blk >> 2) * 4 * R + (blk & 3) + 4 * (l / kLanes);
-    const int voff = (int)(((long)row * ld + (l % kLanes) * 8) * 2);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(
-        rs, (__attribute__((address_space(3))) void*)(S + blk * kMnBlock), 16, voff, 0, 0, 0);
-  }
-}
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
@@ -317,21 +308,22 @@ typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 // the 8-byte reads addressed by lanes (j>>2) + 4t, t = 0..3.  Lane a of the
 // group addresses row k = kb + (a>>2), columns m = mb + 4*(a&3) .. +3 of the
 // [k][m] tile, so lane j receives k = kb..kb+3 of column m = mb + j.
-__device__ inline uint2 read_tr4(const bf16_t* S) {
-  const s16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)S);
+template <int BR>
+__device__ inline uint2 read_tr4(const bf16_t* S, int k, int m) {
+  const int phys = (((m >> 3) ^ (4 * (k & 3))) << 3) + (m & 7);
+  const s16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(S + k * BR + phys));
   return __builtin_bit_cast(uint2, v);
 }
 
 // Register fragments of one k-step (16 of K) for a wave.
-template <int BN, int W>
+template <int BN>
 struct Frags {
-  u32x4 a[WaveCfg<W>::kFM], b[BN / 64];
+  u32x4 a[kFM], b[BN / 64];
 };
 
-// One operand's fragments of k-step kk from an unpadded LDS tile, for the
-// FR 32-row blocks from tile row r0: lane l gets row r0 + i*32 + (l & 31),
-// k = kk*16 + 8*(l >> 5) + 0..7.  KM: the swizzled [row][64 k] layout;
-// otherwise the [k][BR rows] layout, read transposed.
+// One operand's fragments of k-step kk from an LDS unit, for the FR 32-row
+// blocks from tile row r0: lane l gets row r0 + i*32 + (l & 31),
+// k = kk*16 + 8*(l >> 5) + 0..7.
 template <bool KM, int BR, int FR>
 __device__ inline void read_op(const bf16_t* __restrict__ S, int kk, int r0, u32x4 (&f)[FR], int l) {
   if constexpr (KM) {
@@ -342,25 +334,27 @@ __device__ inline void read_op(const bf16_t* __restrict__ S, int kk, int r0, u32
       f[i] = *reinterpret_cast<const u32x4*>(S + r * 64 + ((c ^ swz(r)) << 3));
     }
   } else {
-    // k = kk*16 + 8*(l >> 5) + (a >> 2) and that + 4, a = l & 15
     const int a = l & 15;
-    const bf16_t* const base = S + mn_row<BR>(8 * (l >> 5) + (a >> 2)) + r0 + 16 * ((l >> 4) & 1) + 4 * (a & 3);
+    const int kb = kk * 16 + 8 * (l >> 5) + (a >> 2);
 #pragma unroll
     for (int i = 0; i < FR; ++i) {
-      const uint2 lo = read_tr4(base + mn_row<BR>(kk * 16) + i * 32);
-      const uint2 hi = read_tr4(base + mn_row<BR>(kk * 16) + mn_row<BR>(4) + i * 32);
+      const int mb = r0 + i * 32 + 16 * ((l >> 4) & 1) + 4 * (a & 3);
+      const uint2 lo = read_tr4<BR>(S, kb, mb);
+      const uint2 hi = read_tr4<BR>(S, kb + 4, mb);
       f[i] = u32x4{lo.x, lo.y, hi.x, hi.y};
     }
   }
 }
 
-// v_mfma_f32_32x32x16_bf16 over the kFM x (BN/64) blocks of one k-step.
-template <int BN, int W>
-__device__ inline void mfma_frags(const Frags<BN, W>& f, WaveAcc<BN, W>& acc) {
+// v_mfma_f32_32x32x16_bf16 over the kFM x (BN/64) blocks of one k-step; FIRST:
+// the tile's first, onto zero.
+template <int BN, bool FIRST>
+__device__ inline void mfma_frags(const Frags<BN>& f, WaveAcc<BN>& acc) {
+  const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int i = 0; i < WaveCfg<W>::kFM; ++i)
+  for (int i = 0; i < kFM; ++i)
 #pragma unroll
-    for (int j = 0; j < BN / 64; ++j) acc.v[i][j] = mfma_32x32x16(f.b[j], f.a[i], acc.v[i][j]);
+    for (int j = 0; j < BN / 64; ++j) acc.v[i][j] = mfma_32x32x16(f.b[j], f.a[i], FIRST ? zero : acc.v[i][j]);
 }
 
 // ---------------------------------------------------------------------------
@@ -391,12 +385,12 @@ __host__ __device__ inline float split_cost(int gl, int tn, int s, int ncu) {
 
 // Forward: per-row online (max, sum-exp) in base 2 over the workgroup's run of
 // vocabulary tiles; at the end one partial per (row, split) is written.
-template <int BN, int W, bool HB>
+template <int BN, bool HB>
 struct EpiLseT {
   typedef LseParams Params;
   static constexpr bool kOneTile = false;
   static constexpr bool kDynSplits = true;
-  static constexpr int FM = WaveCfg<W>::kFM;
+  static constexpr int FM = kFM;
   struct State {
     float m[FM], s[FM];
   };
@@ -414,7 +408,6 @@ struct EpiLseT {
     t0 = (int)(((long)p.tiles_n * s) / S);
     t1 = (int)(((long)p.tiles_n * (s + 1)) / S);
   }
-  static constexpr int kStores = 0;  // global stores a tile epilogue issues per wave
   static __device__ inline void init(const Params&, State& st, const GemmShape&, int, int, int) {
 #pragma unroll
     for (int i = 0; i < FM; ++i) {
@@ -422,61 +415,61 @@ struct EpiLseT {
       st.s[i] = 0.f;
     }
   }
-  static constexpr int kScratch = 0;  // LDS elements the epilogue stages through
-  static __device__ inline void tile(const Params& p, State& st, WaveAcc<BN, W>& acc, const GemmShape& g, int tm,
+  static __device__ inline void tile(const Params& p, State& st, WaveAcc<BN>& acc, const GemmShape& g, int tm,
                                      int tn, int wm, int wn, int l, bf16_t*) {
     constexpr int FN = BN / 64;
     pin_epilogue(l, tm, tn);
     const int c0 = tn * BN;
-    if (!HB && c0 + BN <= g.N) {
-      // interior tile: max over raw logits (log2e > 0 commutes with max), then
-      // one fused exp2(x*log2e - m) per element
-#pragma unroll
-      for (int i = 0; i < FM; ++i) {
-        float mx = kNegBig;
-#pragma unroll
-        for (int j = 0; j < FN; ++j)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) mx = fmaxf(mx, acc.v[i][j][r]);
-        const float mn = fmaxf(st.m[i], mx * kLog2e);
-        float sum = 0.f;
-#pragma unroll
-        for (int j = 0; j < FN; ++j)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) sum += fast_exp2(__builtin_fmaf(acc.v[i][j][r], kLog2e, -mn));
-        st.s[i] = st.s[i] * fast_exp2(st.m[i] - mn) + sum;
-        st.m[i] = mn;
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      return;
-    }
-    // edge tile or bias: per-column offset, columns past V excluded
-#pragma unroll
-    for (int i = 0; i < FM; ++i) {
+    // max over raw logits (log2e > 0 commutes with max), then one fused
+    // exp2(x*log2e - m) per element
+    auto update = [&](int i, const f32x16 (&x)[FN]) {
       float mx = kNegBig;
 #pragma unroll
       for (int j = 0; j < FN; ++j)
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int col = c0 + acc_col<BN>(wn, j, q, l) + e;
-            if (col < g.N) mx = fmaxf(mx, (acc.v[i][j][4 * q + e] + (HB ? p.bias[col] : 0.f)) * kLog2e);
-          }
-      const float mn = fmaxf(st.m[i], mx);
+        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, x[j][r]);
+      const float mn = fmaxf(st.m[i], mx * kLog2e);
       float sum = 0.f;
 #pragma unroll
       for (int j = 0; j < FN; ++j)
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int col = c0 + acc_col<BN>(wn, j, q, l) + e;
-            if (col < g.N) sum += fast_exp2((acc.v[i][j][4 * q + e] + (HB ? p.bias[col] : 0.f)) * kLog2e - mn);
-          }
+        for (int r = 0; r < 16; ++r) sum += fast_exp2(__builtin_fmaf(x[j][r], kLog2e, -mn));
       st.s[i] = st.s[i] * fast_exp2(st.m[i] - mn) + sum;
       st.m[i] = mn;
       __builtin_amdgcn_sched_barrier(0);
+    };
+    if (!HB && c0 + BN <= g.N) {
+#pragma unroll
+      for (int i = 0; i < FM; ++i) {
+        f32x16 x[FN];
+#pragma unroll
+        for (int j = 0; j < FN; ++j) x[j] = acc.take(i, j);
+        update(i, x);
+      }
+      return;
+    }
+    // edge tile or bias: the columns' bias added, columns past V at -inf
+    const __amdgpu_buffer_rsrc_t bias = make_rsrc(p.bias, HB ? (long)g.N * 4 : 0L);
+#pragma unroll
+    for (int i = 0; i < FM; ++i) {
+      f32x16 x[FN];
+      int lp = l;
+      asm volatile("" : "+v"(lp));  // the columns' masks and bias are not kept from row block to row block
+#pragma unroll
+      for (int j = 0; j < FN; ++j) {
+        x[j] = acc.take(i, j);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int col = c0 + acc_col<BN>(wn, j, q, lp);
+          f32x4 b = {0.f, 0.f, 0.f, 0.f};
+          if constexpr (HB) b = load4(bias, col * 4);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) x[j][4 * q + e] = col + e < g.N ? x[j][4 * q + e] + b[e] : -INFINITY;
+        }
+        asm volatile("" ::: "memory");  // one block's bias loads at a time
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      update(i, x);
     }
   }
   static __device__ inline void merge(float& m, float& s, float m2, float s2) {
@@ -493,7 +486,7 @@ struct EpiLseT {
     if (wn == 1 && l < 32) {
 #pragma unroll
       for (int i = 0; i < FM; ++i) {
-        const int row = acc_row<W>(wm, i, l);
+        const int row = acc_row(wm, i, l);
         red[row] = st.m[i];
         red[kBM + row] = st.s[i];
       }
@@ -502,7 +495,7 @@ struct EpiLseT {
     if (wn == 0 && l < 32) {
 #pragma unroll
       for (int i = 0; i < FM; ++i) {
-        const int row = acc_row<W>(wm, i, l);
+        const int row = acc_row(wm, i, l);
         merge(st.m[i], st.s[i], red[row], red[kBM + row]);
         const int grow = tm * kBM + row;
         if (grow < g.M) {
@@ -515,10 +508,10 @@ struct EpiLseT {
   }
 };
 
-template <int BN, int W>
-using EpiLse = EpiLseT<BN, W, false>;
-template <int BN, int W>
-using EpiLseBias = EpiLseT<BN, W, true>;
+template <int BN>
+using EpiLse = EpiLseT<BN, false>;
+template <int BN>
+using EpiLseBias = EpiLseT<BN, true>;
 
 struct GradParams {
   const float* bias;     // [V] or null (full vocabulary, indexed by v0 + c)
@@ -527,7 +520,6 @@ struct GradParams {
   bf16_t* G;             // [M][ldg]
   long ldg;
   int v0;                // first vocabulary row of the band
-  int splits;            // column-tile runs per row tile
   int tiles_n;           // column tiles in the band
 };
 
@@ -540,24 +532,14 @@ struct GradParams {
 // row so the 16 lanes of a write phase hit distinct banks), reads it back
 // row-major and stores whole 128-byte row segments, 8 rows per instruction.
 // A wave's LDS operations execute in order, so no barrier is needed.
-// ONE: a workgroup takes one column tile (splits == tiles_n); otherwise it
-// walks a run of column tiles of one row tile, so the next tile's loads are in
-// flight while this tile's epilogue runs.
-template <int BN, int W, bool HB, bool ONE>
+template <int BN, bool HB>
 struct EpiGradT {
   typedef GradParams Params;
-  static constexpr bool kOneTile = ONE;
+  static constexpr bool kOneTile = true;  // splits == tiles_n: a workgroup takes one column tile
   static constexpr bool kDynSplits = false;
-  static constexpr int FM = WaveCfg<W>::kFM;
-  static constexpr int kScratch = W * 2048;  // 32 x 64 bf16 per wave
-  // Without bias the tile epilogue issues exactly kStores buffer stores per
-  // wave and no other vector memory operation (rows past M fall outside the
-  // store descriptor and are dropped, so no wave branches around a store);
-  // the per-row parameters are loaded once per workgroup (its row tile is
-  // fixed), since a load issued after a tile's stores would wait for all of
-  // them.  With bias the epilogue loads bias values, and its stores are
-  // waited for in full at the next barrier (kStores = 0).
-  static constexpr int kStores = HB ? 0 : FM * (BN / 128) * 4;
+  static constexpr int FM = kFM;
+  // The per-row parameters are loaded once, before the K loop; with bias they
+  // are loaded in the epilogue beside the bias values.
   static constexpr int kRows = HB ? 1 : FM;
   struct State {
     float4 rp[kRows];
@@ -566,11 +548,8 @@ struct EpiGradT {
   static __device__ inline void assign(const GemmShape& g, const Params& p, int bid, int nb, int& tm, int& t0,
                                        int& t1, int& split) {
     const int gm = (g.M + kBM - 1) / kBM;
-    int s;
-    grouped_map(bid, nb, gm, p.splits, tm, s);
-    split = s;
-    t0 = (int)(((long)p.tiles_n * s) / p.splits);
-    t1 = (int)(((long)p.tiles_n * (s + 1)) / p.splits);
+    grouped_map(bid, nb, gm, p.tiles_n, tm, t0);
+    split = 0;
   }
   static __device__ inline void row_params(const Params& p, const GemmShape& g, int m, float4& rp, int& lab) {
     const int mc = m < g.M ? m : 0;
@@ -580,10 +559,10 @@ struct EpiGradT {
   static __device__ inline void init(const Params& p, State& st, const GemmShape& g, int tm, int wm, int l) {
     if constexpr (!HB) {
 #pragma unroll
-      for (int i = 0; i < FM; ++i) row_params(p, g, tm * kBM + acc_row<W>(wm, i, l), st.rp[i], st.lab[i]);
+      for (int i = 0; i < FM; ++i) row_params(p, g, tm * kBM + acc_row(wm, i, l), st.rp[i], st.lab[i]);
     }
   }
-  static __device__ inline void tile(const Params& p, State& st, WaveAcc<BN, W>& acc, const GemmShape& g, int tm,
+  static __device__ inline void tile(const Params& p, State& st, WaveAcc<BN>& acc, const GemmShape& g, int tm,
                                      int tn, int wm, int wn, int l, bf16_t* scratch) {
     constexpr int FN = BN / 64;
     static_assert(FN % 2 == 0, "64-column staging blocks");
@@ -598,7 +577,7 @@ struct EpiGradT {
     const bool interior = !HB && (tn + 1) * BN <= g.N;
 #pragma unroll
     for (int i = 0; i < FM; ++i) {
-      const int m = tm * kBM + acc_row<W>(wm, i, l);
+      const int m = tm * kBM + acc_row(wm, i, l);
       const bool mok = m < g.M;
       float4 rp;
       int lab;
@@ -610,6 +589,7 @@ struct EpiGradT {
       }
 #pragma unroll
       for (int jp = 0; jp < FN / 2; ++jp) {
+        const f32x16 x[2] = {acc.take(i, 2 * jp), acc.take(i, 2 * jp + 1)};
         // G without the one-hot term, packed to bf16 into the staging block;
         // the 8-byte piece hc (of 16 per 128-byte row) lives at hc ^ (row & 15)
         auto stage = [&](int jj, int q, const float (&gv)[4]) {
@@ -625,7 +605,7 @@ struct EpiGradT {
               float gv[4];
 #pragma unroll
               for (int e = 0; e < 4; ++e)
-                gv[e] = __builtin_fmaf(rp.y, fast_exp2(__builtin_fmaf(acc.v[i][2 * jp + jj][4 * q + e], kLog2e, -rp.x)),
+                gv[e] = __builtin_fmaf(rp.y, fast_exp2(__builtin_fmaf(x[jj][4 * q + e], kLog2e, -rp.x)),
                                        -rp.w);
               stage(jj, q, gv);
             }
@@ -642,7 +622,7 @@ struct EpiGradT {
                 float gg = 0.f;
                 if (mok && col < g.N) {
                   const float b = HB ? p.bias[p.v0 + col] : 0.f;
-                  gg = rp.y * fast_exp2((acc.v[i][2 * jp + jj][4 * q + e] + b) * kLog2e - rp.x) - rp.w;
+                  gg = rp.y * fast_exp2((x[jj][4 * q + e] + b) * kLog2e - rp.x) - rp.w;
                 }
                 gv[e] = gg;
               }
@@ -666,7 +646,7 @@ struct EpiGradT {
           // 16-byte chunk c = pieces 2c, 2c+1, stored at slot c ^ ((rr & 14) >> 1), halves swapped for odd rows
           u32x4 v = *reinterpret_cast<const u32x4*>(ws + rr * 64 + ((c ^ ((rr & 14) >> 1)) << 3));
           if (rr & 1) v = u32x4{v[2], v[3], v[0], v[1]};
-          const int trow = wm * WaveCfg<W>::kWaveRows + i * 32 + rr;
+          const int trow = wm * kWaveRows + i * 32 + rr;
           const int gcol = tn * BN + wn * (BN / 2) + jp * 64 + c * 8;
           __builtin_amdgcn_raw_buffer_store_b128(v, gr, (int)(((long)trow * p.ldg + gcol) * 2), 0, 0);
         }
@@ -680,14 +660,10 @@ struct EpiGradT {
                                        int) {}
 };
 
-template <int BN, int W>
-using EpiGrad = EpiGradT<BN, W, false, false>;
-template <int BN, int W>
-using EpiGradBias = EpiGradT<BN, W, true, false>;
-template <int BN, int W>
-using EpiGradTile = EpiGradT<BN, W, false, true>;
-template <int BN, int W>
-using EpiGradBiasTile = EpiGradT<BN, W, true, true>;
+template <int BN>
+using EpiGrad = EpiGradT<BN, false>;
+template <int BN>
+using EpiGradBias = EpiGradT<BN, true>;
 
 struct AccParams {
   float* acc32;
@@ -703,13 +679,12 @@ struct AccParams {
 //   mode 0: out = C            1: acc32 = C
 //   mode 2: acc32 += C          3: out = acc32 + C
 //   mode 4: out += C (fp32 output only: the output is its own accumulator)
-template <int BN, int W>
+template <int BN>
 struct EpiAcc {
   typedef AccParams Params;
   static constexpr bool kOneTile = true;
   static constexpr bool kDynSplits = false;
-  static constexpr int FM = WaveCfg<W>::kFM;
-  static constexpr int kScratch = 0;
+  static constexpr int FM = kFM;
   struct State {};
   static __device__ inline void assign(const GemmShape& g, const Params&, int bid, int nb, int& tm, int& t0,
                                        int& t1, int& split) {
@@ -720,16 +695,15 @@ struct EpiAcc {
     t1 = tn + 1;
     split = 0;
   }
-  static constexpr int kStores = 0;  // single-tile workgroups: nothing follows the epilogue
   static __device__ inline void init(const Params&, State&, const GemmShape&, int, int, int) {}
-  static __device__ inline void tile(const Params& p, State&, WaveAcc<BN, W>& acc, const GemmShape& g, int tm,
+  static __device__ inline void tile(const Params& p, State&, WaveAcc<BN>& acc, const GemmShape& g, int tm,
                                      int tn, int wm, int wn, int l, bf16_t*) {
     constexpr int FN = BN / 64;
     constexpr int JG = FN >= 2 ? 2 : 1;  // 32 x 64 column blocks whose old values load together
     pin_epilogue(l, tm, tn);
 #pragma unroll
     for (int i = 0; i < FM; ++i) {
-      const int m = tm * kBM + acc_row<W>(wm, i, l);
+      const int m = tm * kBM + acc_row(wm, i, l);
       if (m >= g.M) continue;
 #pragma unroll
       for (int j0 = 0; j0 < FN; j0 += JG) {
@@ -751,13 +725,14 @@ struct EpiAcc {
             }
         }
 #pragma unroll
-        for (int jj = 0; jj < JG; ++jj)
+        for (int jj = 0; jj < JG; ++jj) {
+        const f32x16 x = acc.take(i, j0 + jj);
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           const int j = j0 + jj;
           const int n = tn * BN + acc_col<BN>(wn, j, q, l);
           if (n >= g.N) continue;
-          f32x4 v = {acc.v[i][j][4 * q], acc.v[i][j][4 * q + 1], acc.v[i][j][4 * q + 2], acc.v[i][j][4 * q + 3]};
+          f32x4 v = {x[4 * q], x[4 * q + 1], x[4 * q + 2], x[4 * q + 3]};
           if (p.mode >= 2) v += old[jj][q];
           if (p.mode == 1 || p.mode == 2) {
             *reinterpret_cast<f32x4*>(p.acc32 + (long)m * p.ldacc + n) = v;
@@ -770,6 +745,7 @@ struct EpiAcc {
             }
           }
         }
+        }
       }
     }
   }
@@ -778,23 +754,38 @@ struct EpiAcc {
 };
 
 // ---------------------------------------------------------------------------
-// The GEMM kernel: C[M,N] = A[M,K] . B[N,K]^T, 256 x BN x 64 tiles, operands
-// copied straight into NST unpadded LDS stages (described at the loop below).
-// AK, BK: the operand is K-major, else MN-major and read back transposed.
-// AROW: a K-major A is read through g.arow (ARows).  KTAIL: K-major operands
-// whose K is no multiple of 64 (dma_kmajor).
+// The GEMM kernel: C[M,N] = A[M,K] . B[N,K]^T, 256 x BN x 64 tiles.  AK, BK: the
+// operand is K-major, else MN-major and read back transposed.  AROW: a K-major
+// A is read through g.arow.  KTAIL: K-major operands whose K is no multiple of
+// 64 (Stream).
+//
+// LDS is a ring of five 32 KB units that hold, in turn, one slab of A and one
+// of B: A(0) B(0) A(1) B(1) A(2) ..., so two and a half slabs are in LDS or on
+// their way.  Per slab s (64 of K) and wave:
+//   k-step 0: the fragments of k-step 1 are read and the second half of B(s+1)
+//             is issued while the MFMAs of k-step 0 run;
+//   k-steps 1, 2: likewise, with A(s+2) going to the unit B(s-1) left;
+//   barrier:  every wave has read all of slab s, and slab s+1 has landed (all
+//             but the 8 newest instructions, A(s+2)'s);
+//   k-step 3: the first fragments of slab s+1 are read and the first half of
+//             B(s+2) goes to the unit A(s) leaves.
+// A wave owns its SIMD, so nothing but this order hides latencies: in each
+// k-step the LDS reads go one by one between the first MFMAs and the DMA
+// instructions between the last (a DMA writes LDS, so it cannot pass reads).
+//
+// Measured against two 64 KB stages with 8 waves of 64 x 128 (two per SIMD) and
+// the slab's DMA in one burst at its end, on products of 8192^3 and
+// 16384 x 896 x 8192: 1220 -> 1330 and 990 -> 1150 TFLOP/s.  The burst was what
+// cost most: it fills the address unit's queue (16 cycles an instruction) and
+// stalls the MFMAs behind it.  128 x 128 wave tiles read a third less LDS.
 // ---------------------------------------------------------------------------
-// LDS elements of an operand's tile of BR rows, and of NST stages.
-template <bool KM, int BR>
-constexpr int tile_elems() { return KM ? BR * kBK : BR * kBK / 512 * kMnBlock; }
-template <int BN, bool AK, bool BK, int NST = 2>
-constexpr int gemm_lds_elems() { return NST * (tile_elems<AK, kBM>() + tile_elems<BK, BN>()); }
+constexpr int kUnit = 256 * kBK;            // elements of a ring unit
+constexpr int kLdsElems = 5 * kUnit;        // 160 KB
 
-template <int BN, int W, bool AK, bool BK, template <int, int> class EpiT, int NST = 2, bool AROW = false,
-          bool KTAIL = false>
-__device__ __forceinline__ void gemm_body(const GemmShape& g_in, const typename EpiT<BN, W>::Params& ep, int bid,
-                                          int nb, bf16_t* smem) {
-  typedef EpiT<BN, W> Epi;
+template <int BN, bool AK, bool BK, template <int> class EpiT, bool AROW = false, bool KTAIL = false>
+__device__ __forceinline__ void gemm_body(const GemmShape& g_in, const typename EpiT<BN>::Params& ep, int bid, int nb,
+                                          bf16_t* smem) {
+  typedef EpiT<BN> Epi;
   GemmShape g = g_in;
   if (g.dyn == kDynK) g.K = min(g.K, live_rows(g.live, g.live_base));
   if (g.dyn == kDynM) {
@@ -811,10 +802,9 @@ __device__ __forceinline__ void gemm_body(const GemmShape& g_in, const typename 
       if (bid >= nb) return;
     }
   }
-  // epilogue staging area, past the pipeline's LDS stages
-  bf16_t* const scratch = smem + gemm_lds_elems<BN, AK, BK, NST>();
 
-  const int tid = threadIdx.x, l = tid & 63, w = tid >> 6;
+  const int l = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // the same for the whole wave: scalar LDS bases
   const int wm = w >> 1, wn = w & 1;
 
   int tm, t0, t1, split;
@@ -826,134 +816,142 @@ __device__ __forceinline__ void gemm_body(const GemmShape& g_in, const typename 
 
   typename Epi::State st;
   Epi::init(ep, st, g, tm, wm, l);
-  WaveAcc<BN, W> acc;
+  WaveAcc<BN> acc;
 
   const int KT = (g.K + kBK - 1) / kBK;
-  const int a_r0 = tm * kBM;
-  // Direct-to-LDS pipeline over the workgroup's slabs s = 0, 1, ... (a run
-  // of column tiles times KT slabs each), LDS stage s & 1.  Per slab:
-  //   k-steps 0..2: MFMAs, with the fragments of the next k-step read
-  //                 from LDS behind them;
-  //   barrier B_s:  its implied vmcnt(0) / lgkmcnt(0) mean slab s+1's DMA
-  //                 (issued after B_{s-1}) has landed for every wave and no
-  //                 wave still reads slab s's stage;
-  //   then the DMA of slab s+2 into that stage and the first fragments of
-  //   slab s+1 are issued while the MFMAs of k-step 3 (whose fragments are
-  //   already in registers) run, so the barrier's read bubble is hidden.
-  constexpr int kStA = tile_elems<AK, kBM>(), kSt = kStA + tile_elems<BK, BN>();  // elements of a stage
-  static_assert(NST >= 2 && NST <= 3, "LDS holds two or three stages");
-  // DMA wave instructions per wave per slab
-  constexpr int kD = (kBM + BN) / (8 * W);
-  auto frags = [&](const bf16_t* Sc, int kk, Frags<BN, W>& f) {
-    read_op<AK, kBM>(Sc, kk, wm * WaveCfg<W>::kWaveRows, f.a, l);
-    read_op<BK, BN>(Sc + kStA, kk, wn * (BN / 2), f.b, l);
-  };
-  // DMA of the next unissued slab (tile it2, k-slab ik2) into stage S
-  int it2 = t0, ik2 = 0;
-  // A through a row map: its lane offsets are computed once per workgroup
-  static_assert((AK && BK) || !(AROW || KTAIL), "the row map and the K tail are for K-major operands");
-  static_assert(!(AROW && KTAIL), "a row-mapped A has whole slabs");
-  ARows<W> arows;
-  if constexpr (AROW) arows.init(g.A, g.lda, a_r0, g.M, g.arow, g.arows, w, l);
-  auto issue = [&](bf16_t* S) {
-    if constexpr (AROW)
-      arows.dma(ik2 * kBK, S, w);
-    else if constexpr (AK)
-      dma_kmajor<kBM, W, KTAIL>(g.A, g.lda, a_r0, g.M, ik2 * kBK, g.K, S, w, l);
-    else
-      dma_mnmajor<kBM, W>(g.A, g.lda, a_r0, ik2 * kBK, g.K, S, w, l);
-    if constexpr (BK)
-      dma_kmajor<BN, W, KTAIL>(g.B, g.ldb, it2 * BN, g.N, g.kb + ik2 * kBK, g.K, S + kStA, w, l);
-    else
-      dma_mnmajor<BN, W>(g.B, g.ldb, g.b0 + it2 * BN, ik2 * kBK, g.K, S + kStA, w, l);
-    if (++ik2 == KT) {
-      ik2 = 0;
-      ++it2;
+  // slabs of A and of B that are still to be issued; the streams cross the
+  // boundaries of the workgroup's tiles
+  int left_a = (t1 - t0) * KT, left_b = left_a;
+  Stream<AK, kBM, KTAIL, AROW> sa;
+  Stream<BK, BN, KTAIL> sb;
+  int ka = KT, kbt = KT, it = t0;  // slabs left in the tile of the next A / B, B's tile
+  sa.init(g.A, g.lda, tm * kBM, g.M, 0, g.K, g.arow, g.arows, w, l);
+  sb.init(g.B, g.ldb, BK ? t0 * BN : g.b0 + t0 * BN, g.N, g.kb, g.K, nullptr, 0, w, l);
+  auto next_a = [&]() {
+    sa.next();
+    --left_a;
+    if constexpr (!Epi::kOneTile) {
+      if (--ka == 0) {
+        ka = KT;
+        sa.k = 0;
+      }
     }
   };
-  // The DMA's LDS writes count on vmcnt; the barrier's own fence does not
-  // reliably wait for them, so each barrier B_s that publishes slab s+1 is
-  // preceded by an explicit wait.  Vector memory operations retire in
-  // issue order, so B_s may leave in flight exactly what was issued after
-  // slab s+1's DMA: the DMAs of slabs s+2 .. s+NST-1, and the previous
-  // tile's epilogue stores for the first NST-1 slabs of a tile (they then
-  // drain behind the MFMAs).  Near the end of the run, where some of those
-  // DMAs were never issued, it waits for everything.  sched_barrier fences
-  // keep the MFMAs on their side of the barrier.
-  auto publish = [&](int s_, bool after_epilogue) {
+  auto next_b = [&]() {
+    sb.next();
+    --left_b;
+    if constexpr (!Epi::kOneTile) {
+      if (--kbt == 0) {
+        kbt = KT;
+        ++it;
+        sb.k = 0;
+        sb.base = g.B + (long)it * BN * g.ldb;
+        sb.bytes = max((long)g.N - it * BN, 0L) * g.ldb * 2;
+      }
+    }
+  };
+  static_assert(Epi::kOneTile || (AK && BK), "runs of tiles: K-major operands");
+  constexpr int IA = decltype(sa)::kI, IB = decltype(sb)::kI;
+  auto unit = [&](int u) { return smem + (u >= 5 ? u - 5 : u) * kUnit; };
+  auto frags = [&](const bf16_t* Sa, const bf16_t* Sb, int kk, Frags<BN>& f) {
+    read_op<AK, kBM>(Sa, kk, wm * kWaveRows, f.a, l);
+    read_op<BK, BN>(Sb, kk, wn * (BN / 2), f.b, l);
+  };
+  // Order of a k-step: the reads behind the first MFMAs, D DMA instructions
+  // behind the rest.
+  constexpr int kReads = (AK ? 1 : 2) * kFM + (BK ? 1 : 2) * (BN / 64), kMfma = kFM * (BN / 64);
+  auto order = [&](auto D) {
+    constexpr int d = decltype(D)::value, half = kMfma / 2;
+#pragma unroll
+    for (int i = 0; i < half; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      if (i < kReads % half)
+        __builtin_amdgcn_sched_group_barrier(0x100, kReads / half + 1, 0);
+      else
+        __builtin_amdgcn_sched_group_barrier(0x100, kReads / half, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < d; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, half / d, 0);
+      __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+    }
+    acc.pin();
     __builtin_amdgcn_sched_barrier(0);
-    const bool deep = s_ + NST - 1 < ((t1 - t0) * KT);
-    if (deep && Epi::kStores > 0 && after_epilogue)
-      __builtin_amdgcn_s_waitcnt(vmcnt_imm((NST - 2) * kD + Epi::kStores));
-    else if (deep && NST > 2)
-      __builtin_amdgcn_s_waitcnt(vmcnt_imm((NST - 2) * kD));
-    else
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
+    __builtin_amdgcn_s_waitcnt(kWaitLds);  // the fragments read in this k-step
     __builtin_amdgcn_sched_barrier(0);
   };
-  // each k-step: the next k-step's fragment reads are issued first, then
-  // the MFMAs they hide behind
-  auto order = [&]() {
-    constexpr int kReads = (AK ? 1 : 2) * WaveCfg<W>::kFM + (BK ? 1 : 2) * (BN / 64);
-    __builtin_amdgcn_sched_group_barrier(0x100, kReads, 0);
-    __builtin_amdgcn_sched_group_barrier(0x008, WaveCfg<W>::kFM * (BN / 64), 0);
-  };
-  const int total = (t1 - t0) * KT;
-  // prologue: slabs 0 .. NST-1 in flight, wait for slab 0
-  issue(smem);
-  if (total > 1) issue(smem + kSt);
-  if constexpr (NST == 3) {
-    if (total > 2) issue(smem + 2 * kSt);
-  }
-  // wait for slab 0 only: after its DMA come those of slabs 1 .. NST-1
-  // (all issued when total > NST)
+  typedef std::integral_constant<int, IA / 2> DA;
+  typedef std::integral_constant<int, IB / 2> DB;
+
+  // prologue: A(0), B(0), A(1) and half of B(1) in flight, wait for slab 0
   __builtin_amdgcn_sched_barrier(0);
-  if (total > NST)
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NST - 1) * kD) : "memory");
-  else
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  sa.template issue<0, IA>(unit(0), left_a > 0, w);
+  next_a();
+  sb.template issue<0, IB>(unit(1), left_b > 0, w);
+  next_b();
+  sa.template issue<0, IA>(unit(2), left_a > 0, w);
+  next_a();
+  sb.template issue<0, IB / 2>(unit(3), left_b > 0, w);
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(IA + IB / 2) : "memory");
   __syncthreads();
   __builtin_amdgcn_sched_barrier(0);
-  Frags<BN, W> fa, fb;
-  frags(smem, 0, fa);
-  int s = 0, cur = 0;  // cur = s % NST
+  Frags<BN> fa, fb;
+  frags(unit(0), unit(1), 0, fa);
+  __builtin_amdgcn_s_waitcnt(kWaitLds);
+  __builtin_amdgcn_sched_barrier(0);
+  int u = 0;  // ring unit of A(s)
+  auto slab = [&](auto FIRST) {
+    bf16_t *const Sa = unit(u), *const Sb = unit(u + 1), *const Na = unit(u + 2), *const Nb = unit(u + 3),
+                  *const Free = unit(u + 4);
+    frags(Sa, Sb, 1, fb);
+    sb.template issue<IB / 2, IB>(Nb, left_b > 0, w);
+    mfma_frags<BN, decltype(FIRST)::value>(fa, acc);
+    order(DB{});
+    next_b();
+    frags(Sa, Sb, 2, fa);
+    sa.template issue<0, IA / 2>(Free, left_a > 0, w);
+    mfma_frags<BN, false>(fb, acc);
+    order(DA{});
+    frags(Sa, Sb, 3, fb);
+    sa.template issue<IA / 2, IA>(Free, left_a > 0, w);
+    mfma_frags<BN, false>(fa, acc);
+    order(DA{});
+    next_a();
+    // The DMA's LDS writes count on vmcnt; the barrier's own fence does not
+    // reliably wait for them.  Vector memory operations retire in issue
+    // order, so all but the IA newest (A(s+2)'s) have landed.
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(IA) : "memory");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    frags(Na, Nb, 0, fa);
+    sb.template issue<0, IB / 2>(Sa, left_b > 0, w);
+    mfma_frags<BN, false>(fb, acc);
+    order(DB{});
+    u = u >= 3 ? u - 3 : u + 2;
+  };
   for (int tn = t0; tn < t1; ++tn) {
-    acc.zero();
-    for (int kt = 0; kt < KT; ++kt, ++s) {
-      const int nxt = (cur + 1 == NST) ? 0 : cur + 1;
-      bf16_t* const Sc = smem + cur * kSt;
-      bf16_t* const Sn = smem + nxt * kSt;
-      frags(Sc, 1, fb);
-      mfma_frags<BN, W>(fa, acc);
-      order();
-      frags(Sc, 2, fa);
-      mfma_frags<BN, W>(fb, acc);
-      order();
-      frags(Sc, 3, fb);
-      mfma_frags<BN, W>(fa, acc);
-      order();
-      publish(s, kt <= NST - 2 && tn != t0);  // B_s
-      // the next tile's first fragments are read after this tile's
-      // epilogue, so they are not live (24 VGPRs) while it runs
-      if (kt + 1 < KT) frags(Sn, 0, fa);
-      mfma_frags<BN, W>(fb, acc);
-      order();
-      __builtin_amdgcn_sched_barrier(0);
-      if (s + NST < total) issue(Sc);  // stage of slab s is free after B_s
-      cur = nxt;
+    slab(std::true_type{});
+    for (int kt = 1; kt < KT; ++kt) slab(std::false_type{});
+    if constexpr (Epi::kOneTile) {
+      // the ring is free for the epilogue once the stream's last writes landed
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
     }
-    Epi::tile(ep, st, acc, g, tm, tn, wm, wn, l, scratch);
-    if (tn + 1 < t1) frags(smem + cur * kSt, 0, fa);  // slab s+1, published at B_s
+    Epi::tile(ep, st, acc, g, tm, tn, wm, wn, l, smem);
+  }
+  if constexpr (!Epi::kOneTile) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
   }
   Epi::finish(ep, st, g, tm, split, smem, wm, wn, l);
 }
 
-template <int BN, int W, bool AK, bool BK, template <int, int> class EpiT, int NST = 2, bool AROW = false,
-          bool KTAIL = false>
-__global__ __launch_bounds__(W * 64) void gemm_kernel(GemmShape g, typename EpiT<BN, W>::Params ep) {
-  __shared__ __attribute__((aligned(16))) bf16_t smem[gemm_lds_elems<BN, AK, BK, NST>() + EpiT<BN, W>::kScratch];
-  gemm_body<BN, W, AK, BK, EpiT, NST, AROW, KTAIL>(g, ep, blockIdx.x, gridDim.x, smem);
+template <int BN, bool AK, bool BK, template <int> class EpiT, bool AROW = false, bool KTAIL = false>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_kernel(
+    GemmShape g, typename EpiT<BN>::Params ep) {
+  __shared__ __attribute__((aligned(16))) bf16_t smem[kLdsElems];
+  gemm_body<BN, AK, BK, EpiT, AROW, KTAIL>(g, ep, blockIdx.x, gridDim.x, smem);
 }
 
 // One launch per vocabulary band b of the backward: the
@@ -963,8 +961,7 @@ __global__ __launch_bounds__(W * 64) void gemm_kernel(GemmShape g, typename EpiT
 // on padding, and the wide tiles do the most work per CU-second).
 // Workgroups are numbered longest first — dW (K = N), dH (K = band width),
 // then the short recompute tiles, which fill the CUs the long tiles leave
-// idle at the end of the band.  The 128-wide tail tiles fit three LDS stages
-// (two slabs in flight) in the space the 256-wide tiles use for two.
+// idle at the end of the band.
 // dH reads W's rows as they are (an MN-major B): against a transposed copy of
 // each band's rows the band launch takes the same time at d = 896 and 1.4% less
 // at d = 4096 (8192 rows), and the copies and their memory are gone.  With dH split over K on very
@@ -1043,7 +1040,7 @@ struct BandLaunch {
 };
 
 // One split workgroup of a K-split dH population (see BandLaunch).
-template <int BN, int NST>
+template <int BN>
 __device__ inline void dh_split_body(const GemmShape& g0, const AccParams& e0, int ks, int kc, long stride, int b,
                                      int nb, bf16_t* smem) {
   const int k = b % ks, k0 = k * kc;
@@ -1053,53 +1050,50 @@ __device__ inline void dh_split_body(const GemmShape& g0, const AccParams& e0, i
   g.B += k0 * g.ldb;
   g.K = min(kc, g0.K - k0);
   e.acc32 += k * stride;
-  gemm_body<BN, kWarp8, true, false, EpiAcc, NST>(g, e, b / ks, nb / ks, smem);
+  gemm_body<BN, true, false, EpiAcc>(g, e, b / ks, nb / ks, smem);
 }
 
 // HB: with a bias.  AROW: the recompute reads H's rows through the row order.
 // KTAIL: d is no multiple of 64 (the recompute's K).
 template <bool HB, bool AROW, bool KTAIL>
-__global__ __launch_bounds__(kWarp8 * 64) void band_kernel(BandLaunch p) {
-  __shared__ __attribute__((aligned(16))) bf16_t smem[gemm_lds_elems<kBN, true, true>() + EpiGrad<kBN, kWarp8>::kScratch];
-  static_assert(sizeof(smem) >= 2 * gemm_lds_elems<kBN, false, true>() && sizeof(smem) >= 2 * gemm_lds_elems<kBN, true, false>() &&
-                sizeof(smem) >= 2 * gemm_lds_elems<kTailBN, false, true, 3>() &&
-                sizeof(smem) >= 2 * gemm_lds_elems<kTailBN, true, false, 3>(), "every population's stages fit");
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))) void band_kernel(BandLaunch p) {
+  __shared__ __attribute__((aligned(16))) bf16_t smem[kLdsElems];
   int b = blockIdx.x;
   if (b < p.nb_dw) {
-    gemm_body<kBN, kWarp8, false, true, EpiAcc>(p.dw, p.e_dw, b, p.nb_dw, smem);
+    gemm_body<kBN, false, true, EpiAcc>(p.dw, p.e_dw, b, p.nb_dw, smem);
     return;
   }
   b -= p.nb_dw;
   if (b < p.nb_dw2) {
-    gemm_body<kTailBN, kWarp8, false, true, EpiAcc, 3>(p.dw2, p.e_dw2, b, p.nb_dw2, smem);
+    gemm_body<kTailBN, false, true, EpiAcc>(p.dw2, p.e_dw2, b, p.nb_dw2, smem);
     return;
   }
   b -= p.nb_dw2;
   if (b < p.nb_dh) {
     if (p.dh_split)
-      dh_split_body<kBN, 2>(p.dh, p.e_dh_part, p.dh_ks, p.dh_kc, p.dh_part_stride, b, p.nb_dh, smem);
+      dh_split_body<kBN>(p.dh, p.e_dh_part, p.dh_ks, p.dh_kc, p.dh_part_stride, b, p.nb_dh, smem);
     else
-      gemm_body<kBN, kWarp8, true, false, EpiAcc>(p.dh, p.e_dh, b, p.nb_dh, smem);
+      gemm_body<kBN, true, false, EpiAcc>(p.dh, p.e_dh, b, p.nb_dh, smem);
     return;
   }
   b -= p.nb_dh;
   if (b < p.nb_dh2) {
     if (p.dh_split)
-      dh_split_body<kTailBN, 3>(p.dh2, p.e_dh2_part, p.dh_ks, p.dh_kc, p.dh_part_stride, b, p.nb_dh2, smem);
+      dh_split_body<kTailBN>(p.dh2, p.e_dh2_part, p.dh_ks, p.dh_kc, p.dh_part_stride, b, p.nb_dh2, smem);
     else
-      gemm_body<kTailBN, kWarp8, true, false, EpiAcc, 3>(p.dh2, p.e_dh2, b, p.nb_dh2, smem);
+      gemm_body<kTailBN, true, false, EpiAcc>(p.dh2, p.e_dh2, b, p.nb_dh2, smem);
     return;
   }
   b -= p.nb_dh2;
   if (b < p.nb_gr) {
     if constexpr (HB)
-      gemm_body<kBN, kWarp8, true, true, EpiGradBiasTile, 2, AROW, KTAIL>(p.gr, p.e_gr, b, p.nb_gr, smem);
+      gemm_body<kBN, true, true, EpiGradBias, AROW, KTAIL>(p.gr, p.e_gr, b, p.nb_gr, smem);
     else
-      gemm_body<kBN, kWarp8, true, true, EpiGradTile, 2, AROW, KTAIL>(p.gr, p.e_gr, b, p.nb_gr, smem);
+      gemm_body<kBN, true, true, EpiGrad, AROW, KTAIL>(p.gr, p.e_gr, b, p.nb_gr, smem);
     return;
   }
   b -= p.nb_gr;
-  dh_reduce_body(p.red, b * (long)(kWarp8 * 64) + threadIdx.x, (long)p.nb_red * (kWarp8 * 64));
+  dh_reduce_body(p.red, b * (long)kThreads + threadIdx.x, (long)p.nb_red * kThreads);
 }
 
 // ---------------------------------------------------------------------------
@@ -2252,15 +2246,15 @@ double gemm_flops(long M, long N, long K) { return 2.0 * (double)M * (double)N *
 
 // A GEMM launch; `credited` is the algorithmic share of its FLOPs (the
 // logits recompute of the backward is executed but not credited).
-template <int BN, int W, template <int, int> class EpiT, bool AROW = false, bool KTAIL = false>
-int launch_gemm(const GemmShape& g, const typename EpiT<BN, W>::Params& ep, int nblocks, hipStream_t st,
+template <int BN, template <int> class EpiT, bool AROW = false, bool KTAIL = false>
+int launch_gemm(const GemmShape& g, const typename EpiT<BN>::Params& ep, int nblocks, hipStream_t st,
                 int kind, bool credited) {
   if (nblocks <= 0) return CCE_OK;
   const int rc = check_operands(g, true, true, KTAIL);
   if (rc) return rc;
   hipEvent_t e0 = nullptr, e1 = nullptr;
   const bool timed = timing_begin(st, &e0, &e1);
-  hipLaunchKernelGGL((gemm_kernel<BN, W, true, true, EpiT, 2, AROW, KTAIL>), dim3(nblocks), dim3(W * 64), 0, st, g, ep);
+  hipLaunchKernelGGL((gemm_kernel<BN, true, true, EpiT, AROW, KTAIL>), dim3(nblocks), dim3(kThreads), 0, st, g, ep);
   HIP_TRY(hipGetLastError());
   if (timed) {
     const double f = gemm_flops(g.M, g.N, g.K);
@@ -2284,14 +2278,10 @@ int zero_fill(void* p, size_t bytes, hipStream_t st) {
 
 // Recompute launch shape of one unit: G[n][c] for the rows [m0, m0 + rows)
 // of the compacted order (a row block) and columns [v0, v0 + vb).
-// A recompute launch of its own runs one round of workgroups, about one per
-// CU, each over a run of column tiles: the pipeline runs on across a run, so
-// a tile's epilogue overlaps the next tile's first loads, and no partly filled
-// last round is left.  Inside the band launch (`in_band`) each workgroup
-// takes one tile, the finest grain for filling the CUs that the long dW / dH
-// tiles leave idle.
+// Each workgroup takes one tile, the finest grain for filling the CUs that the
+// long dW / dH tiles of a band launch leave idle.
 void grad_shape(const bf16_t* H, const bf16_t* W, const float* bias, const BwdLayout& L, bf16_t* G, long m0,
-                long rows, long d, long v0, long vb, int bn, bool in_band, GemmShape& g, GradParams& e, int& nb) {
+                long rows, long d, long v0, long vb, GemmShape& g, GradParams& e, int& nb) {
   const int gm = (int)ceil_div(rows, kBM);
   if (L.Hc || !L.idx) {
     g.A = (L.Hc ? L.Hc : H) + m0 * d;
@@ -2304,9 +2294,8 @@ void grad_shape(const bf16_t* H, const bf16_t* W, const float* bias, const BwdLa
   g.M = (int)rows; g.N = (int)vb; g.K = (int)d;
   g.live = L.live; g.dyn = L.live ? kDynM : kDynNone; g.live_base = (int)m0;
   e.bias = bias; e.rowp = L.rowp + m0; e.rowlab = L.rowlab + m0; e.G = G; e.ldg = L.Vb; e.v0 = (int)v0;
-  e.tiles_n = (int)ceil_div(vb, bn);
-  e.splits = in_band ? e.tiles_n : (int)std::min<long>(e.tiles_n, std::max<long>(1, ceil_div(device_cus(), gm)));
-  nb = gm * e.splits;
+  e.tiles_n = (int)ceil_div(vb, kBN);
+  nb = gm * e.tiles_n;
 }
 
 int launch_band(const BandLaunch& p, bool has_bias, hipStream_t st, int kind = CCE_KERNEL_BWD_BAND) {
@@ -2326,7 +2315,7 @@ int launch_band(const BandLaunch& p, bool has_bias, hipStream_t st, int kind = C
   auto* const kernel = ktail ? (has_bias ? band_kernel<true, false, true> : band_kernel<false, false, true>)
                        : arow ? (has_bias ? band_kernel<true, true, false> : band_kernel<false, true, false>)
                               : (has_bias ? band_kernel<true, false, false> : band_kernel<false, false, false>);
-  hipLaunchKernelGGL(kernel, dim3(nb), dim3(kWarp8 * 64), 0, st, p);
+  hipLaunchKernelGGL(kernel, dim3(nb), dim3(kThreads), 0, st, p);
   HIP_TRY(hipGetLastError());
   if (timed) {
     double cr = 0.0;
@@ -2448,14 +2437,14 @@ int forward_run(const void* hidden, const void* weight, const void* labels, int 
   ep.tiles_n = (int)ceil_div(V, kBN);
   constexpr int kKind = CCE_KERNEL_FWD_LSE;
   if (!whole_slabs(d))
-    rc = bias ? launch_gemm<kBN, kWarp8, EpiLseBias, false, true>(g, ep, slots, st, kKind, true)
-              : launch_gemm<kBN, kWarp8, EpiLse, false, true>(g, ep, slots, st, kKind, true);
+    rc = bias ? launch_gemm<kBN, EpiLseBias, false, true>(g, ep, slots, st, kKind, true)
+              : launch_gemm<kBN, EpiLse, false, true>(g, ep, slots, st, kKind, true);
   else if (g.arow)
-    rc = bias ? launch_gemm<kBN, kWarp8, EpiLseBias, true>(g, ep, slots, st, kKind, true)
-              : launch_gemm<kBN, kWarp8, EpiLse, true>(g, ep, slots, st, kKind, true);
+    rc = bias ? launch_gemm<kBN, EpiLseBias, true>(g, ep, slots, st, kKind, true)
+              : launch_gemm<kBN, EpiLse, true>(g, ep, slots, st, kKind, true);
   else
-    rc = bias ? launch_gemm<kBN, kWarp8, EpiLseBias>(g, ep, slots, st, kKind, true)
-              : launch_gemm<kBN, kWarp8, EpiLse>(g, ep, slots, st, kKind, true);
+    rc = bias ? launch_gemm<kBN, EpiLseBias>(g, ep, slots, st, kKind, true)
+              : launch_gemm<kBN, EpiLse>(g, ep, slots, st, kKind, true);
   if (rc) return rc;
 
   const bool uniform = smoothing_form == CCE_SMOOTH_UNIFORM && label_smoothing > 0.f;
@@ -2754,36 +2743,20 @@ int cce_backward(const float* grad_out, const void* hidden, const void* weight, 
     HIP_TRY(hipGetLastError());
     return CCE_OK;
   };
-  auto grad_unit = [&](long u, bool in_band, int bn, GemmShape& g, GradParams& e, int& nb) {
+  auto grad_unit = [&](long u, GemmShape& g, GradParams& e, int& nb) {
     long v0, vb, m0, rows;
     band_cols(u / R, v0, vb);
     block_span(u % R, m0, rows);
-    grad_shape(H, W, bias, L, L.G[u & 1], m0, rows, d, v0, vb, bn, in_band, g, e, nb);
+    grad_shape(H, W, bias, L, L.G[u & 1], m0, rows, d, v0, vb, g, e, nb);
   };
 
   // launch u: dW and dH of unit u from G[u & 1] and the recompute of unit
   // u+1 into G[(u+1) & 1]; unit 0's recompute runs alone first.
   const long dmain = band_dmain(d);
-  {
-    GemmShape g1 = {};
-    GradParams e1 = {};
-    int nb1 = 0;
-    const bool in_band = (L.idx && !L.Hc) || !whole_slabs(d);
-    grad_unit(0, in_band, kBN, g1, e1, nb1);
-    if (in_band) {
-      // reading H through the row order, or d no multiple of 64: a band launch
-      // with only this recompute population (the stand-alone GEMM kernel's
-      // column runs with the row map spill registers)
-      BandLaunch p0 = {};
-      p0.gr = g1;
-      p0.e_gr = e1;
-      p0.nb_gr = nb1;
-      rc = launch_band(p0, bias != nullptr, st, CCE_KERNEL_BWD_GRAD);
-    } else
-      rc = bias ? launch_gemm<kBN, kWarp8, EpiGradBias>(g1, e1, nb1, st, CCE_KERNEL_BWD_GRAD, false)
-                : launch_gemm<kBN, kWarp8, EpiGrad>(g1, e1, nb1, st, CCE_KERNEL_BWD_GRAD, false);
-    if (rc) return rc;
-  }
+  BandLaunch first = {};
+  grad_unit(0, first.gr, first.e_gr, first.nb_gr);
+  rc = launch_band(first, bias != nullptr, st, CCE_KERNEL_BWD_GRAD);
+  if (rc) return rc;
   // With 4 or more splits (very few rows) the band launches are short and the
   // reduction rides in the next launch, so the partials alternate between
   // two buffers; with 2-3 splits the launches are full and it runs as a
@@ -2859,11 +2832,11 @@ int cce_backward(const float* grad_out, const void* hidden, const void* weight, 
         p.red = dh_reduction(u - 1, prev_ks);
         long pm0, prows;
         block_span((u - 1) % R, pm0, prows);
-        p.nb_red = (int)std::min<long>(ceil_div(prows * (d / 4), kWarp8 * 64 * 4), 1024);
+        p.nb_red = (int)std::min<long>(ceil_div(prows * (d / 4), kThreads * 4), 1024);
       }
       prev_ks = ks;
     }
-    if (u + 1 < units) grad_unit(u + 1, true, kBN, p.gr, p.e_gr, p.nb_gr);
+    if (u + 1 < units) grad_unit(u + 1, p.gr, p.e_gr, p.nb_gr);
     rc = launch_band(p, bias != nullptr, st);
     if (rc) return rc;
     if (need_dh && L.dhpart && (!fold || u + 1 == units)) {

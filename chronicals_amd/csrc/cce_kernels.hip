@@ -191,6 +191,8 @@ __device__ inline int acc_col(int wn, int j, int q, int l) {
 // stay live next to the accumulators.
 __device__ inline void pin_epilogue(int& l, int& tm, int& tn) {
   asm volatile("" : "+v"(l));
+  tm = __builtin_amdgcn_readfirstlane(tm);  // the same for the whole workgroup
+  tn = __builtin_amdgcn_readfirstlane(tn);
   asm volatile("" : "+s"(tm), "+s"(tn));
 }
 
@@ -415,7 +417,7 @@ struct EpiLseT {
       st.s[i] = 0.f;
     }
   }
-  static __device__ inline void tile(const Params& p, State& st, WaveAcc<BN>& acc, const GemmShape& g, int tm,
+  static __device__ __forceinline__ void tile(const Params& p, State& st, WaveAcc<BN>& acc, const GemmShape& g, int tm,
                                      int tn, int wm, int wn, int l, bf16_t*) {
     constexpr int FN = BN / 64;
     pin_epilogue(l, tm, tn);
@@ -562,7 +564,7 @@ struct EpiGradT {
       for (int i = 0; i < FM; ++i) row_params(p, g, tm * kBM + acc_row(wm, i, l), st.rp[i], st.lab[i]);
     }
   }
-  static __device__ inline void tile(const Params& p, State& st, WaveAcc<BN>& acc, const GemmShape& g, int tm,
+  static __device__ __forceinline__ void tile(const Params& p, State& st, WaveAcc<BN>& acc, const GemmShape& g, int tm,
                                      int tn, int wm, int wn, int l, bf16_t* scratch) {
     constexpr int FN = BN / 64;
     static_assert(FN % 2 == 0, "64-column staging blocks");
@@ -575,10 +577,10 @@ struct EpiGradT {
     // interior tile without bias: every column is inside the band and rows
     // past M are dropped by the store descriptor, so no per-element checks
     const bool interior = !HB && (tn + 1) * BN <= g.N;
+    const __amdgpu_buffer_rsrc_t bias = make_rsrc(p.bias + p.v0, HB ? (long)g.N * 4 : 0L);
 #pragma unroll
     for (int i = 0; i < FM; ++i) {
       const int m = tm * kBM + acc_row(wm, i, l);
-      const bool mok = m < g.M;
       float4 rp;
       int lab;
       if constexpr (HB) {
@@ -615,16 +617,14 @@ struct EpiGradT {
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
               const int cb = tn * BN + acc_col<BN>(wn, 2 * jp + jj, q, l);
+              f32x4 b = {0.f, 0.f, 0.f, 0.f};
+              if constexpr (HB) b = load4(bias, cb * 4);
               float gv[4];
 #pragma unroll
               for (int e = 0; e < 4; ++e) {
-                const int col = cb + e;
-                float gg = 0.f;
-                if (mok && col < g.N) {
-                  const float b = HB ? p.bias[p.v0 + col] : 0.f;
-                  gg = rp.y * fast_exp2((x[jj][4 * q + e] + b) * kLog2e - rp.x) - rp.w;
-                }
-                gv[e] = gg;
+                const float gg =
+                    __builtin_fmaf(rp.y, fast_exp2(__builtin_fmaf(x[jj][4 * q + e] + b[e], kLog2e, -rp.x)), -rp.w);
+                gv[e] = cb + e < g.N ? gg : 0.f;
               }
               stage(jj, q, gv);
             }
@@ -696,58 +696,82 @@ struct EpiAcc {
     split = 0;
   }
   static __device__ inline void init(const Params&, State&, const GemmShape&, int, int, int) {}
-  static __device__ inline void tile(const Params& p, State&, WaveAcc<BN>& acc, const GemmShape& g, int tm,
-                                     int tn, int wm, int wn, int l, bf16_t*) {
-    constexpr int FN = BN / 64;
-    constexpr int JG = FN >= 2 ? 2 : 1;  // 32 x 64 column blocks whose old values load together
-    pin_epilogue(l, tm, tn);
+  // A lane holds one row, so a direct store would touch 32 rows with 16 bytes
+  // each.  Each wave stages 32 rows in its part of the ring (rows padded by 16
+  // bytes: the 16 lanes of a write phase hit distinct banks) and goes over them
+  // in whole rows of its columns, 512 or 256 bytes of fp32.
+  static constexpr int kC = BN / 2;          // columns of a wave tile
+  static constexpr int kL = kC / 4;          // lanes per row
+  static constexpr int kPitch = kC + 4;
+  template <int I, bool FULL>
+  static __device__ __forceinline__ void rows32(const Params& p, WaveAcc<BN>& acc, const GemmShape& g, int m0, int n0,
+                                                int l, float* ws) {
+    constexpr int kR = 64 / kL, kT = 32 / kR;  // rows per instruction, instructions
+    const int rr = l / kL, c = (l % kL) * 4;
+    const bool nok = FULL || n0 + c < g.N;
+    long om[kT];
+    f32x4 old[kT];
 #pragma unroll
-    for (int i = 0; i < FM; ++i) {
-      const int m = tm * kBM + acc_row(wm, i, l);
-      if (m >= g.M) continue;
+    for (int t = 0; t < kT; ++t) {
+      const int m = m0 + t * kR + rr;
+      om[t] = p.rowmap && (FULL || m < g.M) ? (long)p.rowmap[m] : (long)m;
+    }
+    // the accumulator's old values: modes 2, 3 from its row m, mode 4 from the output row
+    if (p.mode >= 2) {
 #pragma unroll
-      for (int j0 = 0; j0 < FN; j0 += JG) {
-        // the accumulator's old values for JG column blocks, all loads issued
-        // before any add or store (one memory round trip per group, not per
-        // 16-byte piece)
-        f32x4 old[JG][4];
-        const long om = p.rowmap ? (long)p.rowmap[m] : (long)m;
-        if (p.mode >= 2) {
-          // modes 2, 3 read the accumulator row m; mode 4 the output row om
-          const float* src = p.mode == 4 ? reinterpret_cast<const float*>(p.out) + om * p.ldo
-                                         : p.acc32 + (long)m * p.ldacc;
-#pragma unroll
-          for (int jj = 0; jj < JG; ++jj)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              const int n = tn * BN + acc_col<BN>(wn, j0 + jj, q, l);
-              old[jj][q] = n < g.N ? *reinterpret_cast<const f32x4*>(src + n) : f32x4{0.f, 0.f, 0.f, 0.f};
-            }
-        }
-#pragma unroll
-        for (int jj = 0; jj < JG; ++jj) {
-        const f32x16 x = acc.take(i, j0 + jj);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int j = j0 + jj;
-          const int n = tn * BN + acc_col<BN>(wn, j, q, l);
-          if (n >= g.N) continue;
-          f32x4 v = {x[4 * q], x[4 * q + 1], x[4 * q + 2], x[4 * q + 3]};
-          if (p.mode >= 2) v += old[jj][q];
-          if (p.mode == 1 || p.mode == 2) {
-            *reinterpret_cast<f32x4*>(p.acc32 + (long)m * p.ldacc + n) = v;
-          } else {
-            if (p.out_f32) {
-              *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(p.out) + om * p.ldo + n) = v;
-            } else {
-              const u32x2 pk = {pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
-              *reinterpret_cast<u32x2*>(reinterpret_cast<bf16_t*>(p.out) + om * p.ldo + n) = pk;
-            }
-          }
-        }
-        }
+      for (int t = 0; t < kT; ++t) {
+        const int m = m0 + t * kR + rr;
+        const float* src = p.mode == 4 ? reinterpret_cast<const float*>(p.out) + om[t] * p.ldo
+                                       : p.acc32 + (long)m * p.ldacc;
+        old[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (FULL || (nok && m < g.M)) old[t] = *reinterpret_cast<const f32x4*>(src + n0 + c);
       }
     }
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int j = 0; j < BN / 64; ++j) {
+      const f32x16 x = acc.take(I, j);
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        *reinterpret_cast<f32x4*>(ws + (l & 31) * kPitch + j * 32 + q * 8 + (l >> 5) * 4) =
+            f32x4{x[4 * q], x[4 * q + 1], x[4 * q + 2], x[4 * q + 3]};
+    }
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int t = 0; t < kT; ++t) {
+      const int row = t * kR + rr, m = m0 + row;
+      f32x4 v = *reinterpret_cast<const f32x4*>(ws + row * kPitch + c);
+      if (p.mode >= 2) v += old[t];
+      if (!FULL && !(nok && m < g.M)) continue;
+      if (p.mode == 1 || p.mode == 2) {
+        *reinterpret_cast<f32x4*>(p.acc32 + (long)m * p.ldacc + n0 + c) = v;
+      } else if (p.out_f32) {
+        *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(p.out) + om[t] * p.ldo + n0 + c) = v;
+      } else {
+        *reinterpret_cast<u32x2*>(reinterpret_cast<bf16_t*>(p.out) + om[t] * p.ldo + n0 + c) =
+            u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+      }
+    }
+    asm volatile("" ::: "memory");
+  }
+  static __device__ __forceinline__ void tile(const Params& p, State&, WaveAcc<BN>& acc, const GemmShape& g, int tm,
+                                     int tn, int wm, int wn, int l, bf16_t* scratch) {
+    pin_epilogue(l, tm, tn);
+    float* const ws = reinterpret_cast<float*>(scratch) + (wm * 2 + wn) * 32 * kPitch;
+    const int n0 = tn * BN + wn * kC;
+    auto block = [&](auto I) __attribute__((always_inline)) {
+      constexpr int i = decltype(I)::value;
+      const int m0 = tm * kBM + acc_row(wm, i, 0);
+      if (m0 + 32 <= g.M && n0 + kC <= g.N)
+        rows32<i, true>(p, acc, g, m0, n0, l, ws);
+      else if (m0 < g.M)
+        rows32<i, false>(p, acc, g, m0, n0, l, ws);
+    };
+    static_assert(FM == 4, "four row blocks");
+    block(std::integral_constant<int, 0>{});
+    block(std::integral_constant<int, 1>{});
+    block(std::integral_constant<int, 2>{});
+    block(std::integral_constant<int, 3>{});
   }
   static __device__ inline void finish(const Params&, State&, const GemmShape&, int, int, bf16_t*, int, int,
                                        int) {}

@@ -1,8 +1,12 @@
-"""Build libchronicals_cce.so (HIP, gfx950) in-tree with hipcc.
+"""Build libchronicals_cce.so (HIP, gfx950) and the torch operators over it in-tree.
 
-The library is compiled from ``chronicals_amd/csrc/cce_kernels.hip`` into
-``chronicals_amd/lib/libchronicals_cce.so``; the package loads it from there
-with ctypes.  Building always recompiles.
+The library is compiled with hipcc from ``chronicals_amd/csrc/cce_kernels.hip``
+into ``chronicals_amd/lib/libchronicals_cce.so``; the package loads it from
+there with ctypes.  The torch operators (``csrc/torch_ops.cpp``, host code only)
+are compiled against the installed torch into
+``lib/libchronicals_torch-<hash>.so``, where the hash covers their source, the
+header and torch's version: a build of anything else has another name and is
+never loaded.  Building always recompiles both.
 """
 from __future__ import annotations
 
@@ -16,6 +20,7 @@ PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 REPO_DIR = os.path.dirname(PKG_DIR)
 SRC = os.path.join(PKG_DIR, "csrc", "cce_kernels.hip")
 HEADER = os.path.join(REPO_DIR, "include", "chronicals_cce.h")
+TORCH_SRC = os.path.join(PKG_DIR, "csrc", "torch_ops.cpp")
 LIB_DIR = os.path.join(PKG_DIR, "lib")
 LIB_NAME = "libchronicals_cce.so"
 LIB_PATH = os.path.join(LIB_DIR, LIB_NAME)
@@ -63,6 +68,51 @@ def compile_command(out_path: str, src_hash: str = None) -> list:
     ]
 
 
+def torch_lib_path() -> str:
+    """Where the torch operators of this tree and this torch are built."""
+    import torch
+
+    h = hashlib.sha256((source_hash((TORCH_SRC, HEADER)) + torch.__version__).encode()).hexdigest()
+    return os.path.join(LIB_DIR, f"libchronicals_torch-{h[:16]}.so")
+
+
+def torch_compile_command(out_path: str) -> list:
+    import torch
+
+    base = os.path.join(os.path.dirname(torch.__file__))
+    inc, lib = os.path.join(base, "include"), os.path.join(base, "lib")
+    rocm = os.path.dirname(os.path.dirname(os.path.realpath(hipcc_path())))
+    return [
+        shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared",
+        # what torch's ROCm headers ask of their users
+        "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+        f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+        "-isystem", inc, "-isystem", os.path.join(inc, "torch", "csrc", "api", "include"),
+        "-isystem", os.path.join(rocm, "include"),
+        TORCH_SRC, "-o", out_path,
+        "-L", lib, "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch", f"-Wl,-rpath,{lib}",
+    ]
+
+
+def build_torch(verbose: bool = False) -> str:
+    """Compile the torch operators; returns the path of the built .so and removes builds of other sources."""
+    os.makedirs(LIB_DIR, exist_ok=True)
+    path = torch_lib_path()
+    tmp = path + f".tmp{os.getpid()}"
+    cmd = torch_compile_command(tmp)
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        sys.stderr.write(proc.stdout + proc.stderr)
+        raise RuntimeError(f"g++ failed with exit code {proc.returncode}")
+    os.replace(tmp, path)
+    for name in os.listdir(LIB_DIR):
+        if name.startswith("libchronicals_torch-") and name.endswith(".so") and name != os.path.basename(path):
+            os.remove(os.path.join(LIB_DIR, name))
+    return path
+
+
 def parse_resources(text: str) -> dict:
     """{kernel symbol: {field: int}} from kernel-resource-usage remarks."""
     out, cur = {}, None
@@ -83,7 +133,8 @@ def parse_resources(text: str) -> dict:
 
 
 def build(verbose: bool = False) -> str:
-    """Compile the HIP library; returns the path of the built .so."""
+    """Compile the HIP library and the torch operators; returns the path of the HIP library."""
+    build_torch(verbose)
     os.makedirs(LIB_DIR, exist_ok=True)
     tmp = LIB_PATH + f".tmp{os.getpid()}"
     cmd = compile_command(tmp, source_hash())

@@ -1,7 +1,10 @@
 """torch.library registration of the fused linear-CE entry points.
 
-Custom operators wrap the C ABI (include/chronicals_cce.h) so the path is
-visible to the PyTorch dispatcher and traceable by ``torch.compile``:
+Operators wrap the C ABI (include/chronicals_cce.h) so the path is visible to
+the PyTorch dispatcher and traceable by ``torch.compile``.  Schemas and fake
+(meta) implementations are here; the device kernels are C++
+(csrc/torch_ops.cpp), except those of the two operators that write over their
+logits, which stay Python custom ops:
 
   chronicals_hip::cce_fwd(hidden, weight, labels, bias, ignore_index,
                           label_smoothing, z_loss_weight, smoothing_form,
@@ -28,71 +31,68 @@ touching the device.
 """
 from __future__ import annotations
 
-from typing import Optional, Tuple
+import ctypes
+import os
+from typing import Tuple
 
 import torch
 from torch import Tensor
 
 from . import _lib
+from . import build as _build
 
 __all__ = ["cce_fwd", "cce_bwd", "ce_logits_fwd", "ce_logits_bwd", "ce_logits_bwd_", "ce_logits_fwd_bwd",
            "ce_logits_fwd_bwd_"]
+
+_SCHEMAS = (
+    "cce_fwd(Tensor hidden, Tensor weight, Tensor labels, Tensor? bias, int ignore_index, float label_smoothing, "
+    "float z_loss_weight, int smoothing_form, int reduction, int lse_rows=0) -> (Tensor, Tensor, Tensor, Tensor)",
+    "cce_bwd(Tensor grad_out, Tensor hidden, Tensor weight, Tensor labels, Tensor lse, Tensor n_valid, Tensor? bias, "
+    "int ignore_index, float label_smoothing, float z_loss_weight, int reduction, int chunk_size, bool need_dh, "
+    "bool need_dw, bool need_db, bool dh_f32, bool dw_f32) -> (Tensor, Tensor, Tensor)",
+    "ce_logits_fwd(Tensor logits, Tensor labels, int ignore_index, float label_smoothing, float z_loss_weight, "
+    "int smoothing_form, int reduction) -> (Tensor, Tensor, Tensor)",
+    "ce_logits_bwd(Tensor grad_out, Tensor logits, Tensor labels, Tensor lse, Tensor n_valid, int ignore_index, "
+    "float label_smoothing, float z_loss_weight, int smoothing_form, int reduction, bool f32_grad) -> Tensor",
+    "ce_logits_fwd_bwd(Tensor logits, Tensor labels, int ignore_index, float label_smoothing, float z_loss_weight, "
+    "int smoothing_form, int reduction, bool grad_mean, bool f32_grad) -> (Tensor, Tensor, Tensor, Tensor)",
+)
+_LIBRARY = torch.library.Library("chronicals_hip", "FRAGMENT")
+for _s in _SCHEMAS:
+    _LIBRARY.define(_s)
+
+
+def _load_kernels() -> None:
+    """Load the C++ kernels of the operators and hand them the HIP library's
+    functions.  Without a build the package still imports; calling an operator
+    then raises."""
+    path = _build.torch_lib_path()
+    if not os.path.exists(path):
+        def missing(*args, **kwargs):
+            raise ImportError(f"{path} not found: build it with `python -m chronicals_amd.build` "
+                              f"(or __graft_entry__.build())")
+        for s in _SCHEMAS:
+            _LIBRARY.impl(s.split("(", 1)[0], missing, "CUDA")
+        return
+    torch.ops.load_library(path)
+    try:
+        lib = _lib.load()
+    except ImportError:
+        return  # the operators say so when they are called
+    native = ctypes.CDLL(path)
+    native.chronicals_torch_bind.argtypes = [ctypes.c_void_p]
+    if native.chronicals_torch_bind(lib._handle) != 0:
+        raise ImportError(f"{_lib.lib_path()} lacks functions that {path} needs: rebuild both")
+
+
+_load_kernels()
 
 
 def _stream(device: torch.device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
-def _aligned(t: Tensor) -> Tensor:
-    """The kernels need 16-byte aligned rows: a view at an unaligned storage
-    offset is copied to fresh storage."""
-    return t if t.data_ptr() % 16 == 0 else t.clone()
-
-
-def _check_operands(hidden: Tensor, weight: Tensor, labels: Tensor, bias: Optional[Tensor]) -> None:
-    if hidden.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16:
-        raise RuntimeError(f"cce ops take bf16 hidden and weight, got {hidden.dtype} and {weight.dtype}")
-    if hidden.dim() != 2 or weight.dim() != 2 or hidden.shape[1] != weight.shape[1]:
-        raise RuntimeError(f"cce ops take hidden [N, d] and weight [V, d], got {tuple(hidden.shape)} "
-                           f"and {tuple(weight.shape)}")
-    if labels.dim() != 1 or labels.shape[0] != hidden.shape[0] or labels.dtype not in (torch.int64, torch.int32):
-        raise RuntimeError(f"cce ops take int64/int32 labels [N], got {labels.dtype} {tuple(labels.shape)}")
-    for name, t in (("hidden", hidden), ("weight", weight)):
-        if not t.is_contiguous():
-            raise RuntimeError(f"{name} must be contiguous")
-    if bias is not None and (bias.dtype != torch.float32 or bias.shape != (weight.shape[0],)
-                             or not bias.is_contiguous()):
-        raise RuntimeError("bias must be a contiguous fp32 [V] tensor")
-
-
-@torch.library.custom_op("chronicals_hip::cce_fwd", mutates_args=(), device_types="cuda")
-def cce_fwd(hidden: Tensor, weight: Tensor, labels: Tensor, bias: Optional[Tensor], ignore_index: int,
-            label_smoothing: float, z_loss_weight: float, smoothing_form: int, reduction: int,
-            lse_rows: int = _lib.CCE_LSE_ALL_ROWS) -> Tuple[Tensor, Tensor, Tensor, Tensor]:
-    _check_operands(hidden, weight, labels, bias)
-    hidden, weight = _aligned(hidden), _aligned(weight)
-    lib = _lib.load()
-    device = hidden.device
-    N, d = hidden.shape
-    V = weight.shape[0]
-    with torch.cuda.device(device):
-        ws = torch.empty(_lib.forward_workspace_bytes(N, d, V, reduction, lse_rows), dtype=torch.uint8,
-                         device=device)
-        loss = torch.empty((N,) if reduction == _lib.CCE_REDUCTION_NONE else (1,), dtype=torch.float32,
-                           device=device)
-        lse = torch.empty((N,), dtype=torch.float32, device=device)
-        target = torch.empty((N,), dtype=torch.float32, device=device)
-        n_valid = torch.empty((1,), dtype=torch.int32, device=device)
-        _lib.check(lib.cce_forward(
-            hidden.data_ptr(), weight.data_ptr(), labels.data_ptr(), int(labels.dtype == torch.int64),
-            bias.data_ptr() if bias is not None else None,
-            N, d, V, int(ignore_index), float(label_smoothing), float(z_loss_weight), int(smoothing_form),
-            int(reduction), int(lse_rows), loss.data_ptr(), lse.data_ptr(), target.data_ptr(), n_valid.data_ptr(),
-            ws.data_ptr(), ws.numel(), _stream(device)))
-    return loss, lse, n_valid, target
-
-
-@cce_fwd.register_fake
+@torch.library.register_fake("chronicals_hip::cce_fwd", lib=_LIBRARY)
 def _cce_fwd_fake(hidden, weight, labels, bias, ignore_index, label_smoothing, z_loss_weight, smoothing_form,
                   reduction, lse_rows=_lib.CCE_LSE_ALL_ROWS):
     N = hidden.shape[0]
@@ -101,42 +101,7 @@ def _cce_fwd_fake(hidden, weight, labels, bias, ignore_index, label_smoothing, z
             hidden.new_empty((N,), dtype=torch.float32))
 
 
-@torch.library.custom_op("chronicals_hip::cce_bwd", mutates_args=(), device_types="cuda")
-def cce_bwd(grad_out: Tensor, hidden: Tensor, weight: Tensor, labels: Tensor, lse: Tensor, n_valid: Tensor,
-            bias: Optional[Tensor], ignore_index: int, label_smoothing: float, z_loss_weight: float,
-            reduction: int, chunk_size: int, need_dh: bool, need_dw: bool, need_db: bool, dh_f32: bool,
-            dw_f32: bool) -> Tuple[Tensor, Tensor, Tensor]:
-    _check_operands(hidden, weight, labels, bias)
-    if need_db and bias is None:
-        raise RuntimeError("need_db requires a bias")
-    hidden, weight = _aligned(hidden), _aligned(weight)
-    lib = _lib.load()
-    device = hidden.device
-    N, d = hidden.shape
-    V = weight.shape[0]
-    g = grad_out.detach().to(torch.float32).reshape(-1).contiguous()
-    with torch.cuda.device(device):
-        dh = torch.empty((N, d) if need_dh else (0,), dtype=torch.float32 if dh_f32 else torch.bfloat16,
-                         device=device)
-        dw = torch.empty((V, d) if need_dw else (0,), dtype=torch.float32 if dw_f32 else torch.bfloat16,
-                         device=device)
-        db = torch.empty((V,) if need_db else (0,), dtype=torch.float32, device=device)
-        if need_dh or need_dw or need_db:
-            ws = torch.empty(_lib.backward_workspace_bytes(N, d, V, chunk_size, need_dh, need_dw, dh_f32, dw_f32),
-                             dtype=torch.uint8, device=device)
-            _lib.check(lib.cce_backward(
-                g.data_ptr(), hidden.data_ptr(), weight.data_ptr(), labels.data_ptr(),
-                int(labels.dtype == torch.int64), bias.data_ptr() if bias is not None else None,
-                lse.data_ptr(), n_valid.data_ptr(), N, d, V, int(ignore_index), float(label_smoothing),
-                float(z_loss_weight), int(reduction), int(chunk_size),
-                dh.data_ptr() if need_dh else None, _lib.CCE_DTYPE_F32 if dh_f32 else _lib.CCE_DTYPE_BF16,
-                dw.data_ptr() if need_dw else None, _lib.CCE_DTYPE_F32 if dw_f32 else _lib.CCE_DTYPE_BF16,
-                db.data_ptr() if need_db else None,
-                ws.data_ptr(), ws.numel(), _stream(device)))
-    return dh, dw, db
-
-
-@cce_bwd.register_fake
+@torch.library.register_fake("chronicals_hip::cce_bwd", lib=_LIBRARY)
 def _cce_bwd_fake(grad_out, hidden, weight, labels, lse, n_valid, bias, ignore_index, label_smoothing,
                   z_loss_weight, reduction, chunk_size, need_dh, need_dw, need_db, dh_f32, dw_f32):
     N, d = hidden.shape
@@ -183,28 +148,7 @@ def _row_stride(t: Tensor) -> int:
     return t.stride(0) if t.shape[0] > 1 else t.shape[1]
 
 
-@torch.library.custom_op("chronicals_hip::ce_logits_fwd", mutates_args=(), device_types="cuda")
-def ce_logits_fwd(logits: Tensor, labels: Tensor, ignore_index: int, label_smoothing: float, z_loss_weight: float,
-                  smoothing_form: int, reduction: int) -> Tuple[Tensor, Tensor, Tensor]:
-    _check_logits(logits, labels)
-    lib = _lib.load()
-    device = logits.device
-    N, V = logits.shape
-    with torch.cuda.device(device):
-        ws = torch.empty(_lib.logits_forward_workspace_bytes(N, V, reduction), dtype=torch.uint8, device=device)
-        loss = torch.empty((N,) if reduction == _lib.CCE_REDUCTION_NONE else (1,), dtype=torch.float32,
-                           device=device)
-        lse = torch.empty((N,), dtype=torch.float32, device=device)
-        n_valid = torch.empty((1,), dtype=torch.int32, device=device)
-        _lib.check(lib.cce_logits_forward(
-            logits.data_ptr(), _LOGITS_DTYPES[logits.dtype], _row_stride(logits), labels.data_ptr(),
-            int(labels.dtype == torch.int64), N, V, int(ignore_index), float(label_smoothing), float(z_loss_weight),
-            int(smoothing_form), int(reduction), loss.data_ptr(), lse.data_ptr(), n_valid.data_ptr(), ws.data_ptr(),
-            ws.numel(), _stream(device)))
-    return loss, lse, n_valid
-
-
-@ce_logits_fwd.register_fake
+@torch.library.register_fake("chronicals_hip::ce_logits_fwd", lib=_LIBRARY)
 def _ce_logits_fwd_fake(logits, labels, ignore_index, label_smoothing, z_loss_weight, smoothing_form, reduction):
     N = logits.shape[0]
     loss = logits.new_empty((N,) if reduction == _lib.CCE_REDUCTION_NONE else (1,), dtype=torch.float32)
@@ -229,17 +173,7 @@ def _logits_backward(grad_out: Tensor, logits: Tensor, labels: Tensor, lse: Tens
             _LOGITS_DTYPES[out.dtype], _row_stride(out), _stream(device)))
 
 
-@torch.library.custom_op("chronicals_hip::ce_logits_bwd", mutates_args=(), device_types="cuda")
-def ce_logits_bwd(grad_out: Tensor, logits: Tensor, labels: Tensor, lse: Tensor, n_valid: Tensor, ignore_index: int,
-                  label_smoothing: float, z_loss_weight: float, smoothing_form: int, reduction: int,
-                  f32_grad: bool) -> Tensor:
-    dx = torch.empty(tuple(logits.shape), dtype=torch.float32 if f32_grad else logits.dtype, device=logits.device)
-    _logits_backward(grad_out, logits, labels, lse, n_valid, ignore_index, label_smoothing, z_loss_weight,
-                     smoothing_form, reduction, dx)
-    return dx
-
-
-@ce_logits_bwd.register_fake
+@torch.library.register_fake("chronicals_hip::ce_logits_bwd", lib=_LIBRARY)
 def _ce_logits_bwd_fake(grad_out, logits, labels, lse, n_valid, ignore_index, label_smoothing, z_loss_weight,
                         smoothing_form, reduction, f32_grad):
     return logits.new_empty(tuple(logits.shape), dtype=torch.float32 if f32_grad else logits.dtype)
@@ -291,17 +225,7 @@ def _logits_forward_backward(logits: Tensor, labels: Tensor, ignore_index: int, 
     return loss, lse, n_valid
 
 
-@torch.library.custom_op("chronicals_hip::ce_logits_fwd_bwd", mutates_args=(), device_types="cuda")
-def ce_logits_fwd_bwd(logits: Tensor, labels: Tensor, ignore_index: int, label_smoothing: float, z_loss_weight: float,
-                      smoothing_form: int, reduction: int, grad_mean: bool,
-                      f32_grad: bool) -> Tuple[Tensor, Tensor, Tensor, Tensor]:
-    dx = torch.empty(tuple(logits.shape), dtype=torch.float32 if f32_grad else logits.dtype, device=logits.device)
-    loss, lse, n_valid = _logits_forward_backward(logits, labels, ignore_index, label_smoothing, z_loss_weight,
-                                                  smoothing_form, reduction, grad_mean, dx)
-    return loss, lse, n_valid, dx
-
-
-@ce_logits_fwd_bwd.register_fake
+@torch.library.register_fake("chronicals_hip::ce_logits_fwd_bwd", lib=_LIBRARY)
 def _ce_logits_fwd_bwd_fake(logits, labels, ignore_index, label_smoothing, z_loss_weight, smoothing_form, reduction,
                             grad_mean, f32_grad):
     loss, lse, nv = _ce_logits_fwd_fake(logits, labels, ignore_index, label_smoothing, z_loss_weight, smoothing_form,
@@ -322,3 +246,10 @@ def _ce_logits_fwd_bwd__fake(logits, labels, ignore_index, label_smoothing, z_lo
                              grad_mean):
     return _ce_logits_fwd_fake(logits, labels, ignore_index, label_smoothing, z_loss_weight, smoothing_form,
                                reduction)
+
+
+cce_fwd = torch.ops.chronicals_hip.cce_fwd
+cce_bwd = torch.ops.chronicals_hip.cce_bwd
+ce_logits_fwd = torch.ops.chronicals_hip.ce_logits_fwd
+ce_logits_bwd = torch.ops.chronicals_hip.ce_logits_bwd
+ce_logits_fwd_bwd = torch.ops.chronicals_hip.ce_logits_fwd_bwd

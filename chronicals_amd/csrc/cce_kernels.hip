@@ -156,11 +156,29 @@ struct WaveAcc {
   }
   // Block (i, j) in vector registers, copied here and not earlier (the
   // epilogue holds a few blocks at a time).
-  __device__ inline f32x16 take(int i, int j) {
-    asm volatile("" : "+a"(v[i][j]));
+  __device__ __forceinline__ f32x16 take(int i, int j) const {
+    asm volatile("" ::"a"(v[i][j]));
     f32x16 x = v[i][j];
     asm volatile("" : "+v"(x));
     return x;
+  }
+  // Row block i of an epilogue's loop: one copy of the code that follows
+  // serves the four row blocks (the accumulator registers have no index).
+  __device__ __forceinline__ void take_row(int i, f32x16 (&x)[FN]) const {
+    static_assert(kFM == 4, "four row blocks");
+    if (i == 0) {
+#pragma unroll
+      for (int j = 0; j < FN; ++j) x[j] = take(0, j);
+    } else if (i == 1) {
+#pragma unroll
+      for (int j = 0; j < FN; ++j) x[j] = take(1, j);
+    } else if (i == 2) {
+#pragma unroll
+      for (int j = 0; j < FN; ++j) x[j] = take(2, j);
+    } else {
+#pragma unroll
+      for (int j = 0; j < FN; ++j) x[j] = take(3, j);
+    }
   }
 };
 
@@ -540,12 +558,9 @@ struct EpiGradT {
   static constexpr bool kOneTile = true;  // splits == tiles_n: a workgroup takes one column tile
   static constexpr bool kDynSplits = false;
   static constexpr int FM = kFM;
-  // The per-row parameters are loaded once, before the K loop; with bias they
-  // are loaded in the epilogue beside the bias values.
-  static constexpr int kRows = HB ? 1 : FM;
   struct State {
-    float4 rp[kRows];
-    int lab[kRows];
+    float4 rp;  // of the first row block, loaded before the K loop
+    int lab;
   };
   static __device__ inline void assign(const GemmShape& g, const Params& p, int bid, int nb, int& tm, int& t0,
                                        int& t1, int& split) {
@@ -559,102 +574,100 @@ struct EpiGradT {
     lab = p.rowlab[mc] - p.v0;
   }
   static __device__ inline void init(const Params& p, State& st, const GemmShape& g, int tm, int wm, int l) {
-    if constexpr (!HB) {
-#pragma unroll
-      for (int i = 0; i < FM; ++i) row_params(p, g, tm * kBM + acc_row(wm, i, l), st.rp[i], st.lab[i]);
-    }
+    row_params(p, g, tm * kBM + acc_row(wm, 0, l), st.rp, st.lab);
   }
   static __device__ __forceinline__ void tile(const Params& p, State& st, WaveAcc<BN>& acc, const GemmShape& g, int tm,
                                      int tn, int wm, int wn, int l, bf16_t* scratch) {
     constexpr int FN = BN / 64;
     static_assert(FN % 2 == 0, "64-column staging blocks");
     pin_epilogue(l, tm, tn);
-    bf16_t* const ws = scratch + (wm * 2 + wn) * 2048;
     const int r = l & 31;
     // this row tile of G: rows past M are out of the descriptor's range
     const int rows = min(g.M - tm * kBM, kBM);
     const __amdgpu_buffer_rsrc_t gr = make_rsrc(p.G + (long)tm * kBM * p.ldg, (long)rows * p.ldg * 2);
-    // interior tile without bias: every column is inside the band and rows
-    // past M are dropped by the store descriptor, so no per-element checks
-    const bool interior = !HB && (tn + 1) * BN <= g.N;
     const __amdgpu_buffer_rsrc_t bias = make_rsrc(p.bias + p.v0, HB ? (long)g.N * 4 : 0L);
+    // Row block i is computed and staged in one of two areas, then row block
+    // i - 1 is read back from the other and stored, so that no wave waits for
+    // its own LDS writes.
+    constexpr int kArea = 32 * (BN / 2);  // 32 rows x the wave's columns, in 32 x 64 blocks
+    bf16_t* const ws = scratch + (wm * 2 + wn) * 2 * kArea;
+    const int col0 = tn * BN + wn * (BN / 2);
+    auto stage = [&](int i, float4 rp, int lab, auto INTERIOR) __attribute__((always_inline)) {
+      int lp = l;
+      asm volatile("" : "+v"(lp));  // the columns' masks are not kept from row block to row block
+      f32x16 x[FN];
+      acc.take_row(i, x);
+      bf16_t* const row = ws + (i & 1) * kArea + r * 64;
 #pragma unroll
-    for (int i = 0; i < FM; ++i) {
-      const int m = tm * kBM + acc_row(wm, i, l);
-      float4 rp;
-      int lab;
-      if constexpr (HB) {
-        row_params(p, g, m, rp, lab);
-      } else {
-        rp = st.rp[i];
-        lab = st.lab[i];
-      }
+      for (int j = 0; j < FN; ++j) {
 #pragma unroll
-      for (int jp = 0; jp < FN / 2; ++jp) {
-        const f32x16 x[2] = {acc.take(i, 2 * jp), acc.take(i, 2 * jp + 1)};
-        // G without the one-hot term, packed to bf16 into the staging block;
-        // the 8-byte piece hc (of 16 per 128-byte row) lives at hc ^ (row & 15)
-        auto stage = [&](int jj, int q, const float (&gv)[4]) {
-          const int hc = (jj * 8 + 2 * q + (l >> 5)) ^ (r & 15);
-          *reinterpret_cast<u32x2*>(ws + r * 64 + hc * 4) =
+        for (int q = 0; q < 4; ++q) {
+          // G without the one-hot term; an interior tile without bias needs no
+          // checks (rows past M are dropped by the store descriptor)
+          const int cb = tn * BN + acc_col<BN>(wn, j, q, lp);
+          f32x4 bv = {0.f, 0.f, 0.f, 0.f};
+          if constexpr (HB) bv = load4(bias, cb * 4);
+          float gv[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float xe = HB ? x[j][4 * q + e] + bv[e] : x[j][4 * q + e];
+            const float gg = __builtin_fmaf(rp.y, fast_exp2(__builtin_fmaf(xe, kLog2e, -rp.x)), -rp.w);
+            gv[e] = decltype(INTERIOR)::value || cb + e < g.N ? gg : 0.f;
+          }
+          // packed to bf16; the 8-byte piece hc (of 16 per 128-byte row) lives at hc ^ (row & 15)
+          const int hc = ((j & 1) * 8 + 2 * q + (l >> 5)) ^ (r & 15);
+          *reinterpret_cast<u32x2*>(row + (j >> 1) * 2048 + hc * 4) =
               u32x2{pack_bf16x2(gv[0], gv[1]), pack_bf16x2(gv[2], gv[3])};
-        };
-        if (interior) {
-#pragma unroll
-          for (int jj = 0; jj < 2; ++jj)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              float gv[4];
-#pragma unroll
-              for (int e = 0; e < 4; ++e)
-                gv[e] = __builtin_fmaf(rp.y, fast_exp2(__builtin_fmaf(x[jj][4 * q + e], kLog2e, -rp.x)),
-                                       -rp.w);
-              stage(jj, q, gv);
-            }
-        } else {
-#pragma unroll
-          for (int jj = 0; jj < 2; ++jj)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              const int cb = tn * BN + acc_col<BN>(wn, 2 * jp + jj, q, l);
-              f32x4 b = {0.f, 0.f, 0.f, 0.f};
-              if constexpr (HB) b = load4(bias, cb * 4);
-              float gv[4];
-#pragma unroll
-              for (int e = 0; e < 4; ++e) {
-                const float gg =
-                    __builtin_fmaf(rp.y, fast_exp2(__builtin_fmaf(x[jj][4 * q + e] + b[e], kLog2e, -rp.x)), -rp.w);
-                gv[e] = cb + e < g.N ? gg : 0.f;
-              }
-              stage(jj, q, gv);
-            }
         }
-        asm volatile("" ::: "memory");
-        // the one-hot term: the target column of row r, if it falls in this
-        // 64-column block, is corrected in place by the row's first lane
-        // (labels outside the band are negative or past it and never match)
-        const unsigned lc = (unsigned)(lab - (tn * BN + wn * (BN / 2) + jp * 64));
-        if (l < 32 && lc < 64u) {
-          bf16_t* const t = ws + r * 64 + ((((int)lc >> 2) ^ (r & 15)) << 2) + (lc & 3);
-          const float v = bf16_to_f32(*t) - rp.z;
-          *t = __builtin_bit_cast(bf16_t, (__bf16)v);
-        }
-        asm volatile("" ::: "memory");
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          const int rr = t * 8 + (l >> 3), c = l & 7;
-          // 16-byte chunk c = pieces 2c, 2c+1, stored at slot c ^ ((rr & 14) >> 1), halves swapped for odd rows
-          u32x4 v = *reinterpret_cast<const u32x4*>(ws + rr * 64 + ((c ^ ((rr & 14) >> 1)) << 3));
-          if (rr & 1) v = u32x4{v[2], v[3], v[0], v[1]};
-          const int trow = wm * kWaveRows + i * 32 + rr;
-          const int gcol = tn * BN + wn * (BN / 2) + jp * 64 + c * 8;
-          __builtin_amdgcn_raw_buffer_store_b128(v, gr, (int)(((long)trow * p.ldg + gcol) * 2), 0, 0);
-        }
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_sched_barrier(0);  // one 64-column block live at a time
       }
+      asm volatile("" ::: "memory");
+      // the one-hot term: the target column of row r, if the wave holds it, is
+      // corrected in place by the row's first lane (labels outside the band are
+      // negative or past it and never match)
+      const unsigned lc = (unsigned)(lab - col0);
+      if (l < 32 && lc < (unsigned)(BN / 2)) {
+        bf16_t* const t = row + (lc >> 6) * 2048 + ((((int)(lc & 63) >> 2) ^ (r & 15)) << 2) + (lc & 3);
+        const float v = bf16_to_f32(*t) - rp.z;
+        *t = __builtin_bit_cast(bf16_t, (__bf16)v);
+      }
+      asm volatile("" ::: "memory");
       __builtin_amdgcn_sched_barrier(0);
+    };
+    auto store = [&](int i) __attribute__((always_inline)) {
+      constexpr int kS = FN / 2 * 4;
+      u32x4 v[kS];
+#pragma unroll
+      for (int t = 0; t < kS; ++t) {
+        const int rr = (t & 3) * 8 + (l >> 3), c = l & 7;
+        // 16-byte chunk c = pieces 2c, 2c+1, stored at slot c ^ ((rr & 14) >> 1), halves swapped for odd rows
+        v[t] = *reinterpret_cast<const u32x4*>(ws + (i & 1) * kArea + (t >> 2) * 2048 + rr * 64 +
+                                               ((c ^ ((rr & 14) >> 1)) << 3));
+        if (rr & 1) v[t] = u32x4{v[t][2], v[t][3], v[t][0], v[t][1]};
+      }
+#pragma unroll
+      for (int t = 0; t < kS; ++t) {
+        const int trow = wm * kWaveRows + i * 32 + (t & 3) * 8 + (l >> 3), gcol = col0 + (t >> 2) * 64 + (l & 7) * 8;
+        __builtin_amdgcn_raw_buffer_store_b128(v[t], gr, (int)(((long)trow * p.ldg + gcol) * 2), 0, 0);
+      }
+      asm volatile("" ::: "memory");
+    };
+    const bool interior = !HB && (tn + 1) * BN <= g.N;
+    float4 rp = st.rp;
+    int lab = st.lab;
+#pragma unroll 1
+    for (int i = 0; i < FM; ++i) {
+      float4 rp1;
+      int lab1;
+      row_params(p, g, tm * kBM + acc_row(wm, min(i + 1, FM - 1), l), rp1, lab1);  // the next row block's
+      if (interior)
+        stage(i, rp, lab, std::true_type{});
+      else
+        stage(i, rp, lab, std::false_type{});
+      if (i > 0) store(i - 1);
+      rp = rp1;
+      lab = lab1;
     }
+    store(FM - 1);
   }
   static __device__ inline void finish(const Params&, State&, const GemmShape&, int, int, bf16_t*, int, int,
                                        int) {}
@@ -703,54 +716,71 @@ struct EpiAcc {
   static constexpr int kC = BN / 2;          // columns of a wave tile
   static constexpr int kL = kC / 4;          // lanes per row
   static constexpr int kPitch = kC + 4;
-  template <int I, bool FULL>
-  static __device__ __forceinline__ void rows32(const Params& p, WaveAcc<BN>& acc, const GemmShape& g, int m0, int n0,
-                                                int l, float* ws) {
+  template <bool FULL>
+  static __device__ __forceinline__ void rows32(const Params& p, const f32x16 (&x)[BN / 64], const GemmShape& g, int m0,
+                                                int n0, int l, float* ws) {
     constexpr int kR = 64 / kL, kT = 32 / kR;  // rows per instruction, instructions
     const int rr = l / kL, c = (l % kL) * 4;
     const bool nok = FULL || n0 + c < g.N;
-    long om[kT];
-    f32x4 old[kT];
+    int om[kT];  // output row; negative: outside
 #pragma unroll
     for (int t = 0; t < kT; ++t) {
       const int m = m0 + t * kR + rr;
-      om[t] = p.rowmap && (FULL || m < g.M) ? (long)p.rowmap[m] : (long)m;
+      om[t] = FULL || (nok && m < g.M) ? m : -1;
     }
-    // the accumulator's old values: modes 2, 3 from its row m, mode 4 from the output row
+    if (p.rowmap) {
+#pragma unroll
+      for (int t = 0; t < kT; ++t)
+        if (FULL || om[t] >= 0) om[t] = p.rowmap[om[t]];
+    }
+    const float* const acc32 = p.acc32 + n0 + c;
+    float* const out32 = reinterpret_cast<float*>(p.out) + n0 + c;
+    // the accumulator's old values, all loads in flight at once: modes 2, 3
+    // from its row m, mode 4 from the output row
+    f32x4 old[kT];
     if (p.mode >= 2) {
 #pragma unroll
       for (int t = 0; t < kT; ++t) {
-        const int m = m0 + t * kR + rr;
-        const float* src = p.mode == 4 ? reinterpret_cast<const float*>(p.out) + om[t] * p.ldo
-                                       : p.acc32 + (long)m * p.ldacc;
-        old[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (FULL || (nok && m < g.M)) old[t] = *reinterpret_cast<const f32x4*>(src + n0 + c);
+        const float* const src = p.mode == 4 ? out32 + (long)om[t] * p.ldo
+                                             : acc32 + (long)(m0 + t * kR + rr) * p.ldacc;
+        old[t] = FULL || om[t] >= 0 ? *reinterpret_cast<const f32x4*>(src) : f32x4{0.f, 0.f, 0.f, 0.f};
       }
     }
     asm volatile("" ::: "memory");
 #pragma unroll
     for (int j = 0; j < BN / 64; ++j) {
-      const f32x16 x = acc.take(I, j);
 #pragma unroll
       for (int q = 0; q < 4; ++q)
         *reinterpret_cast<f32x4*>(ws + (l & 31) * kPitch + j * 32 + q * 8 + (l >> 5) * 4) =
-            f32x4{x[4 * q], x[4 * q + 1], x[4 * q + 2], x[4 * q + 3]};
+            f32x4{x[j][4 * q], x[j][4 * q + 1], x[j][4 * q + 2], x[j][4 * q + 3]};
     }
     asm volatile("" ::: "memory");
+    f32x4 v[kT];
+    if constexpr (!FULL) {
 #pragma unroll
-    for (int t = 0; t < kT; ++t) {
-      const int row = t * kR + rr, m = m0 + row;
-      f32x4 v = *reinterpret_cast<const f32x4*>(ws + row * kPitch + c);
-      if (p.mode >= 2) v += old[t];
-      if (!FULL && !(nok && m < g.M)) continue;
-      if (p.mode == 1 || p.mode == 2) {
-        *reinterpret_cast<f32x4*>(p.acc32 + (long)m * p.ldacc + n0 + c) = v;
-      } else if (p.out_f32) {
-        *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(p.out) + om[t] * p.ldo + n0 + c) = v;
-      } else {
-        *reinterpret_cast<u32x2*>(reinterpret_cast<bf16_t*>(p.out) + om[t] * p.ldo + n0 + c) =
-            u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
-      }
+      for (int t = 0; t < kT; ++t) asm volatile("" : "+v"(om[t]));  // the masks are not kept in scalar registers
+    }
+#pragma unroll
+    for (int t = 0; t < kT; ++t) v[t] = *reinterpret_cast<const f32x4*>(ws + (t * kR + rr) * kPitch + c);
+    if (p.mode >= 2) {
+#pragma unroll
+      for (int t = 0; t < kT; ++t) v[t] += old[t];
+    }
+    if (p.mode == 1 || p.mode == 2) {
+#pragma unroll
+      for (int t = 0; t < kT; ++t)
+        if (FULL || om[t] >= 0)
+          *reinterpret_cast<f32x4*>(const_cast<float*>(acc32) + (long)(m0 + t * kR + rr) * p.ldacc) = v[t];
+    } else if (p.out_f32) {
+#pragma unroll
+      for (int t = 0; t < kT; ++t)
+        if (FULL || om[t] >= 0) *reinterpret_cast<f32x4*>(out32 + (long)om[t] * p.ldo) = v[t];
+    } else {
+#pragma unroll
+      for (int t = 0; t < kT; ++t)
+        if (FULL || om[t] >= 0)
+          *reinterpret_cast<u32x2*>(reinterpret_cast<bf16_t*>(p.out) + n0 + c + (long)om[t] * p.ldo) =
+              u32x2{pack_bf16x2(v[t][0], v[t][1]), pack_bf16x2(v[t][2], v[t][3])};
     }
     asm volatile("" ::: "memory");
   }
@@ -759,19 +789,17 @@ struct EpiAcc {
     pin_epilogue(l, tm, tn);
     float* const ws = reinterpret_cast<float*>(scratch) + (wm * 2 + wn) * 32 * kPitch;
     const int n0 = tn * BN + wn * kC;
-    auto block = [&](auto I) __attribute__((always_inline)) {
-      constexpr int i = decltype(I)::value;
+#pragma unroll 1
+    for (int i = 0; i < FM; ++i) {
       const int m0 = tm * kBM + acc_row(wm, i, 0);
+      if (m0 >= g.M) break;
+      f32x16 x[BN / 64];
+      acc.take_row(i, x);
       if (m0 + 32 <= g.M && n0 + kC <= g.N)
-        rows32<i, true>(p, acc, g, m0, n0, l, ws);
-      else if (m0 < g.M)
-        rows32<i, false>(p, acc, g, m0, n0, l, ws);
-    };
-    static_assert(FM == 4, "four row blocks");
-    block(std::integral_constant<int, 0>{});
-    block(std::integral_constant<int, 1>{});
-    block(std::integral_constant<int, 2>{});
-    block(std::integral_constant<int, 3>{});
+        rows32<true>(p, x, g, m0, n0, l, ws);
+      else
+        rows32<false>(p, x, g, m0, n0, l, ws);
+    }
   }
   static __device__ inline void finish(const Params&, State&, const GemmShape&, int, int, bf16_t*, int, int,
                                        int) {}
@@ -1037,6 +1065,7 @@ __device__ inline void dh_reduce_body(const DhReduce& r, long first, long step) 
   }
 }
 
+constexpr int kPopDW = 0, kPopDH = 1, kPopGrad = 2, kPopReduce = 3;  // populations of a band launch
 struct BandLaunch {
   GemmShape dw;
   AccParams e_dw;
@@ -1049,23 +1078,23 @@ struct BandLaunch {
   GemmShape gr;
   GradParams e_gr;
   int nb_dw, nb_dw2, nb_dh, nb_dh2, nb_gr;
-  // dH split over the band's K (few row tiles): with dh_split each dH tile
-  // has dh_ks workgroups (possibly one, for a narrow band); split k covers K
-  // columns [k*dh_kc, (k+1)*dh_kc) and writes its fp32 partial with
-  // e_dh*_part (mode 1) into slice k of the partial buffer (dh_part_stride
-  // floats apart), which a reduction folds into the accumulator afterwards.
-  int dh_split, dh_ks, dh_kc;
+  int pop[3], nb[3];  // the populations in order of their workgroups, and their sizes
+  // Each dH tile has dh_ks workgroups; workgroup k covers K columns
+  // [k*dh_kc, (k+1)*dh_kc).  dH split over the band's K (few row tiles): it
+  // writes its fp32 partial (mode 1) into slice k of the partial buffer
+  // (dh_part_stride floats apart), which a reduction folds into the
+  // accumulator afterwards; unsplit: one workgroup, dh_part_stride 0.
+  int dh_ks, dh_kc;
   long dh_part_stride;
-  AccParams e_dh_part, e_dh2_part;
   // the previous band's K-split dH partials folded into the accumulator by
   // nb_red workgroups (the partials alternate between two buffers)
   DhReduce red;
   int nb_red;
 };
 
-// One split workgroup of a K-split dH population (see BandLaunch).
+// One workgroup of the dH population (see BandLaunch).
 template <int BN>
-__device__ inline void dh_split_body(const GemmShape& g0, const AccParams& e0, int ks, int kc, long stride, int b,
+__device__ __forceinline__ void dh_body(const GemmShape& g0, const AccParams& e0, int ks, int kc, long stride, int b,
                                      int nb, bf16_t* smem) {
   const int k = b % ks, k0 = k * kc;
   GemmShape g = g0;
@@ -1082,41 +1111,40 @@ __device__ inline void dh_split_body(const GemmShape& g0, const AccParams& e0, i
 template <bool HB, bool AROW, bool KTAIL>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))) void band_kernel(BandLaunch p) {
   __shared__ __attribute__((aligned(16))) bf16_t smem[kLdsElems];
-  int b = blockIdx.x;
-  if (b < p.nb_dw) {
-    gemm_body<kBN, false, true, EpiAcc>(p.dw, p.e_dw, b, p.nb_dw, smem);
+  // the populations in the launch's order, then the reduction
+  int b = blockIdx.x, pop = kPopReduce;
+  if (b < p.nb[0]) {
+    pop = p.pop[0];
+  } else if ((b -= p.nb[0]) < p.nb[1]) {
+    pop = p.pop[1];
+  } else if ((b -= p.nb[1]) < p.nb[2]) {
+    pop = p.pop[2];
+  } else {
+    b -= p.nb[2];
+  }
+  if (pop == kPopDW) {
+    if (b < p.nb_dw) {
+      gemm_body<kBN, false, true, EpiAcc>(p.dw, p.e_dw, b, p.nb_dw, smem);
+      return;
+    }
+    gemm_body<kTailBN, false, true, EpiAcc>(p.dw2, p.e_dw2, b - p.nb_dw, p.nb_dw2, smem);
     return;
   }
-  b -= p.nb_dw;
-  if (b < p.nb_dw2) {
-    gemm_body<kTailBN, false, true, EpiAcc>(p.dw2, p.e_dw2, b, p.nb_dw2, smem);
+  if (pop == kPopDH) {
+    if (b < p.nb_dh) {
+      dh_body<kBN>(p.dh, p.e_dh, p.dh_ks, p.dh_kc, p.dh_part_stride, b, p.nb_dh, smem);
+      return;
+    }
+    dh_body<kTailBN>(p.dh2, p.e_dh2, p.dh_ks, p.dh_kc, p.dh_part_stride, b - p.nb_dh, p.nb_dh2, smem);
     return;
   }
-  b -= p.nb_dw2;
-  if (b < p.nb_dh) {
-    if (p.dh_split)
-      dh_split_body<kBN>(p.dh, p.e_dh_part, p.dh_ks, p.dh_kc, p.dh_part_stride, b, p.nb_dh, smem);
-    else
-      gemm_body<kBN, true, false, EpiAcc>(p.dh, p.e_dh, b, p.nb_dh, smem);
-    return;
-  }
-  b -= p.nb_dh;
-  if (b < p.nb_dh2) {
-    if (p.dh_split)
-      dh_split_body<kTailBN>(p.dh2, p.e_dh2_part, p.dh_ks, p.dh_kc, p.dh_part_stride, b, p.nb_dh2, smem);
-    else
-      gemm_body<kTailBN, true, false, EpiAcc>(p.dh2, p.e_dh2, b, p.nb_dh2, smem);
-    return;
-  }
-  b -= p.nb_dh2;
-  if (b < p.nb_gr) {
+  if (pop == kPopGrad) {
     if constexpr (HB)
       gemm_body<kBN, true, true, EpiGradBias, AROW, KTAIL>(p.gr, p.e_gr, b, p.nb_gr, smem);
     else
       gemm_body<kBN, true, true, EpiGrad, AROW, KTAIL>(p.gr, p.e_gr, b, p.nb_gr, smem);
     return;
   }
-  b -= p.nb_gr;
   dh_reduce_body(p.red, b * (long)kThreads + threadIdx.x, (long)p.nb_red * kThreads);
 }
 
@@ -2322,6 +2350,22 @@ void grad_shape(const bf16_t* H, const bf16_t* W, const float* bias, const BwdLa
   nb = gm * e.tiles_n;
 }
 
+// Order of a band launch's populations: the longest workgroups first, by the
+// length of their reductions (dW: the block's rows; dH: its share of the band;
+// recompute: d), so that the short ones fill the CUs the long ones leave idle.
+// N 2048, d 896 (dH 46 slabs, dW 30, recompute 14): a band launch takes 156 us
+// with dW first.
+void order_populations(BandLaunch& p, long k_dw, long k_dh, long k_gr) {
+  const long k[3] = {k_dw, k_dh, k_gr};
+  const int nb[3] = {p.nb_dw + p.nb_dw2, p.nb_dh + p.nb_dh2, p.nb_gr};
+  int o[3] = {kPopDW, kPopDH, kPopGrad};
+  std::stable_sort(o, o + 3, [&](int x, int y) { return k[x] > k[y]; });
+  for (int i = 0; i < 3; ++i) {
+    p.pop[i] = o[i];
+    p.nb[i] = nb[o[i]];
+  }
+}
+
 int launch_band(const BandLaunch& p, bool has_bias, hipStream_t st, int kind = CCE_KERNEL_BWD_BAND) {
   const int nb = p.nb_dw + p.nb_dw2 + p.nb_dh + p.nb_dh2 + p.nb_gr + p.nb_red;
   if (nb <= 0) return CCE_OK;
@@ -2779,6 +2823,7 @@ int cce_backward(const float* grad_out, const void* hidden, const void* weight, 
   const long dmain = band_dmain(d);
   BandLaunch first = {};
   grad_unit(0, first.gr, first.e_gr, first.nb_gr);
+  order_populations(first, 0, 0, d);
   rc = launch_band(first, bias != nullptr, st, CCE_KERNEL_BWD_GRAD);
   if (rc) return rc;
   // With 4 or more splits (very few rows) the band launches are short and the
@@ -2812,6 +2857,8 @@ int cce_backward(const float* grad_out, const void* hidden, const void* weight, 
     const long b = u / R, r = u % R;
     const bf16_t* G = L.G[u & 1];
     BandLaunch p = {};
+    long m0, rows;
+    block_span(r, m0, rows);
     if (need_dw) {
       if (dmain > 0) {
         dw_shape(b, r, G, 0, dmain, p.dw, p.e_dw);
@@ -2823,34 +2870,28 @@ int cce_backward(const float* grad_out, const void* hidden, const void* weight, 
       }
     }
     if (need_dh) {
-      long m0, rows;
-      block_span(r, m0, rows);
       const int gm = (int)ceil_div(rows, kBM);
       // K splits of this unit: every split non-empty and a whole number of slabs
+      long v0, vb;
+      band_cols(b, v0, vb);
+      p.dh_kc = (int)vb;
       int ks = 1;
-      if (L.dhpart) {
-        long v0, vb;
-        band_cols(b, v0, vb);
+      if (L.dhpart) {  // every unit, even one left with a single split
         p.dh_kc = (int)align_up((size_t)ceil_div(vb, L.dh_ks), 64);
         ks = (int)ceil_div(vb, p.dh_kc);
       }
-      p.dh_split = L.dhpart != nullptr;  // every unit, even one left with a single split
       p.dh_ks = ks;
-      p.dh_part_stride = Nb * d;
-      float* const part = L.dhpart ? dh_part(u) : nullptr;
-      if (dmain > 0) {
-        dh_shape(b, r, G, 0, dmain, p.dh, p.e_dh);
-        p.nb_dh = gm * (int)ceil_div(dmain, kBN) * ks;
-        p.e_dh_part = p.e_dh;
-        p.e_dh_part.acc32 = part; p.e_dh_part.ldacc = d; p.e_dh_part.mode = 1; p.e_dh_part.rowmap = nullptr;
-      }
-      if (dmain < d) {
-        dh_shape(b, r, G, dmain, d - dmain, p.dh2, p.e_dh2);
-        p.nb_dh2 = gm * (int)ceil_div(d - dmain, kTailBN) * ks;
-        p.e_dh2_part = p.e_dh2;
-        p.e_dh2_part.acc32 = part ? part + dmain : nullptr; p.e_dh2_part.ldacc = d;
-        p.e_dh2_part.mode = 1; p.e_dh2_part.rowmap = nullptr;
-      }
+      p.dh_part_stride = L.dhpart ? Nb * d : 0;
+      auto dh_tiles = [&](long c0, long nc, int bn, GemmShape& g, AccParams& e, int& nb) {
+        dh_shape(b, r, G, c0, nc, g, e);
+        nb = gm * (int)ceil_div(nc, bn) * ks;
+        if (L.dhpart) {
+          e.acc32 = dh_part(u) + c0;
+          e.ldacc = d; e.mode = 1; e.rowmap = nullptr;
+        }
+      };
+      if (dmain > 0) dh_tiles(0, dmain, kBN, p.dh, p.e_dh, p.nb_dh);
+      if (dmain < d) dh_tiles(dmain, d - dmain, kTailBN, p.dh2, p.e_dh2, p.nb_dh2);
       // the previous unit's partials (the other buffer) into the accumulator
       if (fold && u > 0) {
         p.red = dh_reduction(u - 1, prev_ks);
@@ -2861,6 +2902,7 @@ int cce_backward(const float* grad_out, const void* hidden, const void* weight, 
       prev_ks = ks;
     }
     if (u + 1 < units) grad_unit(u + 1, p.gr, p.e_gr, p.nb_gr);
+    order_populations(p, rows, p.dh_kc, d);
     rc = launch_band(p, bias != nullptr, st);
     if (rc) return rc;
     if (need_dh && L.dhpart && (!fold || u + 1 == units)) {

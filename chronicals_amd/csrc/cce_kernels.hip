@@ -35,6 +35,7 @@
 #include <string.h>
 #include <math.h>
 #include <float.h>
+#include <limits.h>
 
 #include <algorithm>
 #include <mutex>
@@ -1468,13 +1469,24 @@ __global__ __launch_bounds__(256) void ce_logits_fwd_kernel(const T* __restrict_
   }
 }
 
+// Zeroes a gradient row of V elements by NT threads.
+template <int NT, typename TO>
+__device__ inline void zero_row(TO* drow, int V, int tid) {
+  const RowSplit<TO> sp(drow, V);
+  if (tid < sp.head) drow[tid] = f32_to_elem<TO>(0.f);
+  if (tid < V - sp.tail_start) drow[sp.tail_start + tid] = f32_to_elem<TO>(0.f);
+  u32x4* const body = reinterpret_cast<u32x4*>(drow + sp.head);
+  for (int c = tid; c < sp.chunks; c += NT) __builtin_nontemporal_store(u32x4{0u, 0u, 0u, 0u}, body + c);
+}
+
 // Backward: the derivative of the forward's row loss, times g_n, for valid
 // rows (0 for ignored rows), with p_v = exp(x_v - lse):
 //   CCE_SMOOTH_LOGV:    g_n * (((1-eps) + 2z*lse) * p_v - (1-eps) * [v == label])
 //   CCE_SMOOTH_UNIFORM: g_n * ((1 + 2z*lse) * p_v - eps/V - (1-eps) * [v == label])
 // g_n = grad_out[n] ('none'), grad_out[0] ('sum') or grad_out[0] / max(n_valid, 1)
 // ('mean').  dX may be X itself (same dtype and stride): every element is read
-// and then written by the same thread.
+// and then written by the same thread.  An ignored row is zeroed without being
+// read (the rows in the order of the forward or against it: the same time).
 template <typename T, typename TO>
 __global__ __launch_bounds__(256) void ce_logits_bwd_kernel(const float* __restrict__ grad_out, const T* X, long ld,
                                                             const void* labels, int labels64,
@@ -1487,6 +1499,10 @@ __global__ __launch_bounds__(256) void ce_logits_bwd_kernel(const float* __restr
   TO* drow = dX + (long)n * ldg;
   const long lab = load_label(labels, labels64, n);
   const bool valid = lab != ignore_index;
+  if (!valid) {
+    zero_row<256>(drow, V, tid);
+    return;
+  }
   float g = reduction == CCE_REDUCTION_NONE ? grad_out[n] : grad_out[0];
   if (reduction == CCE_REDUCTION_MEAN) g /= (float)(n_valid[0] > 1 ? n_valid[0] : 1);
   const float l = lse[n];
@@ -1621,7 +1637,9 @@ __global__ __launch_bounds__(kFusedThreads) void ce_logits_fused_kernel(
     const float cT = valid ? g * (1.f - eps) : 0.f;
     const float l2 = lse * kLog2e;
     auto grad1 = [&](int v, float x) { return (cP * fast_exp2(x * kLog2e - l2) - cU) - (v == t ? cT : 0.f); };
-    if ((reinterpret_cast<uintptr_t>(drow + sp.head) & 15u) != 0) {
+    if (!valid) {
+      zero_row<kFusedThreads>(drow, V, tid);
+    } else if ((reinterpret_cast<uintptr_t>(drow + sp.head) & 15u) != 0) {
       for (int v = tid; v < V; v += kFusedThreads) drow[v] = f32_to_elem<TO>(grad1(v, elem_to_f32(row[v])));
     } else {
       if (tid < sp.head) drow[tid] = f32_to_elem<TO>(grad1(tid, elem_to_f32(row[tid])));
@@ -1720,12 +1738,13 @@ __global__ __launch_bounds__(1024) void compact_rows_kernel(const void* labels, 
   if (nb_fwd > 0) {
     // the forward's vocabulary splits over the live row tiles (live[1]): the
     // cheapest s of at most nb_fwd / tiles workgroups per row tile by
-    // split_cost, and at least enough for 4 rounds of workgroups when the
-    // launch allows (long single-round schedules leave CUs idle at the end);
-    // thread t prices s = t + 1, ties go to the larger s
+    // split_cost, and at least enough for one round of workgroups; thread t
+    // prices s = t + 1, ties go to the larger s.  With at least four rounds
+    // instead, N 700 / 2048 at d 896, V 151936 took 237 / 484 us, with one
+    // 208 / 466; N 16384 takes 3.41 ms either way
     const int gl = (int)((min((long)tiles * kBM, (long)N) + kBM - 1) / kBM);
     const int smax = max(1, min(min(nb_fwd / gl, tiles_n), 1024));
-    const int smin = min(smax, max(1, (4 * ncu + gl - 1) / gl));
+    const int smin = min(smax, max(1, (ncu + gl - 1) / gl));
     __shared__ float cost[1024];
     __shared__ int arg[1024];
     const int sv = tid + 1;
@@ -1955,17 +1974,30 @@ struct Carver {
 // the 256 CUs several times over.
 bool whole_slabs(long d) { return d % kBK == 0; }
 
-// Vocabulary splits per row tile of a forward over every row tile: about 512
-// workgroups for few row tiles (runs of several vocabulary tiles, so the
-// pipeline's start is paid once per run), never fewer splits than
-// min(32, 2048 / row tiles): large batches keep their split counts.
+// Vocabulary splits per row tile of a forward over every row tile: the
+// cheapest by split_cost of at least one round of workgroups (on the card's 256
+// CUs, so that the workspace does not depend on the device at hand) and at most
+// about 512 of them, or min(32, 2048 / row tiles) splits.  Always the most
+// splits took N 1500, d 1000, V 50257 from 5 tile times (42 splits) to 6.
 int forward_splits(long N, long d, long V) {
+  (void)d;
   if (N <= 0) return 1;
-  const long gm = ceil_div(N, kBM), tn = ceil_div(V, kBN);
-  long s = std::max(ceil_div(512, gm), std::min<long>(32, ceil_div(2048, gm)));
-  if (s > tn) s = tn;
-  if (s < 1) s = 1;
-  return (int)s;
+  constexpr int kCus = 256;
+  const int gm = (int)ceil_div(N, kBM), tn = (int)ceil_div(V, kBN);
+  const int smax = (int)std::min<long>(std::max(ceil_div(512, gm), std::min<long>(32, ceil_div(2048, gm))), tn);
+  const int smin = (int)std::min<long>(smax, ceil_div(kCus, gm));
+  int best = smax;
+  float cost = split_cost(gm, tn, smax, kCus);
+  // one candidate per length of a run: the fewest splits with runs of t tiles
+  for (int t = (int)ceil_div(tn, smax); t <= (int)ceil_div(tn, smin); ++t) {
+    const int sp = std::min(smax, std::max(smin, (int)ceil_div(tn, t)));
+    const float c = split_cost(gm, tn, sp, kCus);
+    if (c < cost) {
+      cost = c;
+      best = sp;
+    }
+  }
+  return best;
 }
 
 // Workgroups of the forward GEMM, each with a slot of 256 rows of (max,
@@ -2353,10 +2385,12 @@ void grad_shape(const bf16_t* H, const bf16_t* W, const float* bias, const BwdLa
 // Order of a band launch's populations: the longest workgroups first, by the
 // length of their reductions (dW: the block's rows; dH: its share of the band;
 // recompute: d), so that the short ones fill the CUs the long ones leave idle.
-// N 2048, d 896 (dH 46 slabs, dW 30, recompute 14): a band launch takes 156 us
-// with dW first.
+// N 2048, d 896, V 151936 (dH 46 slabs, dW 30, recompute 14): forward and
+// backward 2.51 ms with dW always first, 2.32 ms so.  A dW over one row tile is
+// bound by its stores, not its slabs, and starts first: N 256, d 768, V 50257
+// in fp32 288 us behind the others, 254 us first.
 void order_populations(BandLaunch& p, long k_dw, long k_dh, long k_gr) {
-  const long k[3] = {k_dw, k_dh, k_gr};
+  const long k[3] = {k_dw <= kBM ? LONG_MAX : k_dw, k_dh, k_gr};
   const int nb[3] = {p.nb_dw + p.nb_dw2, p.nb_dh + p.nb_dh2, p.nb_gr};
   int o[3] = {kPopDW, kPopDH, kPopGrad};
   std::stable_sort(o, o + 3, [&](int x, int y) { return k[x] > k[y]; });

@@ -549,7 +549,7 @@ struct GradParams {
 //
 // Stores go through LDS: in the MFMA layout a lane holds one row, so a direct
 // store instruction would touch 32 rows with 16 bytes each.  Each wave writes
-// a 32 x 64 block into its own 4 KB of LDS (8-byte pieces, XOR-swizzled by
+// 32 x 64 blocks into its own part of the ring (8-byte pieces, XOR-swizzled by
 // row so the 16 lanes of a write phase hit distinct banks), reads it back
 // row-major and stores whole 128-byte row segments, 8 rows per instruction.
 // A wave's LDS operations execute in order, so no barrier is needed.
@@ -1012,9 +1012,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
 // writes the other G buffer.  Both gradient GEMMs tile d in 256-wide column
 // tiles plus one 128-wide tail tile when d % 256 <= 128 (no MFMA work spent
 // on padding, and the wide tiles do the most work per CU-second).
-// Workgroups are numbered longest first — dW (K = N), dH (K = band width),
-// then the short recompute tiles, which fill the CUs the long tiles leave
-// idle at the end of the band.
+// The populations' workgroups are numbered longest first (order_populations).
 // dH reads W's rows as they are (an MN-major B): against a transposed copy of
 // each band's rows the band launch takes the same time at d = 896 and 1.4% less
 // at d = 4096 (8192 rows), and the copies and their memory are gone.  With dH split over K on very
@@ -1993,8 +1991,6 @@ struct Carver {
   }
 };
 
-// Forward vocabulary splits: enough (row tile x split) workgroups to cover
-// the 256 CUs several times over.
 bool whole_slabs(long d) { return d % kBK == 0; }
 
 // Vocabulary splits per row tile of a forward over every row tile: the
@@ -2002,8 +1998,7 @@ bool whole_slabs(long d) { return d % kBK == 0; }
 // CUs, so that the workspace does not depend on the device at hand) and at most
 // about 512 of them, or min(32, 2048 / row tiles) splits.  Always the most
 // splits took N 1500, d 1000, V 50257 from 5 tile times (42 splits) to 6.
-int forward_splits(long N, long d, long V) {
-  (void)d;
+int forward_splits(long N, long V) {
   if (N <= 0) return 1;
   constexpr int kCus = 256;
   const int gm = (int)ceil_div(N, kBM), tn = (int)ceil_div(V, kBN);
@@ -2032,9 +2027,9 @@ int forward_splits(long N, long d, long V) {
 // row tiles drop out costs little), but no more than 8192 workgroups beyond
 // the count over every row tile, which bounds its partials at large N
 // (16 MiB at N = 2^21 rather than 1 GiB).
-long forward_slots(long N, long d, long V, bool compact) {
+long forward_slots(long N, long V, bool compact) {
   const long gm = ceil_div(std::max<long>(N, 1), kBM);
-  const long base = gm * forward_splits(N, d, V);
+  const long base = gm * forward_splits(N, V);
   if (!compact) return base;
   const long tn = ceil_div(V, kBN);
   return std::max(base, std::min(gm * std::min<long>(64, tn), 8192L));
@@ -2107,7 +2102,7 @@ long block_rows(long N, long Vb) {
 
 // The compacted GEMMs take H's rows either from a gathered copy (Hc, N x d
 // bf16 of workspace, written by gather_rows_kernel) or straight from H
-// through the row order (ARows).  Reading through the order costs each
+// through the row order (Stream, ROWS).  Reading through the order costs each
 // workgroup a dependent load before its first slab (about 1.5% of a C2 band
 // launch, whose recompute workgroups run one tile each), so the copy is kept
 // while it is small next to the band state (H below 256 MiB); from there up
@@ -2151,7 +2146,7 @@ int wsum_splits(long d, long V) {
 }
 
 // The forward compacts its rows when only the labelled rows' lse is wanted
-// and the direct-to-LDS GEMM runs (d a multiple of 64).
+// and d is a multiple of 64.
 // More than one row tile: otherwise there is none to skip.
 bool fwd_compacts(long N, long d, int lse_rows) {
   return lse_rows == CCE_LSE_LABELLED_ROWS && whole_slabs(d) && N > kBM;
@@ -2164,7 +2159,7 @@ FwdLayout fwd_layout(void* ws, long N, long d, long V, int reduction, int lse_ro
   const long nb = ceil_div(N, 4);
   // [S][N rounded up to 256] partials, or for a compacted forward one slot of
   // 256 rows per launched workgroup
-  const size_t parts = (size_t)forward_slots(N, d, V, compact) * kBM;
+  const size_t parts = (size_t)forward_slots(N, V, compact) * kBM;
   L.pm = c.take<float>(parts);
   L.ps = c.take<float>(parts);
   L.bsum = c.take<float>((size_t)(nb > 0 ? nb : 1));
@@ -2278,12 +2273,12 @@ BwdLayout bwd_layout(void* ws, long N, long d, long V, long Vb, bool need_dh, bo
 
 bool misaligned(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) != 0; }
 
-// The direct-to-LDS pipelines read K-major operands in 64-wide slabs with the
-// slab's k offset outside the buffer range check (dma_kmajor), so each
+// The GEMMs read K-major operands in 64-wide slabs with the slab's k offset
+// outside the buffer range check (Stream), so each
 // operand row must hold every slab the GEMM reads: kb + K rounded up to 64
 // columns at most ld.  Checked on the host before each launch; a layout that
 // broke it would otherwise read past the operand.
-// With ktail (dma_kmajor's KTAIL) the columns from K on are not read.
+// With ktail (Stream, TAIL) the columns from K on are not read.
 bool kmajor_fits(long ld, long kb, long K, bool ktail = false) {
   return K <= 0 || kb + (ktail ? K : (long)align_up((size_t)K, kBK)) <= ld;
 }
@@ -2522,8 +2517,8 @@ int forward_run(const void* hidden, const void* weight, const void* labels, int 
     return rc;
   }
   const FwdLayout L = fwd_layout(workspace, N, d, V, reduction, lse_rows, prefer_in_place);
-  const int S = forward_splits(N, d, V);
-  const int slots = (int)forward_slots(N, d, V, L.idx != nullptr);  // workgroups
+  const int S = forward_splits(N, V);
+  const int slots = (int)forward_slots(N, V, L.idx != nullptr);  // workgroups
 
   // CCE_LSE_LABELLED_ROWS: the labelled rows go first and the GEMM runs only
   // over the row tiles that hold them (the partials then follow that order)

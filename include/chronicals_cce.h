@@ -178,19 +178,19 @@ int cce_backward_workspace_bytes(int64_t N, int64_t d, int64_t V, int64_t chunk_
  * grad_*_dtype selects CCE_DTYPE_BF16 or CCE_DTYPE_F32 output; grad_bias is
  * fp32.  The vocabulary is processed in bands of up to 8192 columns: the
  * reference's chunk_size argument (:1028), rounded up to a multiple of 256,
- * bounds the band from above (the partial band, if any, comes first); from
- * 1024 to 4095 rows the bands are up to 4x wider, while G and W^T of a band
- * take no more than at 4096 rows.  The rows are processed in blocks whose
+ * bounds the band from above (the partial band, if any, comes first); below
+ * 3072 rows the bands widen to what the gradient of 3072 rows takes at that
+ * width.  The rows are processed in blocks whose
  * band gradient (two bf16 buffers of rows x band) stays within 512 MiB, so
  * that memory does not grow with N; dW of a band accumulates over the
  * blocks.  fp32 gradients accumulate in place; bf16 ones in fp32 workspace.
  * Deterministic: every reduction runs in a fixed order, including the fp32
  * partials of dH when few rows make the library split each band's columns
  * over several workgroups.
- * grad_hidden and grad_weight double as scratch while the call's kernels run
- * (H^T, and each band's W^T, live in output memory that is not yet written),
- * so neither may overlap an input, and their contents are final only once
- * the stream has run past the call.
+ * grad_hidden doubles as scratch while the call's kernels run (H^T, or H in
+ * row order, lives in it until dH is written).  Neither gradient may overlap
+ * an input, and their contents are final only once the stream has run past
+ * the call.
  */
 int cce_backward(const float* grad_out, const void* hidden, const void* weight, const void* labels,
                  int labels_int64, const float* bias, const float* lse, const int32_t* n_valid,

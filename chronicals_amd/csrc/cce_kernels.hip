@@ -469,8 +469,9 @@ struct EpiLseT {
       }
       return;
     }
-    // edge tile or bias: the columns' bias added, columns past V at -inf
-    const __amdgpu_buffer_rsrc_t bias = make_rsrc(p.bias, HB ? (long)g.N * 4 : 0L);
+    // edge tile or bias: the columns' bias added, columns past V at -inf (the
+    // descriptor starts at the tile: V may be past what 31 bits of bytes span)
+    const __amdgpu_buffer_rsrc_t bias = make_rsrc(p.bias + c0, HB ? (long)(g.N - c0) * 4 : 0L);
 #pragma unroll
     for (int i = 0; i < FM; ++i) {
       f32x16 x[FN];
@@ -481,11 +482,11 @@ struct EpiLseT {
         x[j] = acc.take(i, j);
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const int col = c0 + acc_col<BN>(wn, j, q, lp);
+          const int col = acc_col<BN>(wn, j, q, lp);
           f32x4 b = {0.f, 0.f, 0.f, 0.f};
           if constexpr (HB) b = load4(bias, col * 4);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) x[j][4 * q + e] = col + e < g.N ? x[j][4 * q + e] + b[e] : -INFINITY;
+          for (int e = 0; e < 4; ++e) x[j][4 * q + e] = col + e < g.N - c0 ? x[j][4 * q + e] + b[e] : -INFINITY;
         }
         asm volatile("" ::: "memory");  // one block's bias loads at a time
         __builtin_amdgcn_sched_barrier(0);

@@ -2077,26 +2077,39 @@ int device_cus() {
   return cus[dev];
 }
 
+// Bytes of a backward's two band gradient buffers (rows of a block x band,
+// bf16): 512 MiB, or CHRONICALS_CCE_G_BUDGET_MB from the environment (read on
+// every call, so a workspace query and the call it sizes must see the same
+// value).
+constexpr long kGBudget = 512L << 20;
+long g_budget() {
+  const char* e = getenv("CHRONICALS_CCE_G_BUDGET_MB");
+  if (e && *e) {
+    const long mb = strtol(e, nullptr, 10);
+    if (mb > 0 && mb < (1L << 20)) return mb << 20;
+  }
+  return kGBudget;
+}
+
 // Vocabulary band width: chunk rounded up to a multiple of 256, at most
 // kBandCap (8192) columns and at least 256, within V rounded up.  chunk_size
 // bounds the band from above only: the reference's trainer asks for 16384 at
 // V >= 128K (get_optimal_chunk_size), which here would double the band
 // buffers for no measured gain.
-constexpr long kMaxBand = 1L << 20;
 constexpr long kBandCap = 8192;
-long band_width(long V, long chunk, long N, long d) {
+long band_width(long V, long chunk, long N) {
   long vb = chunk <= 0 ? kBandCap : std::min(chunk, kBandCap);
   vb = align_up((size_t)vb, 256);
   // with few rows a band launch is short and its fixed costs dominate: the
   // bands widen to what 3072 rows' band gradient (rows x band) takes at the
   // unwidened band (which leaves room for the K-split dH's partials within
-  // what 4096 rows take), in equal parts of the vocabulary.  Forward and
-  // backward, against bands that widen from 1024 rows on with W transposed for
-  // each: N 64, d 896, V 32000 305 -> 222 us; N 256, d 768, V 50257 fp32
-  // 463 -> 252 us; N 2048, d 896, V 151936 2492 -> 2446 us.
+  // what 4096 rows take), but not past the G budget, in equal parts of the
+  // vocabulary.  Forward and backward, against bands that widen from 1024 rows
+  // on with W transposed for each: N 64, d 896, V 32000 305 -> 222 us; N 256,
+  // d 768, V 50257 fp32 463 -> 252 us; N 2048, d 896, V 151936 2492 -> 2446 us.
   const long rows = (long)align_up((size_t)(N > 0 ? N : 1), 256);
   if (rows < 3072) {
-    vb = std::min<long>(vb * 3072 / rows, kMaxBand);
+    vb = std::max(vb, std::min(vb * 3072 / rows, g_budget() / (4 * rows) / 256 * 256));
     vb = (long)align_up((size_t)ceil_div(V, ceil_div(V, vb)), 256);
   }
   const long vmax = (long)align_up((size_t)V, 256);
@@ -2109,19 +2122,8 @@ long band_width(long V, long chunk, long N, long d) {
 // (rows x band) bf16 and there are two such buffers (band b+1's recompute
 // overlaps band b's GEMMs), so a block has at most budget / (4 * band) rows,
 // a multiple of 256; a batch that fits is one block.  G's memory is then
-// bounded by the budget whatever N is; dW of a band accumulates over the
-// blocks.  The budget is 512 MiB, or CHRONICALS_CCE_G_BUDGET_MB from the
-// environment (read on every call, so a workspace query and the call it
-// sizes must see the same value).
-constexpr long kGBudget = 512L << 20;
-long g_budget() {
-  const char* e = getenv("CHRONICALS_CCE_G_BUDGET_MB");
-  if (e && *e) {
-    const long mb = strtol(e, nullptr, 10);
-    if (mb > 0 && mb < (1L << 20)) return mb << 20;
-  }
-  return kGBudget;
-}
+// bounded by the budget whatever N is (or by 256 rows of a band, if that is
+// more); dW of a band accumulates over the blocks.
 long block_rows(long N, long Vb) {
   const long n = std::max<long>(N, 1);
   long nb = g_budget() / (4 * Vb) / kBM * kBM;
@@ -2698,7 +2700,7 @@ int cce_backward_workspace_bytes(int64_t N, int64_t d, int64_t V, int64_t chunk_
   if ((need_grad_hidden && grad_hidden_dtype != CCE_DTYPE_BF16 && grad_hidden_dtype != CCE_DTYPE_F32) ||
       (need_grad_weight && grad_weight_dtype != CCE_DTYPE_BF16 && grad_weight_dtype != CCE_DTYPE_F32))
     return fail(CCE_ERR_INVALID_ARG, "gradient dtypes must be CCE_DTYPE_BF16 or CCE_DTYPE_F32");
-  *bytes = bwd_layout(nullptr, N, d, V, band_width(V, chunk_size, N, d), need_grad_hidden != 0,
+  *bytes = bwd_layout(nullptr, N, d, V, band_width(V, chunk_size, N), need_grad_hidden != 0,
                       need_grad_weight != 0, grad_hidden_dtype == CCE_DTYPE_F32,
                       grad_weight_dtype == CCE_DTYPE_F32).bytes;
   return CCE_OK;
@@ -2765,7 +2767,7 @@ int cce_backward(const float* grad_out, const void* hidden, const void* weight, 
   if (need_db && !bias) return fail(CCE_ERR_INVALID_ARG, "grad_bias requested without bias");
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const bool dh_f32 = grad_hidden_dtype == CCE_DTYPE_F32, dw_f32 = grad_weight_dtype == CCE_DTYPE_F32;
-  const long Vb = band_width(V, chunk_size, N, d);
+  const long Vb = band_width(V, chunk_size, N);
   const BwdLayout need = bwd_layout(nullptr, N, d, V, Vb, need_dh, need_dw, dh_f32, dw_f32);
   if (workspace_bytes < need.bytes || (need.bytes && !workspace))
     return fail(CCE_ERR_WORKSPACE, "workspace too small: need %zu bytes, got %zu", need.bytes, workspace_bytes);

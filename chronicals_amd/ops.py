@@ -45,21 +45,22 @@ __all__ = ["cce_fwd", "cce_bwd", "ce_logits_fwd", "ce_logits_bwd", "ce_logits_bw
            "ce_logits_fwd_bwd_"]
 
 _SCHEMAS = (
-    "cce_fwd(Tensor hidden, Tensor weight, Tensor labels, Tensor? bias, int ignore_index, float label_smoothing, "
-    "float z_loss_weight, int smoothing_form, int reduction, int lse_rows=0) -> (Tensor, Tensor, Tensor, Tensor)",
+    "cce_fwd(Tensor hidden, Tensor weight, Tensor labels, Tensor? bias, SymInt ignore_index, float label_smoothing, "
+    "float z_loss_weight, SymInt smoothing_form, SymInt reduction, SymInt lse_rows=0) "
+    "-> (Tensor, Tensor, Tensor, Tensor)",
     "cce_bwd(Tensor grad_out, Tensor hidden, Tensor weight, Tensor labels, Tensor lse, Tensor n_valid, Tensor? bias, "
-    "int ignore_index, float label_smoothing, float z_loss_weight, int reduction, int chunk_size, bool need_dh, "
-    "bool need_dw, bool need_db, bool dh_f32, bool dw_f32) -> (Tensor, Tensor, Tensor)",
-    "ce_logits_fwd(Tensor logits, Tensor labels, int ignore_index, float label_smoothing, float z_loss_weight, "
-    "int smoothing_form, int reduction) -> (Tensor, Tensor, Tensor)",
-    "ce_logits_bwd(Tensor grad_out, Tensor logits, Tensor labels, Tensor lse, Tensor n_valid, int ignore_index, "
-    "float label_smoothing, float z_loss_weight, int smoothing_form, int reduction, bool f32_grad) -> Tensor",
-    "ce_logits_fwd_bwd(Tensor logits, Tensor labels, int ignore_index, float label_smoothing, float z_loss_weight, "
-    "int smoothing_form, int reduction, bool grad_mean, bool f32_grad) -> (Tensor, Tensor, Tensor, Tensor)",
+    "SymInt ignore_index, float label_smoothing, float z_loss_weight, SymInt reduction, SymInt chunk_size, "
+    "bool need_dh, bool need_dw, bool need_db, bool dh_f32, bool dw_f32) -> (Tensor, Tensor, Tensor)",
+    "ce_logits_fwd(Tensor logits, Tensor labels, SymInt ignore_index, float label_smoothing, float z_loss_weight, "
+    "SymInt smoothing_form, SymInt reduction) -> (Tensor, Tensor, Tensor)",
+    "ce_logits_bwd(Tensor grad_out, Tensor logits, Tensor labels, Tensor lse, Tensor n_valid, SymInt ignore_index, "
+    "float label_smoothing, float z_loss_weight, SymInt smoothing_form, SymInt reduction, bool f32_grad) -> Tensor",
+    "ce_logits_fwd_bwd(Tensor logits, Tensor labels, SymInt ignore_index, float label_smoothing, float z_loss_weight, "
+    "SymInt smoothing_form, SymInt reduction, bool grad_mean, bool f32_grad) -> (Tensor, Tensor, Tensor, Tensor)",
 )
 _LIBRARY = torch.library.Library("chronicals_hip", "FRAGMENT")
 for _s in _SCHEMAS:
-    _LIBRARY.define(_s)
+    _LIBRARY.define(_s, tags=(torch.Tag.pt2_compliant_tag,))
 
 
 def _load_kernels() -> None:

@@ -15,6 +15,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 REPO_DIR = os.path.dirname(PKG_DIR)
@@ -79,7 +80,7 @@ def torch_lib_path() -> str:
 def torch_compile_command(out_path: str) -> list:
     import torch
 
-    base = os.path.join(os.path.dirname(torch.__file__))
+    base = os.path.dirname(torch.__file__)
     inc, lib = os.path.join(base, "include"), os.path.join(base, "lib")
     rocm = os.path.dirname(os.path.dirname(os.path.realpath(hipcc_path())))
     return [
@@ -88,9 +89,9 @@ def torch_compile_command(out_path: str) -> list:
         "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
         f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
         "-isystem", inc, "-isystem", os.path.join(inc, "torch", "csrc", "api", "include"),
-        "-isystem", os.path.join(rocm, "include"),
+        "-isystem", os.path.join(rocm, "include"), "-isystem", sysconfig.get_paths()["include"],
         TORCH_SRC, "-o", out_path,
-        "-L", lib, "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch", f"-Wl,-rpath,{lib}",
+        "-L", lib, "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch", "-ltorch_python", f"-Wl,-rpath,{lib}",
     ]
 
 

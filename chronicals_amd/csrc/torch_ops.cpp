@@ -7,13 +7,17 @@
 // V 32000 went from 222 to 143 us.
 //
 // ops.py defines the schemas and the fake (meta) implementations; the kernels
-// are registered here.  The C functions come from the library that the Python loader
-// opened (chronicals_torch_bind), so that CHRONICALS_CCE_LIB and the loader's
-// checks hold for both.
+// are registered here.  The C functions come from the library that the Python
+// loader opens (chronicals_torch_bind), so that CHRONICALS_CCE_LIB and the
+// loader's checks hold for both.  The first call of an operator asks for it
+// through a Python callable that ops.py hands over (chronicals_torch_hooks).
+#include <Python.h>
+
 #include <ATen/ATen.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <dlfcn.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/autograd_not_implemented_fallback.h>
 #include <torch/library.h>
 
@@ -41,10 +45,28 @@ struct Api {
 Api g_api;
 std::atomic<bool> g_bound{false};
 
+PyObject* g_load = nullptr;  // load(): opens the library and binds it here, or raises
+
+// Calls a hook; what it raises goes on as a Python exception.  Operators run
+// without the interpreter's lock.
+void call_hook(PyObject* hook) {
+  TORCH_CHECK(hook != nullptr, "chronicals_amd.ops is not imported");
+  struct Gil {
+    PyGILState_STATE state = PyGILState_Ensure();
+    ~Gil() { PyGILState_Release(state); }
+  } gil;
+  PyObject* const res = PyObject_CallObject(hook, nullptr);
+  if (!res) {
+    python_error e;
+    e.persist();
+    throw e;
+  }
+  Py_DECREF(res);
+}
+
 const Api& api() {
-  TORCH_CHECK(g_bound.load(std::memory_order_acquire),
-              "libchronicals_cce.so is not loaded (chronicals_amd._lib.load() says why): build it with "
-              "`python -m chronicals_amd.build` (or __graft_entry__.build())");
+  if (!g_bound.load(std::memory_order_acquire)) call_hook(g_load);
+  TORCH_CHECK(g_bound.load(std::memory_order_acquire), "libchronicals_cce.so is not bound");
   return g_api;
 }
 
@@ -268,6 +290,12 @@ int chronicals_torch_bind(void* handle) {
     g_bound.store(true, std::memory_order_release);
   }
   return 0;
+}
+
+// The Python callable of api(); called with the interpreter's lock.
+void chronicals_torch_hooks(PyObject* load) {
+  Py_XINCREF(load);
+  Py_XSETREF(g_load, load);
 }
 
 }  // extern "C"

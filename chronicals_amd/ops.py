@@ -63,30 +63,40 @@ for _s in _SCHEMAS:
     _LIBRARY.define(_s, tags=(torch.Tag.pt2_compliant_tag,))
 
 
-def _load_kernels() -> None:
-    """Load the C++ kernels of the operators and hand them the HIP library's
-    functions.  Without a build the package still imports; calling an operator
-    then raises."""
+def _load_kernels() -> bool:
+    """Load the C++ kernels of the operators if they are built.  The HIP library
+    is opened by the first call of an operator: what fails then (no library, a
+    stale one, CHRONICALS_CCE_LIB naming a broken one) raises in that call, and
+    a call after it has been put right works."""
     path = _build.torch_lib_path()
     if not os.path.exists(path):
-        def missing(*args, **kwargs):
-            raise ImportError(f"{path} not found: build it with `python -m chronicals_amd.build` "
-                              f"(or __graft_entry__.build())")
-        for s in _SCHEMAS:
-            _LIBRARY.impl(s.split("(", 1)[0], missing, "CUDA")
-        return
+        return False
     torch.ops.load_library(path)
-    try:
-        lib = _lib.load()
-    except ImportError:
-        return  # the operators say so when they are called
-    native = ctypes.CDLL(path)
+    native = ctypes.PyDLL(path)
     native.chronicals_torch_bind.argtypes = [ctypes.c_void_p]
-    if native.chronicals_torch_bind(lib._handle) != 0:
-        raise ImportError(f"{_lib.lib_path()} lacks functions that {path} needs: rebuild both")
+    native.chronicals_torch_hooks.argtypes = [ctypes.py_object]
+    native.chronicals_torch_hooks.restype = None
+
+    def load():
+        if native.chronicals_torch_bind(_lib.load()._handle) != 0:
+            raise ImportError(f"{_lib.lib_path()} lacks functions that {path} needs: rebuild both")
+    native.chronicals_torch_hooks(load)
+    return True
 
 
-_load_kernels()
+def _unbuilt(name: str):
+    """The kernel of an operator until its C++ kernel is built and loaded."""
+    def call(*args, **kwargs):
+        if not _load_kernels():
+            raise ImportError(f"{_build.torch_lib_path()} not found: build it with `python -m chronicals_amd.build` "
+                              f"(or __graft_entry__.build())")
+        return getattr(torch.ops.chronicals_hip, name)(*args, **kwargs)
+    return call
+
+
+if not _load_kernels():
+    for _s in _SCHEMAS:
+        _LIBRARY.impl(_s.split("(", 1)[0], _unbuilt(_s.split("(", 1)[0]), "CUDA")
 
 
 def _stream(device: torch.device) -> int:

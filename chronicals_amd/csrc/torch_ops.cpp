@@ -9,8 +9,9 @@
 // ops.py defines the schemas and the fake (meta) implementations; the kernels
 // are registered here.  The C functions come from the library that the Python
 // loader opens (chronicals_torch_bind), so that CHRONICALS_CCE_LIB and the
-// loader's checks hold for both.  The first call of an operator asks for it
-// through a Python callable that ops.py hands over (chronicals_torch_hooks).
+// loader's checks hold for both.  The first call of an operator asks for it, and
+// a failing call raises what the package's Python code raises: both through two
+// Python callables that ops.py hands over (chronicals_torch_hooks).
 #include <Python.h>
 
 #include <ATen/ATen.h>
@@ -45,17 +46,18 @@ struct Api {
 Api g_api;
 std::atomic<bool> g_bound{false};
 
-PyObject* g_load = nullptr;  // load(): opens the library and binds it here, or raises
+PyObject* g_load = nullptr;   // load(): opens the library and binds it here, or raises
+PyObject* g_check = nullptr;  // check(rc): raises for a failing rc, with cce_last_error()'s text
 
-// Calls a hook; what it raises goes on as a Python exception.  Operators run
-// without the interpreter's lock.
-void call_hook(PyObject* hook) {
+// Calls a hook with its argument, if any; what it raises goes on as a Python
+// exception.  Operators run without the interpreter's lock.
+void call_hook(PyObject* hook, const long* arg) {
   TORCH_CHECK(hook != nullptr, "chronicals_amd.ops is not imported");
   struct Gil {
     PyGILState_STATE state = PyGILState_Ensure();
     ~Gil() { PyGILState_Release(state); }
   } gil;
-  PyObject* const res = PyObject_CallObject(hook, nullptr);
+  PyObject* const res = arg ? PyObject_CallFunction(hook, "l", *arg) : PyObject_CallObject(hook, nullptr);
   if (!res) {
     python_error e;
     e.persist();
@@ -65,15 +67,17 @@ void call_hook(PyObject* hook) {
 }
 
 const Api& api() {
-  if (!g_bound.load(std::memory_order_acquire)) call_hook(g_load);
+  if (!g_bound.load(std::memory_order_acquire)) call_hook(g_load, nullptr);
   TORCH_CHECK(g_bound.load(std::memory_order_acquire), "libchronicals_cce.so is not bound");
   return g_api;
 }
 
+// cce_last_error() is the calling thread's, and the hook runs in this thread.
 void check(const Api& a, int rc) {
   if (rc == CCE_OK) return;
-  const char* msg = a.last_error();
-  TORCH_CHECK(false, "libchronicals_cce error ", rc, ": ", msg ? msg : "");
+  const long code = rc;
+  call_hook(g_check, &code);
+  TORCH_CHECK(false, "libchronicals_cce error ", rc, ": ", a.last_error());
 }
 
 void* stream(const at::Device& device) {
@@ -292,10 +296,12 @@ int chronicals_torch_bind(void* handle) {
   return 0;
 }
 
-// The Python callable of api(); called with the interpreter's lock.
-void chronicals_torch_hooks(PyObject* load) {
+// The Python callables of api() and check(); called with the interpreter's lock.
+void chronicals_torch_hooks(PyObject* load, PyObject* check) {
   Py_XINCREF(load);
+  Py_XINCREF(check);
   Py_XSETREF(g_load, load);
+  Py_XSETREF(g_check, check);
 }
 
 }  // extern "C"

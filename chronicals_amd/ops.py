@@ -74,13 +74,13 @@ def _load_kernels() -> bool:
     torch.ops.load_library(path)
     native = ctypes.PyDLL(path)
     native.chronicals_torch_bind.argtypes = [ctypes.c_void_p]
-    native.chronicals_torch_hooks.argtypes = [ctypes.py_object]
+    native.chronicals_torch_hooks.argtypes = [ctypes.py_object, ctypes.py_object]
     native.chronicals_torch_hooks.restype = None
 
     def load():
         if native.chronicals_torch_bind(_lib.load()._handle) != 0:
             raise ImportError(f"{_lib.lib_path()} lacks functions that {path} needs: rebuild both")
-    native.chronicals_torch_hooks(load)
+    native.chronicals_torch_hooks(load, _lib.check)
     return True
 
 

@@ -29,7 +29,7 @@ def call():
 
 def works():
     e = call()
-    assert isinstance(e, RuntimeError) and "multiple of 8" in str(e), repr(e)
+    assert type(e) is _lib.CCEError and "multiple of 8" in str(e), repr(e)
 '''
 
 
@@ -49,6 +49,10 @@ def run(tree, code, **env):
     out = subprocess.run([sys.executable, "-c", HEAD + code], capture_output=True, text=True, cwd=tree, env=env,
                          timeout=300)
     assert out.returncode == 0, out.stdout + out.stderr
+
+
+def test_errors_of_the_c_library_keep_their_type(tree):
+    run(tree, "works()\n")
 
 
 def test_a_broken_library_raises_in_the_call(tree):

@@ -4,8 +4,8 @@ The library is compiled with hipcc from ``chronicals_amd/csrc/cce_kernels.hip``
 into ``chronicals_amd/lib/libchronicals_cce.so``; the package loads it from
 there with ctypes.  The torch operators (``csrc/torch_ops.cpp``, host code only)
 are compiled against the installed torch into
-``lib/libchronicals_torch-<hash>.so``, where the hash covers their source, the
-header and torch's version: a build of anything else has another name and is
+``lib/libchronicals_torch-<hash>-<torch version>.so``, where the hash covers
+their source and the header: a build of anything else has another name and is
 never loaded.  Building always recompiles both.
 """
 from __future__ import annotations
@@ -70,11 +70,16 @@ def compile_command(out_path: str, src_hash: str = None) -> list:
 
 
 def torch_lib_path() -> str:
-    """Where the torch operators of this tree and this torch are built."""
+    """Where the torch operators of this tree and this torch are built.  Without
+    the sources (an installed tree): the one build for this torch."""
     import torch
 
-    h = hashlib.sha256((source_hash((TORCH_SRC, HEADER)) + torch.__version__).encode()).hexdigest()
-    return os.path.join(LIB_DIR, f"libchronicals_torch-{h[:16]}.so")
+    tail = f"-{torch.__version__}.so"
+    if not (os.path.exists(TORCH_SRC) and os.path.exists(HEADER)):
+        built = [n for n in (os.listdir(LIB_DIR) if os.path.isdir(LIB_DIR) else ())
+                 if n.startswith("libchronicals_torch-") and n.endswith(tail)]
+        return os.path.join(LIB_DIR, built[0] if len(built) == 1 else f"libchronicals_torch-*{tail}")
+    return os.path.join(LIB_DIR, f"libchronicals_torch-{source_hash((TORCH_SRC, HEADER))[:16]}{tail}")
 
 
 def torch_compile_command(out_path: str) -> list:

@@ -105,3 +105,15 @@ def test_in_place_and_functional_operators_agree(tree):
               "maps = {l.split()[-1] for l in open('/proc/self/maps') if 'libchronicals_cce' in l}\n"
               "assert maps == {os.path.realpath(build.LIB_PATH)}, maps\n"
               "assert _lib.load()._name == build.LIB_PATH\n")
+
+
+def test_a_tree_without_its_sources_works(tree):
+    shutil.rmtree(tree / "include")
+    run(tree, "works()\n")
+    shutil.rmtree(tree / "chronicals_amd" / "csrc")
+    run(tree, "works()\n")
+    # a build for another torch is not loaded
+    lib = tree / "chronicals_amd" / "lib"
+    built = os.path.basename(_build.torch_lib_path())
+    shutil.move(lib / built, lib / built.replace(".so", "x.so"))
+    run(tree, "e = call()\nassert type(e) is ImportError and 'build it' in str(e), repr(e)\n")

@@ -6,11 +6,14 @@ there with ctypes.  The torch operators (``csrc/torch_ops.cpp``, host code only)
 are compiled against the installed torch into
 ``lib/libchronicals_torch-<hash>-<torch version>.so``, where the hash covers
 their source and the header: a build of anything else has another name and is
-never loaded.  Building always recompiles both.
+never loaded.  Building always recompiles both, the HIP library first: it needs
+neither torch nor a host compiler, and stays usable from C where the operators
+cannot be built.
 """
 from __future__ import annotations
 
 import hashlib
+import importlib.util
 import os
 import shutil
 import subprocess
@@ -139,8 +142,17 @@ def parse_resources(text: str) -> dict:
 
 
 def build(verbose: bool = False) -> str:
-    """Compile the HIP library and the torch operators; returns the path of the HIP library."""
-    build_torch(verbose)
+    """Compile the HIP library and, where torch is installed, its operators; returns the path of the HIP library."""
+    build_hip(verbose)
+    if importlib.util.find_spec("torch") is None:
+        sys.stderr.write("torch is not installed: its operators are not built\n")
+    else:
+        build_torch(verbose)
+    return LIB_PATH
+
+
+def build_hip(verbose: bool = False) -> None:
+    """Compile the HIP library."""
     os.makedirs(LIB_DIR, exist_ok=True)
     tmp = LIB_PATH + f".tmp{os.getpid()}"
     cmd = compile_command(tmp, source_hash())
@@ -158,7 +170,6 @@ def build(verbose: bool = False) -> str:
     spills = {n: r.get("VGPRs Spill", 0) for n, r in res.items() if r.get("VGPRs Spill", 0)}
     if spills:
         sys.stderr.write(f"warning: kernels spill VGPRs to scratch: {spills}\n")
-    return LIB_PATH
 
 
 if __name__ == "__main__":

@@ -239,3 +239,59 @@ def assert_grad_close_torch(got: torch.Tensor, ref: torch.Tensor, what: str):
     assert r["frac"] <= GRAD_MAXABS_FRAC, f"{what}: max abs err too large {r}"
     assert r["cos"] >= GRAD_COS_MIN, f"{what}: cosine too small {r}"
 
+
+
+@dataclass(frozen=True)
+class BackwardPlan:
+    """How a backward is cut up: vocabulary bands of `width` columns (the first
+    of `head`), row blocks of `rows`, K splits of dH, and the workspace."""
+    bands: int
+    width: int
+    head: int
+    blocks: int
+    rows: int
+    splits: int
+    scratch: str   # what grad_hidden holds while the bands run: "H^T", "H" (in row order) or ""
+    workspace: int
+
+
+def backward_plan(N, d, V, chunk, need_dh=True, need_dw=True, dh_f32=False, dw_f32=False, budget_mb=0, gather=""):
+    """The library's rules restated, so that a test can say which path its sizes
+    reach (tests/test_band_plan.py holds them against the workspace queries)."""
+    def up(x, a):
+        return -(-x // a) * a
+
+    budget = (budget_mb or 512) << 20
+    Vb = up(min(chunk, 8192) if chunk > 0 else 8192, 256)
+    rows = up(max(N, 1), 256)
+    if rows < 3072:
+        Vb = max(Vb, min(Vb * 3072 // rows, budget // (4 * rows) // 256 * 256))
+        Vb = up(-(-V // -(-V // Vb)), 256)
+    Vb = max(min(Vb, up(V, 256)), 256)
+    Nb = min(max(budget // (4 * Vb) // 256 * 256, 256), max(N, 1))
+    bands, blocks = -(-V // Vb), -(-max(N, 1) // Nb)
+    units = bands * blocks
+    in_place = N * d * 2 <= 0x7ffffff0 and d % 64 == 0 and (gather == "1" or (gather != "0" and N * d * 2 >= 2 ** 28))
+    copied = N > 256 and not in_place
+    late = need_dh and not dh_f32 and bands > 1
+    scratch = "H^T" if late and need_dw and N % 64 == 0 else "H" if late and not need_dw and copied else ""
+    tiles = -(-Nb // 256) * (-(-d // 256) if d % 256 == 0 or d % 256 > 128 else d // 256 + 1)
+    splits = 1
+    if need_dh and tiles < 128:
+        splits = max(1, min(-(-128 // tiles), Vb // 512))
+    parts = [16 * N, 4 * N, 2 * Nb * Vb]
+    if units > 1:
+        parts.append(2 * Nb * Vb)
+    if need_dw and scratch != "H^T":
+        parts.append(2 * d * up(N, 64))
+    if late:
+        parts.append(4 * N * d)
+    if need_dw and blocks > 1 and not dw_f32:
+        parts.append(4 * Vb * d)
+    if N > 256:
+        parts += [4 * N, 4]
+    if copied and scratch != "H":
+        parts.append(2 * N * d)
+    if splits > 1:
+        parts.append(4 * (2 if splits >= 4 and units > 1 else 1) * splits * Nb * d)
+    return BackwardPlan(bands, Vb, V - (bands - 1) * Vb, blocks, Nb, splits, scratch, sum(up(p, 256) for p in parts))

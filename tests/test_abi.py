@@ -126,10 +126,10 @@ def test_stale_library_is_refused(lib, monkeypatch):
 
 @pytest.mark.parametrize("d,V", [(896, 151936), (4096, 128256), (768, 50257), (3584, 152064)])
 def test_small_batch_backward_workspace_bounded(lib, d, V):
-    """Small batches widen the vocabulary bands (from 1024 rows) and split dH
+    """Small batches widen the vocabulary bands (below 3072 rows) and split dH
     into fp32 partials (few row tiles); neither may make a smaller batch need
-    more backward workspace than 4096 rows at the same chunk_size, and below
-    1024 rows none of it may outgrow the materialised fp32 logits and their
+    more backward workspace than 4096 rows at the same chunk_size, and at 256
+    rows none of it may outgrow the materialised fp32 logits and their
     gradient."""
     ref = _lib.backward_workspace_bytes(4096, d, V, 8192, True, True)
     for N in (1, 256, 512, 1024, 2048, 3072):
@@ -201,9 +201,9 @@ def test_backward_band_gradient_bounded_in_N(lib, d, V):
     w1 = _lib.backward_workspace_bytes(n1, d, V, 8192, True, True)
     w2 = _lib.backward_workspace_bytes(n2, d, V, 8192, True, True)
     # at both batches, all but the O(N*d) buffers fit in the G budget plus
-    # the band's W^T (two buffers), its fp32 dW accumulator and the fp32
-    # partials of a K-split dH (about 128 tiles of 256 x 256, two buffers)
-    band_rest = 512 * 2 ** 20 + 2 * d * 8192 * 2 + 8192 * d * 4 + 2 * 160 * 256 * 256 * 4 + 2 ** 20
+    # the band's fp32 dW accumulator and the fp32 partials of a K-split dH
+    # (about 128 tiles of 256 x 256, two buffers)
+    band_rest = 512 * 2 ** 20 + 8192 * d * 4 + 2 * 160 * 256 * 256 * 4 + 2 ** 20
     assert w1 - n1 * per_row <= band_rest
     assert w2 - n2 * per_row <= band_rest
     assert w2 - w1 >= (n2 - n1) * 4 * d  # the O(N*d) buffers are there
@@ -215,10 +215,9 @@ def test_backward_band_gradient_bounded_in_N(lib, d, V):
 
 def test_backward_workspace_borrows_gradient_memory(lib):
     """While the bands run, grad_hidden holds H^T (bf16 dH, several bands) or,
-    with no dW wanted, the two band transposes of W; the rows of band b+1 of
-    grad_weight hold band b's W^T.  None of it takes workspace: C5 needs
-    under 1.5 GiB, the transposes no longer count at C2, and fp32 dH (the
-    output is its own accumulator) keeps H^T in the workspace."""
+    with no dW wanted, H in row order.  Neither takes workspace then: C5 needs
+    under 1.5 GiB, and fp32 dH (the output is its own accumulator) keeps H^T
+    in the workspace."""
     c2 = (16384, 896, 151936)
     c5 = (65536, 3584, 152064)
     w5 = _lib.backward_workspace_bytes(*c5, 8192, True, True)
@@ -229,9 +228,8 @@ def test_backward_workspace_borrows_gradient_memory(lib):
     assert w5 <= 2 * 16384 * 8192 * 2 + N * d * 4 + 8192 * d * 4 + N * 64 + 2 ** 20
     w2 = _lib.backward_workspace_bytes(*c2, 8192, True, True)
     N, d, V = c2
-    # one band of W^T (the last band's) besides G, the dH accumulator, H in
-    # row order (a copy below 256 MiB) and the row data
-    assert w2 <= 2 * N * 8192 * 2 + N * d * 4 + d * 8192 * 2 + N * d * 2 + N * 64 + 2 ** 20
+    # G, the dH accumulator, H in row order (a copy below 256 MiB) and the row data
+    assert w2 <= 2 * N * 8192 * 2 + N * d * 4 + N * d * 2 + N * 64 + 2 ** 20
     assert _lib.backward_workspace_bytes(*c2, 8192, True, False) < w2  # frozen W
     w2_f32 = _lib.backward_workspace_bytes(*c2, 8192, True, True, True, False)
     assert w2_f32 >= w2 - N * d * 4 + d * N * 2  # no dH accumulator, but H^T in the workspace

@@ -18,7 +18,7 @@ pytestmark = pytest.mark.gpu
     (256, 64, 200000, 8192, False, True, torch.bfloat16),  # three bands of equal width
     (255, 192, 5003, 256, True, False, torch.bfloat16),    # frozen weight, ragged band
     (257, 256, 5003, 8192, True, True, torch.bfloat16),    # two row tiles: the row order is back
-    (2900, 64, 9000, 1024, False, True, torch.bfloat16),   # bands widened by 3072 / 3072
+    (2900, 64, 9000, 1024, False, True, torch.bfloat16),   # 3072 rows in tiles: not widened
 ])
 def test_few_rows(gpu, N, d, V, chunk, bias, need_dw, hdtype):
     print(f"case few rows N={N} d={d} V={V} chunk={chunk} bias={bias} dw={need_dw} {hdtype}", flush=True)

@@ -81,8 +81,8 @@ def _rand_case(N, d, V, seed=0, ignore_frac=0.1, bias=False, wscale=0.05):
     (256, 64, 256, 8192),      # one tile
     (1, 8, 1, 8192),           # smallest problem
     (3, 16, 7, 8192),
-    (255, 72, 257, 256),       # ragged rows / columns, two bands
-    (257, 136, 1000, 512),     # d not a multiple of 64, ragged bands
+    (255, 72, 257, 256),       # ragged rows / columns
+    (257, 136, 1000, 512),     # d not a multiple of 64, two row tiles
     (600, 128, 5000, 1024),
     (513, 264, 3001, 8192),
     (300, 192, 2100, 512),     # d % 256 > 128: one padded 256-wide dH column tile
@@ -95,26 +95,25 @@ def test_ragged_shapes(gpu, N, d, V, chunk):
 
 
 @pytest.mark.parametrize("N,d,V,chunk,hdtype,reduction,ignore_frac", [
-    # 9 dH tiles: 15 K splits; a partial first band and two full ones (accumulator modes 1, 2, 3);
-    # fp32 gradients; per-row grad_output
+    # 9 dH tiles: 15 K splits of one band (mode 0); fp32 gradients; per-row grad_output
     (700, 768, 20000, 8192, torch.float32, "none", 0.1),
     # d = 256 + 64: the 128-wide tail tile is split too; most rows ignored (one live row tile of three)
     (600, 320, 9000, 4096, torch.bfloat16, "mean", 0.7),
-    # one band (mode 0: straight to the output; the band is 3072 wide): 6 splits of 512 columns, the last shorter
+    # the band is 3072 wide: 6 splits of 512 columns, the last shorter
     (130, 512, 3000, 8192, torch.bfloat16, "sum", 0.1),
-    # V = 8 * 8192 + 40: 9 bands of 8192 (256 rows are not widened); the 40-column first band is left with a
-    # single split and still writes partials
+    # one band of 65576 columns in 43 splits
     (256, 768, 65576, 8192, torch.bfloat16, "mean", 0.1),
-    # 1100 rows widen chunk 1024 to 3072-column bands: 7 bands; d = 128 is one 128-wide tail tile (5 dH tiles,
-    # 6 K splits: the reduction rides in the next band's launch); 30% of the rows ignored
+    # 1100 rows widen chunk 1024 to 2304-column bands: 9 bands; d = 128 is one 128-wide tail tile (5 dH tiles,
+    # 4 K splits: the reduction rides in the next band's launch); 30% of the rows ignored
     (1100, 128, 20000, 1024, torch.bfloat16, "mean", 0.3),
-    # 1300 rows widen chunk 2048 to 4096: 3 bands (a 808-column first band); 6 dH tiles of 256 columns, 8 splits
+    # 1300 rows widen chunk 2048 to 3072: 3 bands; 6 dH tiles of 256 columns, 6 splits; fp32 dH (modes 0 and 4)
     (1300, 256, 9000, 2048, torch.float32, "sum", 0.1),
 ])
 def test_small_batch_split_dh(gpu, N, d, V, chunk, hdtype, reduction, ignore_frac):
     """With few 256-row tiles the banded dH splits each band's K over several
     workgroups (fp32 partials, then a fixed-order reduction that applies the
-    band's accumulator mode); against the oracle, and bitwise repeatable."""
+    band's accumulator mode; several bands in every mode: test_gpu_bands.py);
+    against the oracle, and bitwise repeatable."""
     print(f"case split dH N={N} d={d} V={V} chunk={chunk} {hdtype} {reduction}", flush=True)
     h, w, lab, _ = _rand_case(N, d, V, seed=N + d, ignore_frac=ignore_frac)
     go = torch.rand(N, generator=torch.Generator().manual_seed(4)) if reduction == "none" else None
@@ -165,7 +164,7 @@ def test_ignored_row_tiles_are_skipped(gpu, reduction, bias, hdtype):
     # The banded backward compacts the labelled rows to the front and skips
     # the 256-row tiles past them: 400 labelled rows of 1100 leave 2 of 5 row
     # tiles live.  The ignored rows' dH must still be exactly zero.  V = 9500
-    # keeps 4 bands (1100 rows widen chunk 1024 to 3072-column bands), so the
+    # keeps 4 bands (1100 rows widen chunk 1024 to 2560-column bands), so the
     # accumulator modes 1, 2 and 3 all run on the compacted rows.
     print(f"case compaction reduction={reduction} bias={bias} hdtype={hdtype}", flush=True)
     h, w, lab, b = _rand_case(1100, 128, 9500, seed=21, ignore_frac=0.0, bias=bias)
@@ -198,8 +197,8 @@ def test_labelled_rows_at_the_end(gpu):
 def test_forward_lse_labelled_rows(gpu, d):
     """CCE_LSE_LABELLED_ROWS: the same loss and n_valid as CCE_LSE_ALL_ROWS, the
     same lse / target on labelled rows, 0 on ignored rows (d = 128 compacts
-    the rows; d = 72 runs the register-staged GEMM over every row).  V = 9500
-    gives the autograd check 4 backward bands of 3072 columns."""
+    the rows; d = 72 runs over every row).  V = 9500
+    gives the autograd check 4 backward bands of 2560 columns."""
     from chronicals_amd import _lib
     print(f"case lse_rows d={d}", flush=True)
     h, w, lab, b = _rand_case(1100, d, 9500, seed=29, ignore_frac=0.0, bias=True)
@@ -275,8 +274,8 @@ def test_frozen_weight_and_int32_labels_and_3d(gpu):
 @pytest.mark.parametrize("need_dh,need_dw,need_db", [(True, False, False), (False, True, False),
                                                     (False, False, True), (False, True, True)])
 def test_gradient_subsets_banded(gpu, need_dh, need_dw, need_db):
-    """Every subset of requested gradients through the banded backward (d % 64 == 0, several
-    bands, so the per-band launch alternates its two G buffers)."""
+    """Every subset of requested gradients from one band of the backward (over several:
+    test_gpu_bands.py)."""
     print(f"case dh={need_dh} dw={need_dw} db={need_db}", flush=True)
     h, w, lab, b = _rand_case(450, 384, 2600, seed=31, bias=True)
     got = run_hip(gpu, h, w, lab, b, chunk=512, need_dh=need_dh, need_dw=need_dw, need_db=need_db)
@@ -503,10 +502,9 @@ def test_peak_memory_bounded(gpu, cfg):
     # what is not O(N*d) (H in row order, the fp32 dH accumulator, the
     # gradients) is the bounded band state
     ws = _lib.backward_workspace_bytes(N, d, V, chunk, True, True)
-    assert ws - N * (8 * d + 64) <= 512 * 2 ** 20 + 2 * d * chunk * 2 + chunk * d * 4 + 2 ** 20
-    # H^T and the band transposes of W live in the gradient outputs until
-    # those are written: at C5 the fwd+bwd peak beside the gradients stays
-    # within 1.5 GiB
+    assert ws - N * (8 * d + 64) <= 512 * 2 ** 20 + chunk * d * 4 + 2 ** 20
+    # H^T lives in grad_hidden until that is written: at C5 the fwd+bwd peak
+    # beside the gradients stays within 1.5 GiB
     assert peak - grads <= {"C2": 640, "C5": 1536}[cfg] * 2 ** 20, (peak - grads) / 2 ** 20
 
 
@@ -604,11 +602,11 @@ def test_row_order_reads_match_gathered_copy(gpu, monkeypatch, N, d, V, chunk, b
 
 
 @pytest.mark.parametrize("N,d,V,chunk,budget_mb,hdtype,reduction,bias,frozen,ignore_frac", [
-    # 6 row blocks of 256 (2048-column bands); dH split 4 ways per block, folded into the next launch
+    # 3 row blocks of 512 in 9 bands; dH split in two per block
     (1300, 128, 9000, 1024, 2, torch.bfloat16, "mean", False, False, 0.1),
     # fp32 gradients accumulate in place over bands (dH) and blocks (dW); dB added over the blocks
     (2100, 256, 7000, 2048, 4, torch.float32, "sum", True, False, 0.1),
-    # d % 64 != 0: the unbanded path in 4 blocks, per-row grad_output
+    # d % 64 != 0, 4 blocks, per-row grad_output
     (1000, 72, 5000, 1024, 1, torch.bfloat16, "none", True, False, 0.1),
     # frozen weight (dH only), 6 blocks of 512
     (3000, 512, 12000, 4096, 8, torch.bfloat16, "mean", False, True, 0.1),
@@ -641,29 +639,26 @@ def test_row_blocks(gpu, monkeypatch, N, d, V, chunk, budget_mb, hdtype, reducti
 
 
 @pytest.mark.parametrize("N,d,V,chunk,budget_mb,hdtype,wdtype,need_dw,bias", [
-    # 2 bands, 4 row blocks: H^T in grad_hidden; band 0's W^T in band 1's dW
-    # rows, band 1's (the last) in its own rows, transposed by a launch of its
-    # own after band 0, and its dW written from the fp32 accumulator at the end
+    # 2 bands, 4 row blocks: H^T in grad_hidden
     (4096, 64, 500, 256, 1, torch.bfloat16, torch.bfloat16, True, False),
-    # fp32 dW (accumulates in place): the last band's W^T in a workspace buffer
+    # fp32 dW (accumulates in place)
     (4096, 64, 500, 256, 1, torch.bfloat16, torch.float32, True, True),
     # fp32 dH (its own accumulator): H^T stays in the workspace
     (4096, 64, 500, 256, 1, torch.float32, torch.bfloat16, True, False),
-    # N % 64 != 0: H^T in the workspace; 4 bands in one block, W^T in the next
-    # band's dW rows, the last band's in a workspace buffer
+    # N % 64 != 0: H^T in the workspace; 4 bands in one block
     (4100, 64, 900, 256, 0, torch.bfloat16, torch.bfloat16, True, False),
     # 5 bands in 2 blocks, 256 + 128-wide hidden tiles, bias
     (4096, 320, 1200, 256, 2, torch.bfloat16, torch.bfloat16, True, True),
-    # frozen weight, N >= 2 x band: both W^T buffers in grad_hidden
+    # frozen weight: H in row order in grad_hidden
     (4096, 128, 900, 256, 0, torch.bfloat16, torch.bfloat16, False, False),
-    # frozen weight, N < 2 x band: W^T in the workspace
+    # frozen weight, one band: dH goes straight to the output
     (300, 128, 900, 256, 0, torch.bfloat16, torch.bfloat16, False, False),
 ])
 def test_gradient_outputs_as_scratch(gpu, monkeypatch, N, d, V, chunk, budget_mb, hdtype, wdtype, need_dw, bias):
-    """While the bands run, H^T and the band transposes of W live in gradient
-    output memory that is not yet written (grad_hidden; the rows of the next
-    band of grad_weight); each placement and its fallback against the oracle,
-    and bitwise repeatable."""
+    """While the bands run, H^T, or H in row order without a dW, lives in
+    grad_hidden, which is not yet written; each placement and its fallback
+    against the oracle, and bitwise repeatable (with few rows:
+    test_gpu_bands.py)."""
     print(f"case outputs-as-scratch N={N} d={d} V={V} chunk={chunk} budget={budget_mb} {hdtype} {wdtype} "
           f"dw={need_dw} bias={bias}", flush=True)
     if budget_mb:
@@ -745,7 +740,7 @@ def test_random_sweep(gpu, monkeypatch, case):
     # lies the rest of the workspace
     (1001, 128, 3000, 1024, "workspace"),
     (1000, 128, 1000, 1024, "workspace"),
-    (999, 72, 2000, 512, "workspace"),       # d % 64 != 0: the separate dW launch
+    (999, 72, 2000, 512, "workspace"),       # d % 64 != 0
 ])
 def test_dw_reads_stop_at_the_end_of_ht(gpu, N, d, V, chunk, where):
     """dW = G^T . H reads H^T ([d][N rounded up to 8]) in 64-row slabs of N;

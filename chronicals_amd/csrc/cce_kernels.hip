@@ -2434,12 +2434,20 @@ void grad_shape(const bf16_t* H, const bf16_t* W, const float* bias, const BwdLa
 // Order of a band launch's populations: the longest workgroups first, by the
 // length of their reductions (dW: the block's rows; dH: its share of the band;
 // recompute: d), so that the short ones fill the CUs the long ones leave idle.
-// N 2048, d 896, V 151936 (dH 46 slabs, dW 30, recompute 14): forward and
-// backward 2.51 ms with dW always first, 2.32 ms so.  A dW over one row tile is
-// bound by its stores, not its slabs, and starts first: N 256, d 768, V 50257
-// in fp32 288 us behind the others, 254 us first.
+// The rows are the block's, ignored ones included: how many are live is known
+// on the device only.  N 2048, d 896, V 151936 (dH 46 slabs, dW 30, recompute
+// 14): forward and backward 2.51 ms with dW always first, 2.32 ms so.
+//
+// An fp32 dW over one row tile starts first: its tiles are four slabs and 256 KB
+// of stores.  Behind the others / first, forward and backward in us (rows x d x
+// V): 256 x 768 x 50257 248 / 231, 51 x 448 x 108581 247 / 241, but 158 x 624 x
+// 114692 384 / 391, 168 x 1856 x 50098 427 / 437, 71 x 384 x 83806 258 / 272.
+// A bf16 dW stores half of that and keeps its place: 62 x 1544 x 36645 190 / 203,
+// 244 x 1856 x 105749 572 / 612, 166 x 256 x 96209 128 / 129, 64 x 2752 x 13306
+// 226 / 231.
 void order_populations(BandLaunch& p, long k_dw, long k_dh, long k_gr) {
-  const long k[3] = {k_dw <= kBM ? LONG_MAX : k_dw, k_dh, k_gr};
+  const bool dw_first = k_dw <= kBM && (p.e_dw.out_f32 || p.e_dw2.out_f32);
+  const long k[3] = {dw_first ? LONG_MAX : k_dw, k_dh, k_gr};
   const int nb[3] = {p.nb_dw + p.nb_dw2, p.nb_dh + p.nb_dh2, p.nb_gr};
   int o[3] = {kPopDW, kPopDH, kPopGrad};
   std::stable_sort(o, o + 3, [&](int x, int y) { return k[x] > k[y]; });

@@ -1202,7 +1202,7 @@ __global__ __launch_bounds__(256) void fwd_combine_kernel(
     const float* __restrict__ pm, const float* __restrict__ ps, int splits, const bf16_t* __restrict__ H,
     const bf16_t* __restrict__ W, const void* labels, int labels64, const float* __restrict__ bias, int N, int d,
     int V, long ignore_index, float eps, float zw, float logV, const float* __restrict__ wsum, int labelled_only,
-    const int* __restrict__ idx, const int* __restrict__ live, int nb_fwd, int tiles_n, float* __restrict__ lse_out,
+    const int* __restrict__ idx, const int* __restrict__ live, float* __restrict__ lse_out,
     float* __restrict__ target_out, float* __restrict__ rowloss, float* __restrict__ bsum, int* __restrict__ bcnt) {
   // wave w handles partial row i; its source row is idx[i] (identity without
   // idx).  With labelled_only, ignored rows get lse 0 and their partials,
@@ -1536,8 +1536,7 @@ __global__ __launch_bounds__(256) void ce_logits_bwd_kernel(const float* __restr
   const T* row = X + (long)n * ld;
   TO* drow = dX + (long)n * ldg;
   const long lab = load_label(labels, labels64, n);
-  const bool valid = lab != ignore_index;
-  if (!valid) {
+  if (lab == ignore_index) {
     zero_row<256>(drow, V, tid);
     return;
   }
@@ -1545,11 +1544,11 @@ __global__ __launch_bounds__(256) void ce_logits_bwd_kernel(const float* __restr
   if (reduction == CCE_REDUCTION_MEAN) g /= (float)(n_valid[0] > 1 ? n_valid[0] : 1);
   const float l = lse[n];
   const bool uni = smooth_mode == CCE_SMOOTH_UNIFORM;
-  const float cP = valid ? g * ((uni ? 1.f : 1.f - eps) + 2.f * zw * l) : 0.f;
-  const float cU = valid && uni ? g * eps / (float)V : 0.f;
-  const float cT = valid ? g * (1.f - eps) : 0.f;
+  const float cP = g * ((uni ? 1.f : 1.f - eps) + 2.f * zw * l);
+  const float cU = uni ? g * eps / (float)V : 0.f;
+  const float cT = g * (1.f - eps);
   const float l2 = l * kLog2e;
-  const long t = (valid && lab >= 0 && lab < V) ? lab : -1;
+  const long t = (lab >= 0 && lab < V) ? lab : -1;
   auto grad1 = [&](int v, float x) { return (cP * fast_exp2(x * kLog2e - l2) - cU) - (v == t ? cT : 0.f); };
   const RowSplit<T> sp(row, V);
   // 16-byte chunks of X map onto (sizeof(TO)/sizeof(T)) aligned 16-byte
@@ -2621,8 +2620,8 @@ int forward_run(const void* hidden, const void* weight, const void* labels, int 
   hipLaunchKernelGGL(fwd_combine_kernel, dim3(nb), dim3(256), 0, st, L.pm, L.ps, S,
                      static_cast<const bf16_t*>(hidden), static_cast<const bf16_t*>(weight), labels, labels_int64,
                      bias, (int)N, (int)d, (int)V, (long)ignore_index, label_smoothing, z_loss_weight, logV,
-                     uniform ? L.wsum : nullptr, lse_rows == CCE_LSE_LABELLED_ROWS, L.idx, L.live, slots,
-                     ep.tiles_n, lse_out, target_out, rowloss, L.bsum, L.bcnt);
+                     uniform ? L.wsum : nullptr, lse_rows == CCE_LSE_LABELLED_ROWS, L.idx, L.live, lse_out,
+                     target_out, rowloss, L.bsum, L.bcnt);
   HIP_TRY(hipGetLastError());
   hipLaunchKernelGGL(fwd_finalize_kernel, dim3(1), dim3(1024), 0, st, L.bsum, L.bcnt, nb, reduction, loss_out,
                      n_valid_out);

@@ -90,14 +90,15 @@ const char* cce_last_error(void);
  *
  * Two environment variables, read on every query and every call (so a query
  * and the call it sizes must see the same values), change the workspace
- * layout and so its size, never the results:
+ * layout and so its size, not what is computed:
  *   CHRONICALS_CCE_ROW_GATHER  0: the labelled-rows GEMMs always read a
  *       gathered N x d bf16 copy of hidden; 1: they read hidden's rows in
  *       place wherever byte offsets into hidden fit 32 bits; unset: in place
  *       for hidden of 256 MiB to 2 GiB, the copy otherwise.
  *   CHRONICALS_CCE_G_BUDGET_MB (backward only) the memory budget of the two
  *       band-gradient buffers, in MiB (default 512); a smaller budget means
- *       more, smaller row blocks.
+ *       more, smaller row blocks and narrower bands for few rows (the same
+ *       fp32 terms, added in another order).
  */
 int cce_forward_workspace_bytes(int64_t N, int64_t d, int64_t V, int reduction, int lse_rows, size_t* bytes);
 
@@ -180,10 +181,10 @@ int cce_backward_workspace_bytes(int64_t N, int64_t d, int64_t V, int64_t chunk_
  * reference's chunk_size argument (:1028), rounded up to a multiple of 256,
  * bounds the band from above (the partial band, if any, comes first); below
  * 3072 rows the bands widen to what the gradient of 3072 rows takes at that
- * width.  The rows are processed in blocks whose
- * band gradient (two bf16 buffers of rows x band) stays within 512 MiB, so
- * that memory does not grow with N; dW of a band accumulates over the
- * blocks.  fp32 gradients accumulate in place; bf16 ones in fp32 workspace.
+ * width (up to 12x, within the budget below).  The rows are processed in
+ * blocks whose band gradient (two bf16 buffers of rows x band) stays within
+ * 512 MiB (CHRONICALS_CCE_G_BUDGET_MB), so that memory does not grow with N;
+ * dW of a band accumulates over the blocks.  fp32 gradients accumulate in place; bf16 ones in fp32 workspace.
  * Deterministic: every reduction runs in a fixed order, including the fp32
  * partials of dH when few rows make the library split each band's columns
  * over several workgroups.

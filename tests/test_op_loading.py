@@ -8,7 +8,6 @@ import sys
 
 import pytest
 
-from chronicals_amd import _lib
 from chronicals_amd import build as _build
 
 HEAD = '''
